@@ -852,6 +852,7 @@ int run_pass(edpp_ctx* c, int strategy, const SplitCall<K>& a, int32_t* his) {
         // the hash join's partition: the WG strategy with the varied reorder
         (void)strategy;
         const bool bal = a.lg <= kBallotMatchBits;
+        if (wide_8<K>(c, a.lg)) return run_wg<K, 8, false, 512>(c, a, his);  // the shape his_len counts tiles of
         if (wg_ipt<K>(c, a.lg) == 16) {
             if (wg_block<K>(c, a.lg) == 512)
                 return bal ? run_wg<K, 16, true, 512>(c, a, his) : run_wg<K, 16, false, 512>(c, a, his);
