@@ -217,9 +217,10 @@ def cpu_primitives(orc, ref, b, n, gsrc, gidx):
     return res
 
 
-def pmc_traffic(kernel_prefix, profile, passes, timeout_s=150):
-    """HBM bytes per launch of one kernel from two rocprofv3 --pmc child runs
-    (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch) of ``bench.py --profile``.
+def pmc_traffic(kernel_parts, profile, passes, timeout_s=150):
+    """HBM bytes per call, over every kernel whose name holds one of
+    ``kernel_parts``, from two rocprofv3 --pmc child runs (FETCH_SIZE, then
+    WRITE_SIZE, KiB per dispatch) of ``bench.py --profile``.
     Each counter is scaled by what it reads for the STREAM copy kernel of 2^28
     int32 in the same run (1 GiB read, 1 GiB written).  Returns a dict, or
     None with the reason when the profiler is absent or fails."""
@@ -231,6 +232,7 @@ def pmc_traffic(kernel_prefix, profile, passes, timeout_s=150):
                                          else None)
     if prof is None:
         return None, "rocprofv3 not found"
+    calls = 2
     known = float(N_FULL * 4) / 1024.0  # KiB read (FETCH) or written (WRITE) by the copy
     out = {}
     env = dict(os.environ, TMPDIR="/tmp")
@@ -238,7 +240,7 @@ def pmc_traffic(kernel_prefix, profile, passes, timeout_s=150):
         d = tempfile.mkdtemp(prefix="edpp_pmc_", dir="/tmp")
         cmd = ["timeout", "-s", "KILL", str(timeout_s), prof, "--pmc", ctr, "--output-format", "csv", "-d", d,
                "-o", "run", "--", sys.executable, os.path.join(REPO, "bench.py"), "--profile", profile,
-               "--steps", "2", "--passes", str(passes)]
+               "--steps", str(calls), "--passes", str(passes)]
         r = subprocess.run(cmd, cwd="/tmp", env=env, capture_output=True, text=True)
         rows = []
         for root, _, files in os.walk(d):
@@ -247,13 +249,14 @@ def pmc_traffic(kernel_prefix, profile, passes, timeout_s=150):
                     with open(os.path.join(root, fn), newline="") as f:
                         rows += [row for row in csv.DictReader(f) if row.get("Counter_Name") == ctr]
         shutil.rmtree(d, ignore_errors=True)
-        kern = [float(rw["Counter_Value"]) for rw in rows if rw["Kernel_Name"].startswith(kernel_prefix)]
+        kern = [float(rw["Counter_Value"]) for rw in rows if any(k in rw["Kernel_Name"] for k in kernel_parts)]
         copy = [float(rw["Counter_Value"]) for rw in rows if rw["Kernel_Name"].startswith("void edpp::k_stream<0,")]
         if r.returncode != 0 or not kern or not copy:
             return None, f"{ctr} run rc={r.returncode}, {len(kern)} kernel / {len(copy)} copy dispatches"
         factor = known / float(np.mean(copy))
-        out[ctr] = {"kib_per_dispatch": float(np.mean(kern)), "copy_kib": float(np.mean(copy)),
-                    "factor": round(factor, 4), "bytes": float(np.mean(kern)) * factor * 1024.0}
+        per_call = float(np.sum(kern)) / calls
+        out[ctr] = {"kib_per_call": per_call, "kernels_per_call": len(kern) / calls, "copy_kib": float(np.mean(copy)),
+                    "factor": round(factor, 4), "bytes": per_call * factor * 1024.0}
     return out, None
 
 
@@ -354,11 +357,12 @@ def main():
         profile_only(args, ctx, edpp, torch)
         ctx.close()
         return
-    # HBM bytes per launch of the dominant kernel, from profiler child runs made
-    # before this process touches the GPU
+    # HBM bytes of the step's gather call (the window-ordered kernels, or a
+    # k_gather per pass), from profiler child runs made before this process
+    # touches the GPU
     traffic, traffic_note = (None, "skipped (--no-traffic)")
     if not args.no_traffic:
-        traffic, traffic_note = pmc_traffic("void edpp::k_gather<", "gather", args.passes)
+        traffic, traffic_note = pmc_traffic(("::k_gather<", "::k_st_"), "gather", args.passes)
     import importlib
     import torch
     edpp = importlib.import_module("efficient-dpp_amd")
@@ -407,11 +411,10 @@ def main():
     # bit-exact spot check of the step's result (scatter undoes gather)
     assert torch.equal(dst2, src), "gather/scatter round trip mismatch"
 
-    # dominant kernel: the gather launch(es) of the timed steps
+    # the gather calls of the timed steps
     g_ms = float(np.mean([e[0].elapsed_time(e[1]) for e in ev]))
     s_ms = float(np.mean([e[1].elapsed_time(e[2]) for e in ev]))
-    g_passes = passes if passes > 0 else ctx.schedule_passes(n, scatter=False)
-    s_passes = passes if passes > 0 else ctx.schedule_passes(n, scatter=True)
+    g_passes = s_passes = passes
     achieved = gbs(12.0 * n, g_ms)
     copy = T.time(lambda: ctx.stream_op(edpp.STREAM_COPY, src, None, dst, n), reps=20)
     copy_gbs = gbs(8.0 * n, copy["hampel_ms"])
@@ -431,15 +434,16 @@ def main():
         "data": "synthetic (SplitMix64 values, keyed-Feistel random permutation; generated on device)",
         "config": {"workload": "multi-pass gather + scatter, 2^28 int32, full random permutation",
                    "n": n, "gather_passes": g_passes, "scatter_passes": s_passes,
-                   "passes_from": "argument" if passes else "library schedule", "index": "random permutation",
+                   "passes_from": "argument" if passes else "library schedule (indices in window order, no passes)", "index": "random permutation",
                    "bytes_per_element_per_primitive": 12},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": round(traffic["FETCH_SIZE"]["bytes"] + traffic["WRITE_SIZE"]["bytes"]) if traffic
                      else None,
-                     "kernel": "k_gather (one launch per pass)",
-                     "algorithmic_bytes_per_launch": 12 * n // g_passes,
-                     "avg_launch_ms": round(g_ms / g_passes, 4),
+                     "kernel": "k_gather, one launch per pass" if passes else
+                     "gather call (k_st_first, k_st_prefix, k_st_split, k_st_gather, k_st_return)",
+                     "algorithmic_bytes_per_call": 12 * n,
+                     "avg_call_ms": round(g_ms, 4),
                      "vs_stream_copy": round(achieved / copy_gbs, 4), "stream_copy_gbs": round(copy_gbs, 2),
                      "traffic_counters": traffic if traffic else traffic_note},
         "per_primitive": {"gather_gbs": round(achieved, 2), "scatter_gbs": round(gbs(12.0 * n, s_ms), 2),

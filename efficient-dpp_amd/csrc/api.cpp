@@ -263,11 +263,13 @@ int edpp_ctx_create(int device, void* stream, edpp_ctx** out) {
             rc = EDPP_EHIP;
             break;
         }
-        if (hipMalloc(&c->tickets, 64) != hipSuccess || hipMalloc(&c->d_err, 64) != hipSuccess) {
+        if (hipMalloc(&c->tickets, 64) != hipSuccess || hipMalloc(&c->d_err, 64) != hipSuccess ||
+            hipMalloc(&c->gs_gate, kGsGateBytes) != hipSuccess) {
             rc = EDPP_ENOMEM;
             break;
         }
-        if (hipMemset(c->tickets, 0, 64) != hipSuccess || hipMemset(c->d_err, 0, 64) != hipSuccess) {
+        if (hipMemset(c->tickets, 0, 64) != hipSuccess || hipMemset(c->d_err, 0, 64) != hipSuccess ||
+            hipMemset(c->gs_gate, 0, kGsGateBytes) != hipSuccess) {
             rc = EDPP_EHIP;
             break;
         }
@@ -293,6 +295,7 @@ int edpp_ctx_destroy(edpp_ctx* c) {
     hipFree(c->chain_status);
     hipFree(c->tickets);
     hipFree(c->d_err);
+    hipFree(c->gs_gate);
     if (c->ev_start) hipEventDestroy(c->ev_start);
     if (c->ev_stop) hipEventDestroy(c->ev_stop);
     delete c;
@@ -383,7 +386,9 @@ static int gs_common(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
     if (n > 0 && (const void*)in == (const void*)out) return fail(c, EDPP_EINVAL, "in and out must differ");
     int rc = timing_begin(c, ms);
     if (!rc) {
-        if (passes == 0 && c->model && n > 0) {
+        // the staged path is faster than every pass count where it applies, so
+        // the model, which chooses among pass counts, is not asked there
+        if (passes == 0 && c->model && n > 0 && !gs_staged_applies(in, out, idx, n, (int)sizeof(T), scatter)) {
             edpp_call q = {};
             q.op = scatter ? EDPP_OP_SCATTER : EDPP_OP_GATHER;
             q.elem_bytes = (int32_t)sizeof(T);

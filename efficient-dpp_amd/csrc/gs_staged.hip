@@ -1,0 +1,1138 @@
+// gs_staged.hip — gather and scatter through windows of the random side, for
+// tables that no XCD's L2 holds.
+//
+// Semantics are those of the pass loop of gather.hip (reference:
+// opencl/primitives/gatherImpl.cpp:7-55, scatterImpl.cpp:9-54) for any pass
+// count: out[i] = in[idx[i]] / out[idx[i]] = in[i] for idx[i] in [0, n), other
+// indices skipped.
+//
+// A random 4-byte read of a table larger than an XCD's 4 MiB L2 fetches a
+// 128-byte line (56 G lines/s at most, whatever holds them), and a random
+// write leaves as a piece of a line.  Here the indices are first put in order
+// of the window of the random side they fall in.  A gather then reads window
+// after window, each from the L2 of the XCD that works on it, and brings the
+// values back into index order; a scatter moves its values along, down to
+// bins of 64 KiB of output, which it assembles in LDS.
+//   k_st_first   one read of the indices: chunks that are local are done at
+//                once; the others' elements are counted per window
+//   k_st_prefix  the counts become positions
+//   k_st_split   indices (scatter: and values) to window order, tile by tile
+//                through LDS; a gather keeps each element's slot in its tile
+//   gather:      k_st_gather    values, window after window
+//                k_st_return    values back to their tiles and into order
+//   scatter:     k_st_hist2, k_st_rows2, k_st_split2   a second split, above
+//                               1024 bins
+//                k_st_bins      every bin of the output through LDS
+// The order of a window's elements is free, so ranks come from LDS counters
+// (one atomic with return per element) and need no matching of lanes.
+// (Random writes do not gather in an L2 as reads do: writing 2 MiB windows
+// straight from window order sent 211 M write requests to memory for 2^28
+// elements, where whole lines are 17 M, and took 2.9 ms against 1.7 ms for the
+// second split and the bins.)
+//
+// 2^28 4-byte elements, random permutation, us per kernel: gather 185 + 62 +
+// 518 + 1420 + 587 (k_st_gather: 290 M L2 requests, 204 G/s; the others move
+// 10 to 12 B per element at 4.6 to 5 TB/s); scatter 170 + 37 + 885 + 255 + 14
+// + 885 + 579.
+#include <algorithm>
+#include "ctx.hpp"
+#include "device.hpp"
+#include "split_tile.hpp"
+
+namespace edpp {
+
+namespace {
+
+constexpr int64_t kStWindow = 2 << 20;    // bytes of the random side per window (an XCD's L2 holds 4 MiB)
+constexpr int kStMaxWindows = 1024;
+constexpr int kStBin = 64 << 10;          // bytes of the output a scatter's workgroup assembles in LDS
+constexpr int kStOneLevel = 1024;         // bins up to which a scatter splits once (2^24 4-byte elements: 151 against
+                                          // 167 us in two, with 32 windows of 32 bins)
+constexpr int kStLocal = 4096;            // elements of a local chunk's LDS window
+constexpr int kStBlock = 512;              // lanes of the splits and the return
+constexpr uint32_t kStNone = 0xFFFFFFFFu; // no element / index out of range
+constexpr int kStRowBlock = 1024;
+
+// Elements per 16-byte vector of T: 4 or 2.  A lane's step is one such vector
+// of values (and 16 or 8 bytes of indices), so that a wave's accesses are
+// contiguous for both widths.
+template <class T>
+constexpr int kStE = 16 / (int)sizeof(T);
+
+// elements [v*E, v*E + E) of p; `none` for the ones at or past n
+template <class T, int E>
+__device__ __forceinline__ void st_load(const T* __restrict__ p, int64_t v, int64_t n, T none, T* x) {
+    if (E * v + E <= n) {
+        typedef T vec __attribute__((ext_vector_type(E)));
+        const vec y = ld_stream(reinterpret_cast<const vec*>(p) + v);
+        #pragma unroll
+        for (int k = 0; k < E; ++k) x[k] = y[k];
+    } else {
+        #pragma unroll
+        for (int k = 0; k < E; ++k) x[k] = E * v + k < n ? p[E * v + k] : none;
+    }
+}
+// p[E*v + k] = x[k] where ok[k] (elements at or past n are never ok)
+template <class T, int E>
+__device__ __forceinline__ void st_store(T* __restrict__ p, int64_t v, const T* x, const bool* ok) {
+    bool all = true;
+    #pragma unroll
+    for (int k = 0; k < E; ++k) all = all && ok[k];
+    if (all) {
+        typedef T vec __attribute__((ext_vector_type(E)));
+        vec y;
+        #pragma unroll
+        for (int k = 0; k < E; ++k) y[k] = x[k];
+        st_stream(y, reinterpret_cast<vec*>(p) + v);
+    } else {
+        #pragma unroll
+        for (int k = 0; k < E; ++k)
+            if (ok[k]) p[E * v + k] = x[k];
+    }
+}
+
+// What every kernel of one call shares.  The indices are cut into chunks of
+// 4096 and tiles of 64 KiB of values (4 or 2 chunks, kStEpl elements for each
+// lane of the splits); lane t's elements [16h, 16h + 16) of a tile are vectors
+// u*256 + t%256 of chunk 2h + t/256.  Prefixes over the tiles are kept for
+// groups of kStGroup tiles.
+constexpr int kStChunk = 4096;
+template <class T>
+constexpr int kStEpl = 128 / (int)sizeof(T);
+template <class T>
+constexpr int kStTile = kStBlock * kStEpl<T>;
+template <class T>
+constexpr int kStCh = kStTile<T> / kStChunk;
+constexpr int kStGroup = 64;
+constexpr int kStGates = 64, kStGatePad = 32;  // words, a 128-byte line each
+struct StGeom {
+    int64_t n;
+    int shift;          // window of an index: idx >> shift
+    int W;              // windows
+    int WP;             // W, rounded up to even
+    int64_t chunks, tiles, groups;
+    int xcds;
+    uint32_t near;      // a chunk whose indices span fewer elements is done directly
+    uint8_t* done;      // [tiles * chunks per tile] chunk is finished
+    uint16_t* count;    // [chunk][WP] elements per window of the chunks that are not
+    uint32_t* rows;     // [tile][WP] elements of the window in the group's earlier tiles
+    uint32_t* gsum;     // [group][WP] the group's elements, then the position of its first one
+    uint32_t* base;     // [W + 1] first position of each window; base[W] = elements staged:
+                        // 0 when every chunk was finished, and the later kernels return
+    // a scatter's second split: windows into bins
+    int sub_shift;      // bin of an index: idx >> sub_shift
+    int lg_subs;
+    uint32_t* tile2;    // [W + 1] first second-level tile of each window
+    uint16_t* win2;     // window of each second-level tile
+    uint32_t* rows2;    // [window][bin][tile of the window]
+    uint32_t* bins;     // [W << lg_subs] first position of each bin
+    uint32_t* gate;     // [kStGates] some not 0: some chunk is not finished; 0 between calls
+    uint32_t* arrived;  // k_st_prefix's workgroups done; 0 between calls
+};
+// the lane's vector u of a tile: of its half h = u / (16/E)
+template <class T>
+__device__ __forceinline__ int64_t st_vec(int64_t tile, int u, uint32_t tid) {
+    constexpr int E = kStE<T>;
+    return tile * (kStTile<T> / E) + (int64_t)((u / (16 / E)) * (kStBlock / 256) + (int)(tid >> 8)) * (kStChunk / E) +
+           u % (16 / E) * 256 + (tid & 255);
+}
+// whether the chunk of the lane's half h is finished, from st_done's bits
+__device__ __forceinline__ bool st_skip(uint32_t mask, int h, uint32_t tid) {
+    return (mask >> (h * (kStBlock / 256) + (int)(tid >> 8))) & 1u;
+}
+__device__ __forceinline__ uint32_t* st_gate(const StGeom& g, uint32_t i) {
+    return g.gate + i % kStGates * kStGatePad;
+}
+// by the call's last kernel
+__device__ __forceinline__ void st_close(const StGeom& g) {
+    if (blockIdx.x == 0 && threadIdx.x < kStGates) *st_gate(g, threadIdx.x) = 0u;
+}
+// The o-th of `count` workgroups or steps in XCD order: contiguous ranges per
+// XCD, as split_tile.hpp's xcd_tile, for the 8 XCDs of the chip
+__device__ __forceinline__ uint32_t st_order(uint32_t o, uint32_t count, int xcds) {
+    if (xcds == 8 && count >= 8) {
+        const uint32_t per = count >> 3, rem = count & 7u, x = o & 7u;
+        return x * per + std::min(x, rem) + (o >> 3);
+    }
+    return o;
+}
+// finished chunks of a tile as bits (the last tile's missing ones among them)
+template <int CH>
+__device__ __forceinline__ uint32_t st_done(const StGeom& g, int64_t tile) {
+    uint32_t m = 0;
+    #pragma unroll
+    for (int q = 0; q < CH; ++q) m |= (tile * CH + q >= g.chunks || g.done[tile * CH + q] ? 1u : 0u) << q;
+    return m;
+}
+
+// Counters per bucket: lanes that count the same bucket at once serialize, so
+// few buckets get several counters each, taken by lane
+__host__ __device__ constexpr int st_copies_lg(int B) { return B <= 64 ? 3 : B <= 128 ? 2 : B <= 256 ? 1 : 0; }
+
+// One chunk per workgroup, of as many lanes as give a CU 32 waves beside the
+// LDS windows.  A chunk whose indices fall inside
+// kStLocal elements (a block-local permutation) goes through an LDS window: a
+// gather loads the window with consecutive loads and reads its values from
+// LDS; a scatter writes its values into the window and stores the covered
+// positions as runs.  One whose indices fall inside g.near elements is
+// addressed directly, as L2 holds that many.  The others are counted.
+template <class T>
+constexpr int kStFirstBlock = 64 * (int)sizeof(T);  // 256 or 512
+template <class T, bool SC>
+__global__ __launch_bounds__(kStFirstBlock<T>) void k_st_first(const T* __restrict__ in, T* __restrict__ out,
+                                                  const int32_t* __restrict__ idx, StGeom g) {
+    constexpr int E = kStE<T>;
+    constexpr int BL = kStFirstBlock<T>;
+    constexpr int NW = BL / kWave;
+    constexpr int N = kStChunk / BL;  // elements per lane
+    extern __shared__ uint32_t cnt[];  // [W << cl]
+    __shared__ T win[kStLocal];
+    __shared__ uint32_t wlo[NW], whi[NW];
+    __shared__ uint32_t cov[SC ? kStLocal / 32 : 1];
+    const int t = threadIdx.x, w = t / kWave;
+    const int64_t v0 = (int64_t)blockIdx.x * (kStChunk / E) + t;
+    const uint32_t nall = (uint32_t)g.n;
+    uint32_t pos[N];
+    T val[N];
+    #pragma unroll
+    for (int u = 0; u < N / E; ++u)
+        st_load<uint32_t, E>(reinterpret_cast<const uint32_t*>(idx), v0 + u * BL, g.n, kStNone, pos + E * u);
+    const int cl = st_copies_lg(g.W);
+    for (int i = t; i < (g.WP << cl); i += BL) cnt[i] = 0;
+    if (SC)
+        for (int i = t; i < kStLocal / 32; i += BL) cov[i] = 0;
+    uint32_t lo = kStNone, hi = 0;
+    #pragma unroll
+    for (int e = 0; e < N; ++e)
+        if (pos[e] < nall) {
+            lo = std::min(lo, pos[e]);
+            hi = std::max(hi, pos[e]);
+        }
+    #pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        lo = std::min(lo, (uint32_t)__shfl_xor((int)lo, o));
+        hi = std::max(hi, (uint32_t)__shfl_xor((int)hi, o));
+    }
+    if (lane_id() == 0) {
+        wlo[w] = lo;
+        whi[w] = hi;
+    }
+    __syncthreads();
+    #pragma unroll
+    for (int x = 0; x < NW; ++x) {
+        lo = std::min(lo, wlo[x]);
+        hi = std::max(hi, whi[x]);
+    }
+    // the same in the whole workgroup from here on
+    const bool some = lo <= hi;
+    const bool near = !some || hi - lo < g.near;
+    const bool window = some && hi - lo < (uint32_t)kStLocal;
+    if (t == 0) {
+        g.done[blockIdx.x] = near ? 1 : 0;
+        // read first, and many words: one address that every workgroup stores
+        // to takes them one after the other (35 us at 2^23 elements)
+        uint32_t* w = st_gate(g, blockIdx.x);
+        if (!near && ld_relaxed(w) == 0) st_relaxed(w, 1u);
+    }
+    if (!near) {
+        const uint32_t copy = t & ((1u << cl) - 1u);
+        #pragma unroll
+        for (int e = 0; e < N; ++e)
+            if (pos[e] < nall)
+                __hip_atomic_fetch_add(cnt + ((pos[e] >> g.shift) << cl) + copy, 1u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();
+        uint32_t* row = reinterpret_cast<uint32_t*>(g.count + (int64_t)blockIdx.x * g.WP);
+        for (int i = t; i < g.WP / 2; i += BL) {
+            uint32_t a = 0, b = 0;
+            for (int c = 0; c < (1 << cl); ++c) {
+                a += cnt[((2 * i) << cl) + c];
+                b += cnt[((2 * i + 1) << cl) + c];
+            }
+            row[i] = a | (b << 16);
+        }
+        return;
+    }
+    if constexpr (SC) {
+        #pragma unroll
+        for (int u = 0; u < N / E; ++u) st_load<T, E>(in, v0 + u * BL, g.n, T(0), val + E * u);
+        if (window) {
+            #pragma unroll
+            for (int e = 0; e < N; ++e)
+                if (pos[e] < nall) {
+                    const uint32_t o = pos[e] - lo;
+                    win[o] = val[e];
+                    atomicOr(cov + (o >> 5), 1u << (o & 31));
+                }
+            __syncthreads();
+            for (uint32_t o = t; o <= hi - lo; o += BL)
+                if ((cov[o >> 5] >> (o & 31)) & 1u) out[lo + o] = win[o];
+        } else {
+            #pragma unroll
+            for (int e = 0; e < N; ++e)
+                if (pos[e] < nall) out[pos[e]] = val[e];
+        }
+    } else {
+        if (window) {
+            for (uint32_t o = t; o <= hi - lo; o += BL) win[o] = in[lo + o];
+            __syncthreads();
+            #pragma unroll
+            for (int e = 0; e < N; ++e) val[e] = pos[e] < nall ? win[pos[e] - lo] : T(0);
+        } else {
+            #pragma unroll
+            for (int e = 0; e < N; ++e) val[e] = pos[e] < nall ? in[pos[e]] : T(0);
+        }
+        #pragma unroll
+        for (int u = 0; u < N / E; ++u) {
+            bool ok[E];
+            #pragma unroll
+            for (int k = 0; k < E; ++k) ok[k] = pos[E * u + k] < nall;
+            st_store<T, E>(out, v0 + u * BL, val + E * u, ok);
+        }
+    }
+}
+
+// exclusive prefix over the workgroup's lanes of s, plus carry; carry grows by
+// the sum.  wt: one word per wave.  Two barriers.
+template <int BLOCK>
+__device__ __forceinline__ uint32_t st_block_prefix(uint32_t s, uint32_t* wt, uint32_t& carry) {
+    const int w = threadIdx.x / kWave;
+    const uint32_t inc = wave_inclusive_add(s);
+    if (lane_id() == kWave - 1) wt[w] = inc;
+    __syncthreads();
+    uint32_t before = carry, all = 0;
+    #pragma unroll
+    for (int q = 0; q < BLOCK / kWave; ++q) {
+        before += q < w ? wt[q] : 0u;
+        all += wt[q];
+    }
+    carry += all;
+    __syncthreads();
+    return before + inc - s;
+}
+
+// Prefixes of the windows' counts.  Workgroup = one group of kStGroup tiles,
+// cut into parts of `per` tiles, one lane for two windows of a part: rows[]
+// within the group, gsum[] the group's sums.  The last workgroup to arrive
+// turns gsum[] into positions and sets base[] (and, for a scatter's second
+// split, tile2[] and win2[]).
+template <int CH>
+__global__ __launch_bounds__(kStRowBlock) void k_st_prefix(StGeom g, int lgp) {
+    __shared__ uint32_t part[2 * kStRowBlock], wt[kStRowBlock / kWave], t2s[kStMaxWindows];
+    __shared__ uint8_t fin[kStGroup * CH];
+    __shared__ uint32_t last;
+    const int x = threadIdx.x;
+    const int p = x & ((1 << lgp) - 1), q = x >> lgp;  // windows 2p and 2p + 1, part q
+    const int np = kStRowBlock >> lgp;                 // parts, at most kStGroup
+    const int per = kStGroup / np;
+    const int P = g.WP / 2;
+    const bool in = p < P;
+    const int64_t t0 = (int64_t)blockIdx.x * kStGroup;
+    if (ballot(*st_gate(g, lane_id()) != 0) == 0) {  // the same in every wave
+        if (blockIdx.x == 0 && x == 0) g.base[g.W] = 0;
+        return;
+    }
+    bool open = false;
+    for (int i = x; i < kStGroup * CH; i += kStRowBlock) {
+        fin[i] = t0 * CH + i >= g.chunks || g.done[t0 * CH + i] ? 1 : 0;
+        open = open || !fin[i];
+    }
+    const bool any = __syncthreads_or(open ? 1 : 0) != 0;  // the same in the whole workgroup
+    if (!any) {
+        for (int i = x; i < P; i += kStRowBlock) reinterpret_cast<uint2*>(g.gsum)[(int64_t)blockIdx.x * P + i] = make_uint2(0, 0);
+    } else {
+        const uint32_t* cnt = reinterpret_cast<const uint32_t*>(g.count) + p;
+        uint32_t a = 0, b = 0;
+        auto tile = [&](int t, uint32_t& u, uint32_t& v) {  // the counts of one tile; finished chunks have none
+            #pragma unroll
+            for (int k = 0; k < CH; ++k) {
+                const int64_t c = std::min<int64_t>((t0 + t) * CH + k, g.chunks - 1);
+                const uint32_t y = cnt[c * P];
+                const bool f = fin[t * CH + k] != 0;
+                u += f ? 0u : y & 0xFFFFu;
+                v += f ? 0u : y >> 16;
+            }
+        };
+        if (in) {
+            #pragma unroll 4
+            for (int t = q * per; t < (q + 1) * per; ++t) tile(t, a, b);
+        }
+        part[2 * x] = a;
+        part[2 * x + 1] = b;
+        __syncthreads();
+        a = b = 0;
+        for (int k = 0; k < q; ++k) {
+            a += part[2 * ((k << lgp) + p)];
+            b += part[2 * ((k << lgp) + p) + 1];
+        }
+        if (in) {
+            uint2* rows = reinterpret_cast<uint2*>(g.rows) + p;
+            #pragma unroll 4
+            for (int t = q * per; t < (q + 1) * per; ++t) {
+                if (t0 + t < g.tiles) rows[(t0 + t) * P] = make_uint2(a, b);
+                tile(t, a, b);
+            }
+            if (q == np - 1) reinterpret_cast<uint2*>(g.gsum)[(int64_t)blockIdx.x * P + p] = make_uint2(a, b);
+        }
+    }
+    __syncthreads();
+    if (x == 0) {
+        __threadfence();  // the group's sums before the arrival
+        last = fetch_add(g.arrived, 1u) == gridDim.x - 1 ? 1u : 0u;
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    if (x == 0) st_relaxed(g.arrived, 0u);
+    // the parts now share the groups
+    uint2* gs = reinterpret_cast<uint2*>(g.gsum) + p;
+    const int64_t gper = (g.groups + np - 1) / np;
+    const int64_t g0 = std::min<int64_t>(q * gper, g.groups), g1 = std::min<int64_t>(g0 + gper, g.groups);
+    uint32_t a = 0, b = 0;
+    if (in) {
+        #pragma unroll 16
+        for (int64_t k = g0; k < g1; ++k) {
+            const uint2 y = gs[k * P];
+            a += y.x;
+            b += y.y;
+        }
+    }
+    part[2 * x] = a;
+    part[2 * x + 1] = b;
+    __syncthreads();
+    uint32_t ta = 0, tb = 0, ba = 0, bb = 0;
+    for (int k = 0; k < np; ++k) {
+        const uint32_t ya = part[2 * ((k << lgp) + p)], yb = part[2 * ((k << lgp) + p) + 1];
+        ba += k < q ? ya : 0u;
+        bb += k < q ? yb : 0u;
+        ta += ya;
+        tb += yb;
+    }
+    // the lanes of part 0 hold the windows in order; the others take the
+    // result through part[]
+    const bool lead = q == 0 && in;
+    constexpr uint32_t kTile = CH * kStChunk;
+    uint32_t all = 0, tiles2 = 0;
+    const uint32_t first = st_block_prefix<kStRowBlock>(lead ? ta + tb : 0u, wt, all);
+    const uint32_t na = (ta + kTile - 1) / kTile, nb = (tb + kTile - 1) / kTile;
+    const uint32_t t2 = st_block_prefix<kStRowBlock>(lead ? na + nb : 0u, wt, tiles2);
+    if (lead) {
+        part[2 * p] = first;
+        part[2 * p + 1] = first + ta;
+        g.base[2 * p] = first;  // base[] and tile2[] have room for WP + 1
+        g.base[2 * p + 1] = first + ta;
+        if (g.tile2) {
+            g.tile2[2 * p] = t2s[2 * p] = t2;
+            g.tile2[2 * p + 1] = t2s[2 * p + 1] = t2 + na;
+        }
+    }
+    __syncthreads();
+    if (x == 0) {
+        g.base[g.W] = all;
+        if (g.tile2) g.tile2[g.W] = tiles2;
+    }
+    if (in) {
+        a = part[2 * p] + ba;
+        b = part[2 * p + 1] + bb;
+        #pragma unroll 16
+        for (int64_t k = g0; k < g1; ++k) {
+            const uint2 y = gs[k * P];
+            gs[k * P] = make_uint2(a, b);
+            a += y.x;
+            b += y.y;
+        }
+    }
+    if (g.tile2) {
+        for (uint32_t t = x; t < tiles2; t += kStRowBlock) {
+            int lo = 0, hi = g.W;  // last window whose first tile is at or before t: empty windows have none
+            while (hi - lo > 1) {
+                const int m = (lo + hi) / 2;
+                if (t2s[m] <= t) lo = m;
+                else hi = m;
+            }
+            g.win2[t] = (uint16_t)lo;
+        }
+    }
+}
+
+// LDS of the two splits: [S] indices, then [S] values through the same
+// buffer; counts and offsets of the buckets
+constexpr int kStBuckets = 1024 + 8;
+template <class T, bool SC>
+constexpr size_t st_split_lds() {
+    return (size_t)kStTile<T> * (SC ? sizeof(T) : 4) + 8 * kStBuckets;
+}
+
+// Bucket of an element among B from b0 on; B for one that is none (its shift
+// is above every window: n < 2^31)
+__device__ __forceinline__ uint32_t st_bucket(uint32_t x, int shift, uint32_t b0, uint32_t B) {
+    return std::min((x >> shift) - b0, B);
+}
+
+// Exclusive prefix of cnt[0, C) into off[], C <= 2*kStBlock, two entries per
+// lane; returns the sum.  A barrier before and after.
+__device__ __forceinline__ uint32_t st_scan(uint32_t tid, const uint32_t* cnt, uint32_t* off, int C, uint32_t* wtmp) {
+    const int t = (int)tid, w = __builtin_amdgcn_readfirstlane(t / kWave);
+    __syncthreads();
+    const uint32_t a = 2 * t < C ? cnt[2 * t] : 0u, b = 2 * t + 1 < C ? cnt[2 * t + 1] : 0u;
+    const uint32_t inc = wave_inclusive_add(a + b);
+    if (lane_id() == kWave - 1) wtmp[w] = inc;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+    #pragma unroll
+    for (int q = 0; q < kStBlock / kWave; ++q) {
+        before += q < w ? wtmp[q] : 0u;
+        all += wtmp[q];
+    }
+    const uint32_t x = before + inc - a - b;
+    if (2 * t < C) off[2 * t] = x;
+    if (2 * t + 1 < C) off[2 * t + 1] = x + a;
+    __syncthreads();
+    return all;
+}
+
+// Slots of the lane's elements in bucket order, two per word of at[], from
+// one counter atomic each (1 << cl counters per bucket, taken by lane); off[b
+// << cl] = first slot of bucket b.  Returns the number of elements that are
+// some; the others all get the last slot, which is then past them.
+template <int EPL>
+__device__ __forceinline__ uint32_t st_rank(uint32_t tid, uint32_t (&x)[EPL], uint32_t (&at)[EPL / 2], int shift,
+                                            uint32_t b0, int B, int cl, uint32_t* cnt, uint32_t* off, uint32_t* wtmp) {
+    for (int i = (int)tid; i < ((B + 1) << cl); i += kStBlock) cnt[i] = 0;
+    __syncthreads();
+    const uint32_t copy = tid & ((1u << cl) - 1u);
+    #pragma unroll
+    for (int e = 0; e < EPL / 2; ++e) {
+        const uint32_t r0 = __hip_atomic_fetch_add(cnt + (st_bucket(x[2 * e], shift, b0, (uint32_t)B) << cl) + copy,
+                                                   1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint32_t r1 = __hip_atomic_fetch_add(cnt + (st_bucket(x[2 * e + 1], shift, b0, (uint32_t)B) << cl) + copy,
+                                                   1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        at[e] = r0 | (r1 << 16);
+    }
+    // Packed before the scan, and the buckets worked out again after it: held
+    // across it, ranks and counter addresses do not fit the registers of two
+    // workgroups per CU.
+    #pragma unroll
+    for (int e = 0; e < EPL / 2; ++e) asm volatile("" : "+v"(at[e]), "+v"(x[2 * e]), "+v"(x[2 * e + 1]));
+    constexpr uint32_t kLast = kStBlock * EPL - 1;
+    if (tid < (1u << cl)) off[(B << cl) + tid] = kLast;
+    const uint32_t m = st_scan(tid, cnt, off, B << cl, wtmp);
+    #pragma unroll
+    for (int e = 0; e < EPL / 2; ++e) {
+        const uint32_t o0 = off[(st_bucket(x[2 * e], shift, b0, (uint32_t)B) << cl) + copy];
+        const uint32_t o1 = off[(st_bucket(x[2 * e + 1], shift, b0, (uint32_t)B) << cl) + copy];
+        at[e] = std::min((at[e] & 0xFFFFu) + o0, kLast) | std::min((at[e] >> 16) + o1, kLast) << 16;
+    }
+    return m;
+}
+// v[e] to slot e's place in buf
+template <class V, int EPL>
+__device__ __forceinline__ void st_place(V* buf, const uint32_t (&at)[EPL / 2], const V (&v)[EPL]) {
+    #pragma unroll
+    for (int e = 0; e < EPL / 2; ++e) {
+        buf[at[e] & 0xFFFFu] = v[2 * e];
+        buf[at[e] >> 16] = v[2 * e + 1];
+    }
+}
+// The m slots' indices to their output positions d[] (slot + dlt[bucket]; past
+// the output, where the store is dropped, for the slots of no element)
+template <int EPL>
+__device__ __forceinline__ void st_put_index(uint32_t tid, uint32_t m, const uint32_t* buf, const uint32_t* dlt,
+                                             int shift, uint32_t b0, int B, const BufSink<uint32_t>& out,
+                                             uint32_t (&d)[EPL]) {
+    #pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+        const uint32_t i = tid + j * kStBlock;
+        const uint32_t k = buf[i];
+        const uint32_t p = dlt[st_bucket(k, shift, b0, (uint32_t)B)] + i;
+        d[j] = i < m ? p : kStNone;
+        out.put(d[j], k);
+    }
+}
+
+// The lane's elements of a tile of p (T: the values' type, which sets the
+// layout); in the last tile through a buffer descriptor that ends at n (loads
+// past it read 0)
+template <class T, class V>
+__device__ __forceinline__ void st_load_tile(const V* __restrict__ p, int64_t tile, int64_t n, uint32_t tid,
+                                             V (&x)[kStEpl<T>]) {
+    constexpr int E = kStE<T>;
+    if ((tile + 1) * kStTile<T> <= n) {
+        typedef V vec __attribute__((ext_vector_type(E)));
+        #pragma unroll
+        for (int u = 0; u < kStEpl<T> / E; ++u) {
+            const vec v = ld_stream(reinterpret_cast<const vec*>(p) + st_vec<T>(tile, u, tid));
+            #pragma unroll
+            for (int k = 0; k < E; ++k) x[E * u + k] = v[k];
+        }
+    } else {
+        const int64_t e0 = tile * kStTile<T>;
+        const __amdgpu_buffer_rsrc_t r = buf_rsrc(p + e0, n - e0);
+        const uint32_t l = (tid >> 8) * kStChunk + (tid & 255) * E;
+        #pragma unroll
+        for (int e = 0; e < kStEpl<T>; ++e)
+            x[e] = buf_load<V>(r, l * (uint32_t)sizeof(V),
+                               (uint32_t)((e / 16 * (kStBlock / 256) * kStChunk + e % 16 / E * 256 * E + e % E) * sizeof(V)));
+    }
+}
+// its indices, kStNone for none
+template <class T>
+__device__ __forceinline__ void st_load_idx(const int32_t* __restrict__ idx, int64_t tile, int64_t n, uint32_t mask,
+                                            uint32_t tid, uint32_t (&x)[kStEpl<T>]) {
+    constexpr int E = kStE<T>;
+    const uint32_t nall = (uint32_t)n;
+    st_load_tile<T, uint32_t>(reinterpret_cast<const uint32_t*>(idx), tile, n, tid, x);
+    // elements of the tile before n, less the lane's first one
+    const int left = (int)std::min<int64_t>(n - tile * kStTile<T>, kStTile<T>) -
+                     (int)((tid >> 8) * kStChunk + (tid & 255) * E);
+    #pragma unroll
+    for (int e = 0; e < kStEpl<T>; ++e) {
+        const int l = st_skip(mask, e / 16, tid) ? 0 : left;
+        x[e] = e / 16 * (kStBlock / 256) * kStChunk + e % 16 / E * 256 * E + e % E < l && x[e] < nall ? x[e] : kStNone;
+    }
+}
+
+// Indices (and a scatter's values) of one tile to window order: sidx / sval
+// [gsum[w] + rows[w] ...].  A gather's element keeps its slot in the
+// window-ordered tile in slot[].
+template <class T, bool SC>
+__global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_split(const T* __restrict__ in,
+                                                                       const int32_t* __restrict__ idx, StGeom g,
+                                                                       uint32_t* __restrict__ sidx, T* __restrict__ sval,
+                                                                       uint16_t* __restrict__ slot) {
+    constexpr int CH = kStCh<T>;
+    constexpr int E = kStE<T>;
+    constexpr int EPL = kStEpl<T>;
+    extern __shared__ char smem[];
+    uint32_t* buf = reinterpret_cast<uint32_t*>(smem);
+    T* vbuf = reinterpret_cast<T*>(smem);
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(smem + (size_t)kStTile<T> * (SC ? sizeof(T) : 4));
+    uint32_t* off = cnt + kStBuckets;
+    __shared__ uint32_t wtmp[kStBlock / kWave];
+    if (g.base[g.W] == 0) return;
+    const int64_t tile = st_order(blockIdx.x, (uint32_t)g.tiles, g.xcds);
+    const uint32_t mask = st_done<CH>(g, tile);
+    if (mask == (1u << CH) - 1u) return;
+    const uint32_t tid = threadIdx.x;
+    const int cl = st_copies_lg(g.W);
+    uint32_t at[EPL / 2], m;
+    {
+        uint32_t x[EPL];
+        st_load_idx<T>(idx, tile, g.n, mask, tid, x);
+        m = st_rank<EPL>(tid, x, at, g.shift, 0u, g.W, cl, cnt, off, wtmp);
+        st_place<uint32_t, EPL>(buf, at, x);
+    }
+    if (!SC) {
+        // the workspace holds whole tiles
+        #pragma unroll
+        for (int u = 0; u < EPL / E; ++u) {
+            if (st_skip(mask, u / (16 / E), tid)) continue;
+            if constexpr (E == 4)
+                st_stream((uint64_t)at[2 * u + 1] << 32 | at[2 * u], reinterpret_cast<uint64_t*>(slot) + st_vec<T>(tile, u, tid));
+            else
+                st_stream(at[u], reinterpret_cast<uint32_t*>(slot) + st_vec<T>(tile, u, tid));
+        }
+    }
+    __syncthreads();
+    // cnt[w] becomes the distance from slot to output position
+    const uint32_t* gs = g.gsum + tile / kStGroup * g.WP;
+    const uint32_t* rw = g.rows + tile * g.WP;
+    for (int i = (int)tid; i < g.W; i += kStBlock) cnt[i] = gs[i] + rw[i] - off[i << cl];
+    T val[EPL];
+    if (SC) st_load_tile<T, T>(in, tile, g.n, tid, val);
+    __syncthreads();
+    uint32_t d[EPL];
+    st_put_index<EPL>(tid, m, buf, cnt, g.shift, 0u, g.W, buf_sink(sidx, g.n), d);
+    if constexpr (SC) {
+        __syncthreads();
+        st_place<T, EPL>(vbuf, at, val);
+        __syncthreads();
+        const BufSink<T> sink = buf_sink(sval, g.n);
+        #pragma unroll
+        for (int j = 0; j < EPL; ++j) sink.put(d[j], vbuf[tid + j * kStBlock]);
+    }
+}
+
+// A second-level tile: elements [lo, hi) of one window's stretch of the
+// window order; t is its number among the window's nt tiles.
+struct StTile2 {
+    int w;
+    uint32_t lo, hi, t, nt;
+};
+template <int S>
+__device__ __forceinline__ void st_tile2(const StGeom& g, uint32_t tile, StTile2& r) {
+    const int a = g.win2[tile];
+    r.w = a;
+    r.t = tile - g.tile2[a];
+    r.nt = g.tile2[a + 1] - g.tile2[a];
+    r.lo = g.base[a] + r.t * (uint32_t)S;
+    r.hi = std::min(r.lo + (uint32_t)S, g.base[a + 1]);
+}
+
+// bin counts of the second-level tiles
+template <class T>
+__global__ __launch_bounds__(kStBlock) void k_st_hist2(StGeom g, const uint32_t* __restrict__ sidx) {
+    constexpr int S = kStTile<T>;
+    __shared__ uint32_t cnt[kStBuckets];
+    if (g.base[g.W] == 0) return;
+    const uint32_t tiles = g.tile2[g.W];
+    if (blockIdx.x >= tiles) return;
+    const int B = 1 << g.lg_subs;
+    const int cl = st_copies_lg(B);
+    StTile2 r;
+    st_tile2<S>(g, st_order(blockIdx.x, tiles, g.xcds), r);
+    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sidx + r.lo, r.hi - r.lo);
+    uint32_t x[kStEpl<T>];
+    #pragma unroll
+    for (int j = 0; j < kStEpl<T>; ++j) x[j] = buf_load<uint32_t>(rs, threadIdx.x * 4, j * kStBlock * 4);
+    for (int i = threadIdx.x; i < (B << cl); i += kStBlock) cnt[i] = 0;
+    __syncthreads();
+    const uint32_t b0 = (uint32_t)r.w << g.lg_subs, copy = threadIdx.x & ((1u << cl) - 1u);
+    #pragma unroll
+    for (int j = 0; j < kStEpl<T>; ++j)
+        if (threadIdx.x + j * kStBlock < r.hi - r.lo)
+            __hip_atomic_fetch_add(cnt + (((x[j] >> g.sub_shift) - b0) << cl) + copy, 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+    __syncthreads();
+    uint32_t* rows = g.rows2 + ((int64_t)g.tile2[r.w] << g.lg_subs) + r.t;
+    for (int i = threadIdx.x; i < B; i += kStBlock) {
+        uint32_t s = 0;
+        for (int c = 0; c < (1 << cl); ++c) s += cnt[(i << cl) + c];
+        rows[(int64_t)i * r.nt] = s;
+    }
+}
+
+// One window's bin counts become output positions; the bins' first positions
+__global__ __launch_bounds__(kStRowBlock) void k_st_rows2(StGeom g) {
+    __shared__ uint32_t wt[kStRowBlock / kWave];
+    if (g.base[g.W] == 0) return;
+    const int w = blockIdx.x;
+    const uint32_t nt = g.tile2[w + 1] - g.tile2[w];
+    uint32_t* rows = g.rows2 + ((int64_t)g.tile2[w] << g.lg_subs);
+    const int64_t len = (int64_t)nt << g.lg_subs;
+    uint32_t carry = g.base[w];
+    if (nt == 0)
+        for (int i = threadIdx.x; i < (1 << g.lg_subs); i += kStRowBlock) g.bins[((int64_t)w << g.lg_subs) + i] = carry;
+    for (int64_t b = 0; b < len; b += kStRowBlock * 4) {
+        uint32_t x[4], s = 0;
+        const int64_t i0 = b + (int64_t)threadIdx.x * 4;
+        #pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            x[k] = i0 + k < len ? rows[i0 + k] : 0u;
+            s += x[k];
+        }
+        uint32_t y = st_block_prefix<kStRowBlock>(s, wt, carry);
+        #pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (i0 + k < len) {
+                rows[i0 + k] = y;
+                if ((i0 + k) % nt == 0) g.bins[((int64_t)w << g.lg_subs) + (i0 + k) / nt] = y;
+            }
+            y += x[k];
+        }
+    }
+}
+
+// One second-level tile to bin order
+template <class T>
+__global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_split2(StGeom g, const uint32_t* __restrict__ sidx,
+                                                                        const T* __restrict__ sval,
+                                                                        uint32_t* __restrict__ didx,
+                                                                        T* __restrict__ dval) {
+    constexpr int S = kStTile<T>;
+    constexpr int EPL = kStEpl<T>;
+    extern __shared__ char smem[];
+    uint32_t* buf = reinterpret_cast<uint32_t*>(smem);
+    T* vbuf = reinterpret_cast<T*>(smem);
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(smem + (size_t)S * sizeof(T));
+    uint32_t* off = cnt + kStBuckets;
+    __shared__ uint32_t wtmp[kStBlock / kWave];
+    if (g.base[g.W] == 0) return;
+    const uint32_t tiles = g.tile2[g.W];
+    if (blockIdx.x >= tiles) return;
+    const int B = 1 << g.lg_subs;
+    const int cl = st_copies_lg(B);
+    StTile2 r;
+    st_tile2<S>(g, st_order(blockIdx.x, tiles, g.xcds), r);
+    const uint32_t b0 = (uint32_t)r.w << g.lg_subs;
+    const uint32_t have = r.hi - r.lo;
+    const uint32_t tid = threadIdx.x;
+    uint32_t at[EPL / 2];
+    {
+        uint32_t x[EPL];
+        const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sidx + r.lo, have);
+        #pragma unroll
+        for (int j = 0; j < EPL; ++j) x[j] = buf_load<uint32_t>(rs, tid * 4, j * kStBlock * 4);
+        #pragma unroll
+        for (int j = 0; j < EPL; ++j) x[j] = tid + j * kStBlock < have ? x[j] : kStNone;
+        st_rank<EPL>(tid, x, at, g.sub_shift, b0, B, cl, cnt, off, wtmp);
+        st_place<uint32_t, EPL>(buf, at, x);
+    }
+    __syncthreads();
+    const uint32_t* rows = g.rows2 + ((int64_t)g.tile2[r.w] << g.lg_subs) + r.t;
+    for (int i = (int)tid; i < B; i += kStBlock) cnt[i] = rows[(int64_t)i * r.nt] - off[i << cl];
+    T val[EPL];
+    const __amdgpu_buffer_rsrc_t rv = buf_rsrc(sval + r.lo, have);
+    #pragma unroll
+    for (int j = 0; j < EPL; ++j) val[j] = buf_load<T>(rv, tid * (uint32_t)sizeof(T), j * kStBlock * (uint32_t)sizeof(T));
+    __syncthreads();
+    uint32_t d[EPL];
+    st_put_index<EPL>(tid, have, buf, cnt, g.sub_shift, b0, B, buf_sink(didx, g.n), d);
+    __syncthreads();
+    st_place<T, EPL>(vbuf, at, val);
+    __syncthreads();
+    const BufSink<T> sink = buf_sink(dval, g.n);
+    #pragma unroll
+    for (int j = 0; j < EPL; ++j) sink.put(d[j], vbuf[tid + j * kStBlock]);
+}
+
+// out[didx[j]] = dval[j] for one bin of kStBin bytes of the output, through
+// LDS: every covered line leaves whole
+constexpr int kStBinBlock = 1024;
+template <class T>
+__global__ __launch_bounds__(kStBinBlock, kStBinBlock / 128) void k_st_bins(StGeom g, const uint32_t* __restrict__ first,
+                                                                            int64_t nbins,
+                                                                            const uint32_t* __restrict__ didx,
+                                                                            const T* __restrict__ dval,
+                                                                            T* __restrict__ out) {
+    constexpr int E = kStBin / (int)sizeof(T);
+    extern __shared__ char smem[];
+    T* win = reinterpret_cast<T*>(smem);                              // [E]
+    uint32_t* cov = reinterpret_cast<uint32_t*>(smem + kStBin);       // [E / 32]
+    if (g.base[g.W] == 0) return;
+    st_close(g);
+    for (uint32_t ob = blockIdx.x; ob < (uint32_t)nbins; ob += gridDim.x) {
+    const int64_t bin = st_order(ob, (uint32_t)nbins, g.xcds);
+    const uint32_t m = std::min<uint32_t>(g.base[g.W], (uint32_t)g.n);
+    const uint32_t lo = std::min(first[bin], m), hi = bin + 1 < nbins ? std::min(first[bin + 1], m) : m;
+    if (lo >= hi) continue;  // the same in the whole workgroup
+    const uint32_t o0 = (uint32_t)bin * (uint32_t)E;
+    for (int i = threadIdx.x; i < E / 32; i += kStBinBlock) cov[i] = 0;
+    __syncthreads();
+    for (uint32_t b = lo; b < hi; b += kStBinBlock * 8) {
+        uint32_t x[8];
+        T v[8];
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t e = b + threadIdx.x + j * kStBinBlock;
+            x[j] = e < hi ? ld_stream(didx + e) : kStNone;
+            v[j] = e < hi ? ld_stream(dval + e) : T(0);
+        }
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t o = x[j] - o0;
+            if (o < (uint32_t)E) {
+                win[o] = v[j];
+                atomicOr(cov + (o >> 5), 1u << (o & 31));
+            }
+        }
+    }
+    __syncthreads();
+    constexpr int V = kStE<T>;
+    for (int q = threadIdx.x; q < E / V; q += kStBinBlock) {
+        const uint32_t c = cov[q / (32 / V)] >> (V * (q % (32 / V)));
+        T v[V];
+        bool ok[V];
+        #pragma unroll
+        for (int k = 0; k < V; ++k) {
+            v[k] = win[V * q + k];
+            ok[k] = (c >> k) & 1u;  // positions at or past n are never covered
+        }
+        st_store<T, V>(out, (int64_t)(o0 / V) + q, v, ok);
+    }
+    __syncthreads();
+    }
+}
+
+// sval[j] = in[sidx[j]]: workgroups of one XCD walk one range of the window
+// order, so the windows being read at one time are few and stay in its L2
+template <class T>
+constexpr int kStGe = 128 / (int)sizeof(T);  // staged elements per lane
+template <class T>
+constexpr int kStPart = 256 * kStGe<T>;      // and per workgroup
+template <class T>
+__global__ __launch_bounds__(256) void k_st_gather(const T* __restrict__ in, StGeom g,
+                                                   const uint32_t* __restrict__ sidx, T* __restrict__ sval) {
+    constexpr int E = kStE<T>;
+    if (g.base[g.W] == 0) return;
+    const int64_t m = std::min<int64_t>(g.base[g.W], g.n);
+    const uint32_t parts = (uint32_t)((m + kStPart<T> - 1) / kStPart<T>);
+    if (blockIdx.x >= parts) return;
+    const int64_t v0 = (int64_t)st_order(blockIdx.x, parts, g.xcds) * (kStPart<T> / E) + threadIdx.x;
+    const uint32_t nall = (uint32_t)g.n;
+    uint32_t pos[kStGe<T>];
+    T val[kStGe<T>];
+    #pragma unroll
+    for (int u = 0; u < kStGe<T> / E; ++u) st_load<uint32_t, E>(sidx, v0 + u * 256, m, kStNone, pos + E * u);
+    #pragma unroll
+    for (int e = 0; e < kStGe<T>; ++e) val[e] = pos[e] < nall ? in[pos[e]] : T(0);
+    #pragma unroll
+    for (int u = 0; u < kStGe<T> / E; ++u) {
+        bool ok[E];
+        #pragma unroll
+        for (int k = 0; k < E; ++k) ok[k] = E * (v0 + u * 256) + k < m;
+        st_store<T, E>(sval, v0 + u * 256, val + E * u, ok);
+    }
+}
+
+// A gather's values back into order: the tile's runs of sval are copied to
+// LDS slot by slot, then every element takes its slot's value.  first[] holds
+// the window of every kStStep-th slot; runs are longer than that on average,
+// so two steps from there reach a slot's window but for a few.
+constexpr int kStStep = 8;
+template <class T>
+constexpr size_t st_return_lds() {
+    return (size_t)kStTile<T> * sizeof(T) + 8 * kStBuckets + kStTile<T> / kStStep * 2;
+}
+template <class T>
+__global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_return(T* __restrict__ out, StGeom g,
+                                                                        const T* __restrict__ sval,
+                                                                        const uint16_t* __restrict__ slot) {
+    constexpr int CH = kStCh<T>;
+    constexpr int E = kStE<T>;
+    constexpr int EPL = kStEpl<T>;
+    extern __shared__ char smem[];
+    T* vbuf = reinterpret_cast<T*>(smem);                                                // [tile]
+    uint32_t* end = reinterpret_cast<uint32_t*>(smem + (size_t)kStTile<T> * sizeof(T));  // [W] counts, then slot ends
+    uint32_t* dlt = end + kStBuckets;                                 // [W] slot starts, then slot to position
+    uint16_t* first = reinterpret_cast<uint16_t*>(dlt + kStBuckets);  // [tile / kStStep]
+    __shared__ uint32_t wtmp[kStBlock / kWave];
+    if (g.base[g.W] == 0) return;
+    st_close(g);
+    const uint32_t nall = (uint32_t)g.n;
+    const int64_t tile = st_order(blockIdx.x, (uint32_t)g.tiles, g.xcds);
+    const uint32_t mask = st_done<CH>(g, tile);
+    if (mask == (1u << CH) - 1u) return;
+    const uint32_t tid = threadIdx.x;
+    uint32_t sl[EPL / 2];  // two slots per word
+    #pragma unroll
+    for (int u = 0; u < EPL / E; ++u) {
+        const bool skip = st_skip(mask, u / (16 / E), tid);
+        if constexpr (E == 4) {
+            const uint64_t p = skip ? ~0ull : ld_stream(reinterpret_cast<const uint64_t*>(slot) + st_vec<T>(tile, u, tid));
+            sl[2 * u] = (uint32_t)p;
+            sl[2 * u + 1] = (uint32_t)(p >> 32);
+        } else {
+            sl[u] = skip ? ~0u : ld_stream(reinterpret_cast<const uint32_t*>(slot) + st_vec<T>(tile, u, tid));
+        }
+    }
+    for (int i = (int)tid; i < g.W; i += kStBlock) {
+        uint32_t s = 0;
+        #pragma unroll
+        for (int q = 0; q < CH; ++q)  // chunks past the last one are marked done
+            if (!((mask >> q) & 1u)) s += g.count[(tile * CH + q) * g.WP + i];
+        end[i] = std::min<uint32_t>(s, (uint32_t)kStTile<T>);
+    }
+    const uint32_t m = std::min<uint32_t>(st_scan(tid, end, dlt, g.W, wtmp), (uint32_t)kStTile<T>);
+    for (int i = (int)tid; i < g.W; i += kStBlock) {
+        const uint32_t a = dlt[i], e = std::min<uint32_t>(a + end[i], (uint32_t)kStTile<T>);
+        for (uint32_t k = (a + kStStep - 1) / kStStep; k * kStStep < e; ++k) first[k] = (uint16_t)i;
+        end[i] = e;
+        dlt[i] = g.gsum[tile / kStGroup * g.WP + i] + g.rows[tile * g.WP + i] - a;
+    }
+    __syncthreads();
+    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sval, g.n);
+    #pragma unroll
+    for (int h = 0; h < EPL; h += 8) {  // eight slots at a time
+        uint32_t w[8];
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t i = tid + (h + j) * kStBlock;
+            w[j] = first[std::min(i, m - 1) / kStStep];  // m > 0: some chunk is not finished
+        }
+        #pragma unroll
+        for (int r = 0; r < 2; ++r)
+            #pragma unroll
+            for (int j = 0; j < 8; ++j)
+                w[j] += std::min<uint32_t>(tid + (h + j) * kStBlock, m - 1) >= end[w[j]] ? 1u : 0u;
+        T v[8];
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t i = std::min<uint32_t>(tid + (h + j) * kStBlock, m - 1);
+            while (i >= end[w[j]]) ++w[j];  // ends at the latest at the last window, whose end is m
+            v[j] = buf_load<T>(rs, std::min(dlt[w[j]] + i, nall) * (uint32_t)sizeof(T));
+        }
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) vbuf[tid + (h + j) * kStBlock] = v[j];
+    }
+    __syncthreads();
+    #pragma unroll
+    for (int u = 0; u < EPL / E; ++u) {
+        T y[E];
+        bool ok[E];
+        #pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const int e = E * u + k;
+            const uint32_t s = e & 1 ? sl[e / 2] >> 16 : sl[e / 2] & 0xFFFFu;
+            ok[k] = s < m;
+            y[k] = vbuf[ok[k] ? s : 0u];
+        }
+        st_store<T, E>(out, st_vec<T>(tile, u, tid), y, ok);
+    }
+}
+
+struct StBufs {
+    uint32_t *sidx, *didx;  // window order; a scatter's bin order
+    void *sval, *dval;
+    uint16_t* slot;
+};
+
+template <class T, bool SC>
+int run_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, const StGeom& g, const StBufs& b, int64_t nbins) {
+    constexpr int CH = kStCh<T>;
+    const unsigned grid = (unsigned)g.tiles;
+    constexpr size_t l3 = st_split_lds<T, SC>();
+    const size_t l1 = ((size_t)g.WP << st_copies_lg(g.W)) * 4;
+    T* sval = static_cast<T*>(b.sval);
+    int lgp = 4;  // at most one part per tile
+    while ((2 << lgp) < g.WP) ++lgp;
+    EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_split<T, SC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l3));
+    hipLaunchKernelGGL((k_st_first<T, SC>), dim3((unsigned)g.chunks), dim3(kStFirstBlock<T>), l1, c->stream, in, out, idx, g);
+    hipLaunchKernelGGL((k_st_prefix<CH>), dim3((unsigned)g.groups), dim3(kStRowBlock), 0, c->stream, g, lgp);
+    hipLaunchKernelGGL((k_st_split<T, SC>), dim3(grid), dim3(kStBlock), l3, c->stream, in, idx, g, b.sidx, sval, b.slot);
+    if constexpr (SC) {
+        const uint32_t* first = g.base;
+        const uint32_t* fidx = b.sidx;
+        const T* fval = sval;
+        if (g.tile2) {
+            const unsigned grid2 = (unsigned)(g.tiles + g.W);  // a window's last tile may be short
+            EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_split2<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l3));
+            hipLaunchKernelGGL((k_st_hist2<T>), dim3(grid2), dim3(kStBlock), 0, c->stream, g, (const uint32_t*)b.sidx);
+            hipLaunchKernelGGL(k_st_rows2, dim3((unsigned)g.W), dim3(kStRowBlock), 0, c->stream, g);
+            hipLaunchKernelGGL((k_st_split2<T>), dim3(grid2), dim3(kStBlock), l3, c->stream, g, (const uint32_t*)b.sidx,
+                               (const T*)sval, b.didx, static_cast<T*>(b.dval));
+            first = g.bins;
+            fidx = b.didx;
+            fval = static_cast<const T*>(b.dval);
+        }
+        constexpr size_t l6 = kStBin + kStBin / sizeof(T) / 8;
+        EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_bins<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l6));
+        hipLaunchKernelGGL((k_st_bins<T>), dim3((unsigned)std::min<int64_t>(nbins, (int64_t)std::max(c->cus, 1) * 4)),
+                           dim3(kStBinBlock), l6, c->stream, g, first, nbins, fidx, fval, out);
+    } else {
+        constexpr size_t l5 = st_return_lds<T>();
+        EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_return<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l5));
+        hipLaunchKernelGGL((k_st_gather<T>), dim3((unsigned)ceil_div(g.n, (int64_t)kStPart<T>)), dim3(256), 0, c->stream, in,
+                           g, (const uint32_t*)b.sidx, sval);
+        hipLaunchKernelGGL((k_st_return<T>), dim3(grid), dim3(kStBlock), l5, c->stream, out, g, (const T*)sval,
+                           (const uint16_t*)b.slot);
+    }
+    EDPP_HIP(c, hipGetLastError());
+    return EDPP_OK;
+}
+
+int st_ceil_lg(int64_t x) {
+    int l = 0;
+    while ((1ll << l) < x) ++l;
+    return l;
+}
+
+}  // namespace
+
+template <class T>
+int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t n, bool scatter, bool* ran) {
+    *ran = false;
+    if (!gs_staged_applies(in, out, idx, n, (int)sizeof(T), scatter)) return EDPP_OK;
+    constexpr int64_t S = kStTile<T>;
+    StGeom g = {};
+    g.n = n;
+    g.chunks = ceil_div(n, (int64_t)kStChunk);
+    g.tiles = ceil_div(n, S);
+    g.groups = ceil_div(g.tiles, (int64_t)kStGroup);
+    g.xcds = c->xcds;
+    g.near = (uint32_t)(kStWindow / (int64_t)sizeof(T));
+    bool two = false;
+    int64_t nbins = 0;
+    if (!scatter) {
+        g.shift = st_ceil_lg(kStWindow / (int64_t)sizeof(T));
+    } else {
+        g.sub_shift = st_ceil_lg(kStBin / (int64_t)sizeof(T));
+        nbins = ceil_div(n, 1ll << g.sub_shift);
+        two = nbins > kStOneLevel;
+        g.lg_subs = two ? st_ceil_lg(nbins) / 2 : 0;
+        g.shift = g.sub_shift + g.lg_subs;
+    }
+    g.W = (int)ceil_div(n, 1ll << g.shift);
+    g.WP = (g.W + 1) & ~1;
+    const int64_t tiles2 = two ? g.tiles + g.W : 0;
+    // workspace, in this order
+    size_t at = 0;
+    auto take = [&at](size_t bytes) {
+        const size_t p = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return p;
+    };
+    const size_t o_done = take((size_t)(g.tiles * S / kStChunk)), o_count = take((size_t)g.chunks * g.WP * 2),
+                 o_rows = take((size_t)g.tiles * g.WP * 4), o_gsum = take((size_t)g.groups * g.WP * 4), o_base = take(((size_t)g.WP + 1) * 4),
+                 o_tile2 = take(((size_t)g.WP + 1) * 4), o_win2 = take((size_t)tiles2 * 2), o_rows2 = take(((size_t)tiles2 << g.lg_subs) * 4),
+                 o_bins = take(((size_t)g.W << g.lg_subs) * 4), o_sidx = take((size_t)n * 4),
+                 o_sval = take((size_t)n * sizeof(T)), o_didx = take(two ? (size_t)n * 4 : 0),
+                 o_dval = take(two ? (size_t)n * sizeof(T) : 0), o_slot = take(scatter ? 0 : (size_t)g.tiles * S * 2);
+    if (at > c->ws_bytes) {
+        // a stream under capture must not allocate: the direct passes then run
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess) {
+            (void)hipGetLastError();  // some other capture forbids the question
+            return EDPP_OK;
+        }
+        if (cap != hipStreamCaptureStatusNone) return EDPP_OK;
+    }
+    void* w;
+    int rc = ws_reserve(c, at, &w);
+    if (rc == EDPP_ENOMEM) {  // the direct passes need no copies
+        (void)hipGetLastError();
+        return EDPP_OK;
+    }
+    if (rc) return rc;
+    char* p = static_cast<char*>(w);
+    auto u32 = [p](size_t o) { return reinterpret_cast<uint32_t*>(p + o); };
+    g.done = reinterpret_cast<uint8_t*>(p + o_done);
+    g.count = reinterpret_cast<uint16_t*>(p + o_count);
+    g.rows = u32(o_rows);
+    g.gsum = u32(o_gsum);
+    g.base = u32(o_base);
+    if (two) {
+        g.tile2 = u32(o_tile2);
+        g.win2 = reinterpret_cast<uint16_t*>(p + o_win2);
+        g.rows2 = u32(o_rows2);
+        g.bins = u32(o_bins);
+    }
+    const StBufs b = {u32(o_sidx), u32(o_didx), p + o_sval, p + o_dval, reinterpret_cast<uint16_t*>(p + o_slot)};
+    g.gate = c->gs_gate;
+    g.arrived = c->gs_gate + kStGates * kStGatePad;
+    *ran = true;
+    return scatter ? run_staged<T, true>(c, in, out, idx, g, b, nbins)
+                   : run_staged<T, false>(c, in, out, idx, g, b, 0);
+}
+
+// A call whose chunks all turn out local pays for the kernels behind the first
+// one, which return at once (2 to 9 us each with their dispatch), but not for
+// the later passes of the direct schedule.  us, direct / staged:
+//                      random permutation    4096-element blocks
+//   gather  4 B  2^26      1297 /  657           113 / 127
+//   gather  4 B  2^27      2581 / 1332           292 / 311
+//   gather  4 B  2^28      5464 / 2780           567 / 598
+//   scatter 4 B  2^26      1245 /  670           128 / 135
+//   scatter 4 B  2^27      2277 / 1376           347 / 331
+//   scatter 4 B  2^28      4485 / 2810           690 / 657
+//   gather  8 B  2^23       162 /  119            35 /  31
+//   gather  8 B  2^26      1327 /  870           283 / 247
+//   gather  8 B  2^27      2922 / 1822           554 / 484
+//   scatter 8 B  2^24       302 /  247            58 /  62
+//   scatter 8 B  2^26      1398 / 1021           286 / 279
+//   scatter 8 B  2^27      2798 / 2106           570 / 549
+// So calls start at 512 MiB, from where a local gather and scatter together
+// take no longer than before (4 B, 2^26: 262 against 241 us), and gathers of
+// 8-byte elements, whose local chunks got faster, at 64 MiB.  The upper bound
+// is 1024 windows, and byte offsets of 31 bits.
+bool gs_staged_applies(const void* in, const void* out, const int32_t* idx, int64_t n, int elem_bytes, bool scatter) {
+    const int64_t bytes = n * elem_bytes;
+    const int64_t least = (elem_bytes == 8 && !scatter ? 64ll : 512ll) << 20;
+    return aligned16(in) && aligned16(out) && aligned16(idx) && bytes >= least && bytes <= kStWindow * kStMaxWindows &&
+           bytes < (1ll << 31);
+}
+
+template int launch_gs_staged<uint32_t>(edpp_ctx*, const uint32_t*, uint32_t*, const int32_t*, int64_t, bool, bool*);
+template int launch_gs_staged<uint64_t>(edpp_ctx*, const uint64_t*, uint64_t*, const int32_t*, int64_t, bool, bool*);
+
+}  // namespace edpp

@@ -596,7 +596,9 @@ int edpp_call_run(edpp_ctx* c, const edpp_call* q, int32_t cand, double* ms) {
     if (rc) return rc;
     if (q->n > 0) {
         if (cand < 0) {
-            if (c->model) {
+            const bool staged = (q->op == EDPP_OP_GATHER || q->op == EDPP_OP_SCATTER) &&
+                                gs_staged_applies(q->in, q->out, q->idx, q->n, q->elem_bytes, q->op == EDPP_OP_SCATTER);
+            if (c->model && !staged) {
                 int k;
                 rc = model_choose(c, *q, &k);
                 if (!rc) rc = run_candidate(c, *q, k, nullptr);

@@ -145,7 +145,12 @@ int edpp_stream_i32(edpp_ctx* ctx, int op, const int32_t* a, const int32_t* b,
 /* ---- multi-pass gather / scatter ----------------------------------------
  * opencl/primitives/gatherImpl.cpp:7-55, scatterImpl.cpp:9-54.  Pass k of
  * `passes` touches only indices in [k*ceil(n/passes), (k+1)*ceil(n/passes)).
- * passes == 0 picks the count from the context's schedule (tuner or model).
+ * passes == 0 picks the count from the context's schedule (tuner or model);
+ * calls on large tables (512 MiB to 2 GiB; gathers of 8-byte elements from
+ * 64 MiB) then order their indices by windows of the random side in the
+ * context's workspace instead (up to 24 bytes per element), unless that
+ * memory is not to be had or the stream is under capture and the workspace
+ * too small; the output is the same.
  * idx must hold values in [0,n); for scatter it must be a permutation.      */
 int edpp_gather_i32 (edpp_ctx* ctx, const int32_t* in, int32_t* out, const int32_t* idx,
                      int64_t n, int passes, double* ms);
@@ -155,8 +160,9 @@ int edpp_gather_i64 (edpp_ctx* ctx, const int64_t* in, int64_t* out, const int32
                      int64_t n, int passes, double* ms);
 int edpp_scatter_i64(edpp_ctx* ctx, const int64_t* in, int64_t* out, const int32_t* idx,
                      int64_t n, int passes, double* ms);
-/* The pass count a passes == 0 call on n elements of elem_bytes (4 or 8) uses
- * while no cost model is set (the built-in schedule).  No reference
+/* The pass count of the built-in schedule for n elements of elem_bytes (4 or
+ * 8): what a passes == 0 call uses while no cost model is set, where it runs
+ * in passes.  No reference
  * counterpart: the reference always takes the pass count from its caller.   */
 int edpp_default_passes(edpp_ctx* ctx, int64_t n, int elem_bytes, int scatter, int* passes);
 
