@@ -29,7 +29,7 @@ struct edpp_ctx {
     uint64_t* scan_status64 = nullptr;  // u64 scans: two tagged words per tile
     int64_t scan_cap_tiles = 0;
     uint32_t* tickets = nullptr;        // [2]
-    uint32_t* gs_gate = nullptr;        // kGsGateBytes of flags and a counter of the staged gather / scatter, 0 between calls
+    uint32_t* gs_gate = nullptr;        // kGsGateBytes of flags of the window-ordered gather / scatter, 0 between calls
     int32_t* d_err = nullptr;           // device error word written by watchdogs
     uint32_t epoch = 1;                 // 30-bit, 0 never used
     // chained split: per-tile, per-bucket status words tagged like the scan's,
@@ -98,7 +98,7 @@ int launch_gather(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t 
 template <class T>
 int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t n, bool scatter, bool* ran);
 bool gs_staged_applies(const void* in, const void* out, const int32_t* idx, int64_t n, int elem_bytes, bool scatter);
-constexpr size_t kGsGateBytes = 65 * 128;
+constexpr size_t kGsGateBytes = 64 * 128;
 int noalloc_setup(edpp_ctx* c);
 int launch_scan_lookback_u32_on(edpp_ctx* c, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* d_total,
                                 uint64_t* status, int64_t status_cap, uint32_t* tickets);

@@ -15,7 +15,7 @@
 // bins of 64 KiB of output, which it assembles in LDS.
 //   k_st_first   one read of the indices: chunks that are local are done at
 //                once; the others' elements are counted per window
-//   k_st_prefix  the counts become positions
+//   k_st_groups, k_st_totals   prefixes of the counts
 //   k_st_split   indices (scatter: and values) to window order, tile by tile
 //                through LDS; a gather keeps each element's slot in its tile
 //   gather:      k_st_gather    values, window after window
@@ -38,20 +38,17 @@
 #include "ctx.hpp"
 #include "device.hpp"
 #include "split_tile.hpp"
+#include "window_tile.hpp"
 
 namespace edpp {
 
 namespace {
 
 constexpr int64_t kStWindow = 2 << 20;    // bytes of the random side per window (an XCD's L2 holds 4 MiB)
-constexpr int kStMaxWindows = 1024;
 constexpr int kStBin = 64 << 10;          // bytes of the output a scatter's workgroup assembles in LDS
 constexpr int kStOneLevel = 1024;         // bins up to which a scatter splits once (2^24 4-byte elements: 151 against
                                           // 167 us in two, with 32 windows of 32 bins)
 constexpr int kStLocal = 4096;            // elements of a local chunk's LDS window
-constexpr int kStBlock = 512;              // lanes of the splits and the return
-constexpr uint32_t kStNone = 0xFFFFFFFFu; // no element / index out of range
-constexpr int kStRowBlock = 1024;
 
 // Elements per 16-byte vector of T: 4 or 2.  A lane's step is one such vector
 // of values (and 16 or 8 bytes of indices), so that a wave's accesses are
@@ -59,76 +56,16 @@ constexpr int kStRowBlock = 1024;
 template <class T>
 constexpr int kStE = 16 / (int)sizeof(T);
 
-// elements [v*E, v*E + E) of p; `none` for the ones at or past n
-template <class T, int E>
-__device__ __forceinline__ void st_load(const T* __restrict__ p, int64_t v, int64_t n, T none, T* x) {
-    if (E * v + E <= n) {
-        typedef T vec __attribute__((ext_vector_type(E)));
-        const vec y = ld_stream(reinterpret_cast<const vec*>(p) + v);
-        #pragma unroll
-        for (int k = 0; k < E; ++k) x[k] = y[k];
-    } else {
-        #pragma unroll
-        for (int k = 0; k < E; ++k) x[k] = E * v + k < n ? p[E * v + k] : none;
-    }
-}
-// p[E*v + k] = x[k] where ok[k] (elements at or past n are never ok)
-template <class T, int E>
-__device__ __forceinline__ void st_store(T* __restrict__ p, int64_t v, const T* x, const bool* ok) {
-    bool all = true;
-    #pragma unroll
-    for (int k = 0; k < E; ++k) all = all && ok[k];
-    if (all) {
-        typedef T vec __attribute__((ext_vector_type(E)));
-        vec y;
-        #pragma unroll
-        for (int k = 0; k < E; ++k) y[k] = x[k];
-        st_stream(y, reinterpret_cast<vec*>(p) + v);
-    } else {
-        #pragma unroll
-        for (int k = 0; k < E; ++k)
-            if (ok[k]) p[E * v + k] = x[k];
-    }
-}
-
 // What every kernel of one call shares.  The indices are cut into chunks of
 // 4096 and tiles of 64 KiB of values (4 or 2 chunks, kStEpl elements for each
 // lane of the splits); lane t's elements [16h, 16h + 16) of a tile are vectors
-// u*256 + t%256 of chunk 2h + t/256.  Prefixes over the tiles are kept for
-// groups of kStGroup tiles.
-constexpr int kStChunk = 4096;
+// u*256 + t%256 of chunk 2h + t/256.
 template <class T>
 constexpr int kStEpl = 128 / (int)sizeof(T);
 template <class T>
 constexpr int kStTile = kStBlock * kStEpl<T>;
 template <class T>
 constexpr int kStCh = kStTile<T> / kStChunk;
-constexpr int kStGroup = 64;
-constexpr int kStGates = 64, kStGatePad = 32;  // words, a 128-byte line each
-struct StGeom {
-    int64_t n;
-    int shift;          // window of an index: idx >> shift
-    int W;              // windows
-    int WP;             // W, rounded up to even
-    int64_t chunks, tiles, groups;
-    int xcds;
-    uint32_t near;      // a chunk whose indices span fewer elements is done directly
-    uint8_t* done;      // [tiles * chunks per tile] chunk is finished
-    uint16_t* count;    // [chunk][WP] elements per window of the chunks that are not
-    uint32_t* rows;     // [tile][WP] elements of the window in the group's earlier tiles
-    uint32_t* gsum;     // [group][WP] the group's elements, then the position of its first one
-    uint32_t* base;     // [W + 1] first position of each window; base[W] = elements staged:
-                        // 0 when every chunk was finished, and the later kernels return
-    // a scatter's second split: windows into bins
-    int sub_shift;      // bin of an index: idx >> sub_shift
-    int lg_subs;
-    uint32_t* tile2;    // [W + 1] first second-level tile of each window
-    uint16_t* win2;     // window of each second-level tile
-    uint32_t* rows2;    // [window][bin][tile of the window]
-    uint32_t* bins;     // [W << lg_subs] first position of each bin
-    uint32_t* gate;     // [kStGates] some not 0: some chunk is not finished; 0 between calls
-    uint32_t* arrived;  // k_st_prefix's workgroups done; 0 between calls
-};
 // the lane's vector u of a tile: of its half h = u / (16/E)
 template <class T>
 __device__ __forceinline__ int64_t st_vec(int64_t tile, int u, uint32_t tid) {
@@ -140,22 +77,6 @@ __device__ __forceinline__ int64_t st_vec(int64_t tile, int u, uint32_t tid) {
 __device__ __forceinline__ bool st_skip(uint32_t mask, int h, uint32_t tid) {
     return (mask >> (h * (kStBlock / 256) + (int)(tid >> 8))) & 1u;
 }
-__device__ __forceinline__ uint32_t* st_gate(const StGeom& g, uint32_t i) {
-    return g.gate + i % kStGates * kStGatePad;
-}
-// by the call's last kernel
-__device__ __forceinline__ void st_close(const StGeom& g) {
-    if (blockIdx.x == 0 && threadIdx.x < kStGates) *st_gate(g, threadIdx.x) = 0u;
-}
-// The o-th of `count` workgroups or steps in XCD order: contiguous ranges per
-// XCD, as split_tile.hpp's xcd_tile, for the 8 XCDs of the chip
-__device__ __forceinline__ uint32_t st_order(uint32_t o, uint32_t count, int xcds) {
-    if (xcds == 8 && count >= 8) {
-        const uint32_t per = count >> 3, rem = count & 7u, x = o & 7u;
-        return x * per + std::min(x, rem) + (o >> 3);
-    }
-    return o;
-}
 // finished chunks of a tile as bits (the last tile's missing ones among them)
 template <int CH>
 __device__ __forceinline__ uint32_t st_done(const StGeom& g, int64_t tile) {
@@ -164,10 +85,6 @@ __device__ __forceinline__ uint32_t st_done(const StGeom& g, int64_t tile) {
     for (int q = 0; q < CH; ++q) m |= (tile * CH + q >= g.chunks || g.done[tile * CH + q] ? 1u : 0u) << q;
     return m;
 }
-
-// Counters per bucket: lanes that count the same bucket at once serialize, so
-// few buckets get several counters each, taken by lane
-__host__ __device__ constexpr int st_copies_lg(int B) { return B <= 64 ? 3 : B <= 128 ? 2 : B <= 256 ? 1 : 0; }
 
 // One chunk per workgroup, of as many lanes as give a CU 32 waves beside the
 // LDS windows.  A chunk whose indices fall inside
@@ -292,172 +209,8 @@ __global__ __launch_bounds__(kStFirstBlock<T>) void k_st_first(const T* __restri
     }
 }
 
-// exclusive prefix over the workgroup's lanes of s, plus carry; carry grows by
-// the sum.  wt: one word per wave.  Two barriers.
-template <int BLOCK>
-__device__ __forceinline__ uint32_t st_block_prefix(uint32_t s, uint32_t* wt, uint32_t& carry) {
-    const int w = threadIdx.x / kWave;
-    const uint32_t inc = wave_inclusive_add(s);
-    if (lane_id() == kWave - 1) wt[w] = inc;
-    __syncthreads();
-    uint32_t before = carry, all = 0;
-    #pragma unroll
-    for (int q = 0; q < BLOCK / kWave; ++q) {
-        before += q < w ? wt[q] : 0u;
-        all += wt[q];
-    }
-    carry += all;
-    __syncthreads();
-    return before + inc - s;
-}
-
-// Prefixes of the windows' counts.  Workgroup = one group of kStGroup tiles,
-// cut into parts of `per` tiles, one lane for two windows of a part: rows[]
-// within the group, gsum[] the group's sums.  The last workgroup to arrive
-// turns gsum[] into positions and sets base[] (and, for a scatter's second
-// split, tile2[] and win2[]).
-template <int CH>
-__global__ __launch_bounds__(kStRowBlock) void k_st_prefix(StGeom g, int lgp) {
-    __shared__ uint32_t part[2 * kStRowBlock], wt[kStRowBlock / kWave], t2s[kStMaxWindows];
-    __shared__ uint8_t fin[kStGroup * CH];
-    __shared__ uint32_t last;
-    const int x = threadIdx.x;
-    const int p = x & ((1 << lgp) - 1), q = x >> lgp;  // windows 2p and 2p + 1, part q
-    const int np = kStRowBlock >> lgp;                 // parts, at most kStGroup
-    const int per = kStGroup / np;
-    const int P = g.WP / 2;
-    const bool in = p < P;
-    const int64_t t0 = (int64_t)blockIdx.x * kStGroup;
-    if (ballot(*st_gate(g, lane_id()) != 0) == 0) {  // the same in every wave
-        if (blockIdx.x == 0 && x == 0) g.base[g.W] = 0;
-        return;
-    }
-    bool open = false;
-    for (int i = x; i < kStGroup * CH; i += kStRowBlock) {
-        fin[i] = t0 * CH + i >= g.chunks || g.done[t0 * CH + i] ? 1 : 0;
-        open = open || !fin[i];
-    }
-    const bool any = __syncthreads_or(open ? 1 : 0) != 0;  // the same in the whole workgroup
-    if (!any) {
-        for (int i = x; i < P; i += kStRowBlock) reinterpret_cast<uint2*>(g.gsum)[(int64_t)blockIdx.x * P + i] = make_uint2(0, 0);
-    } else {
-        const uint32_t* cnt = reinterpret_cast<const uint32_t*>(g.count) + p;
-        uint32_t a = 0, b = 0;
-        auto tile = [&](int t, uint32_t& u, uint32_t& v) {  // the counts of one tile; finished chunks have none
-            #pragma unroll
-            for (int k = 0; k < CH; ++k) {
-                const int64_t c = std::min<int64_t>((t0 + t) * CH + k, g.chunks - 1);
-                const uint32_t y = cnt[c * P];
-                const bool f = fin[t * CH + k] != 0;
-                u += f ? 0u : y & 0xFFFFu;
-                v += f ? 0u : y >> 16;
-            }
-        };
-        if (in) {
-            #pragma unroll 4
-            for (int t = q * per; t < (q + 1) * per; ++t) tile(t, a, b);
-        }
-        part[2 * x] = a;
-        part[2 * x + 1] = b;
-        __syncthreads();
-        a = b = 0;
-        for (int k = 0; k < q; ++k) {
-            a += part[2 * ((k << lgp) + p)];
-            b += part[2 * ((k << lgp) + p) + 1];
-        }
-        if (in) {
-            uint2* rows = reinterpret_cast<uint2*>(g.rows) + p;
-            #pragma unroll 4
-            for (int t = q * per; t < (q + 1) * per; ++t) {
-                if (t0 + t < g.tiles) rows[(t0 + t) * P] = make_uint2(a, b);
-                tile(t, a, b);
-            }
-            if (q == np - 1) reinterpret_cast<uint2*>(g.gsum)[(int64_t)blockIdx.x * P + p] = make_uint2(a, b);
-        }
-    }
-    __syncthreads();
-    if (x == 0) {
-        __threadfence();  // the group's sums before the arrival
-        last = fetch_add(g.arrived, 1u) == gridDim.x - 1 ? 1u : 0u;
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    if (x == 0) st_relaxed(g.arrived, 0u);
-    // the parts now share the groups
-    uint2* gs = reinterpret_cast<uint2*>(g.gsum) + p;
-    const int64_t gper = (g.groups + np - 1) / np;
-    const int64_t g0 = std::min<int64_t>(q * gper, g.groups), g1 = std::min<int64_t>(g0 + gper, g.groups);
-    uint32_t a = 0, b = 0;
-    if (in) {
-        #pragma unroll 16
-        for (int64_t k = g0; k < g1; ++k) {
-            const uint2 y = gs[k * P];
-            a += y.x;
-            b += y.y;
-        }
-    }
-    part[2 * x] = a;
-    part[2 * x + 1] = b;
-    __syncthreads();
-    uint32_t ta = 0, tb = 0, ba = 0, bb = 0;
-    for (int k = 0; k < np; ++k) {
-        const uint32_t ya = part[2 * ((k << lgp) + p)], yb = part[2 * ((k << lgp) + p) + 1];
-        ba += k < q ? ya : 0u;
-        bb += k < q ? yb : 0u;
-        ta += ya;
-        tb += yb;
-    }
-    // the lanes of part 0 hold the windows in order; the others take the
-    // result through part[]
-    const bool lead = q == 0 && in;
-    constexpr uint32_t kTile = CH * kStChunk;
-    uint32_t all = 0, tiles2 = 0;
-    const uint32_t first = st_block_prefix<kStRowBlock>(lead ? ta + tb : 0u, wt, all);
-    const uint32_t na = (ta + kTile - 1) / kTile, nb = (tb + kTile - 1) / kTile;
-    const uint32_t t2 = st_block_prefix<kStRowBlock>(lead ? na + nb : 0u, wt, tiles2);
-    if (lead) {
-        part[2 * p] = first;
-        part[2 * p + 1] = first + ta;
-        g.base[2 * p] = first;  // base[] and tile2[] have room for WP + 1
-        g.base[2 * p + 1] = first + ta;
-        if (g.tile2) {
-            g.tile2[2 * p] = t2s[2 * p] = t2;
-            g.tile2[2 * p + 1] = t2s[2 * p + 1] = t2 + na;
-        }
-    }
-    __syncthreads();
-    if (x == 0) {
-        g.base[g.W] = all;
-        if (g.tile2) g.tile2[g.W] = tiles2;
-    }
-    if (in) {
-        a = part[2 * p] + ba;
-        b = part[2 * p + 1] + bb;
-        #pragma unroll 16
-        for (int64_t k = g0; k < g1; ++k) {
-            const uint2 y = gs[k * P];
-            gs[k * P] = make_uint2(a, b);
-            a += y.x;
-            b += y.y;
-        }
-    }
-    if (g.tile2) {
-        for (uint32_t t = x; t < tiles2; t += kStRowBlock) {
-            int lo = 0, hi = g.W;  // last window whose first tile is at or before t: empty windows have none
-            while (hi - lo > 1) {
-                const int m = (lo + hi) / 2;
-                if (t2s[m] <= t) lo = m;
-                else hi = m;
-            }
-            g.win2[t] = (uint16_t)lo;
-        }
-    }
-}
-
 // LDS of the two splits: [S] indices, then [S] values through the same
 // buffer; counts and offsets of the buckets
-constexpr int kStBuckets = 1024 + 8;
 template <class T, bool SC>
 constexpr size_t st_split_lds() {
     return (size_t)kStTile<T> * (SC ? sizeof(T) : 4) + 8 * kStBuckets;
@@ -469,71 +222,6 @@ __device__ __forceinline__ uint32_t st_bucket(uint32_t x, int shift, uint32_t b0
     return std::min((x >> shift) - b0, B);
 }
 
-// Exclusive prefix of cnt[0, C) into off[], C <= 2*kStBlock, two entries per
-// lane; returns the sum.  A barrier before and after.
-__device__ __forceinline__ uint32_t st_scan(uint32_t tid, const uint32_t* cnt, uint32_t* off, int C, uint32_t* wtmp) {
-    const int t = (int)tid, w = __builtin_amdgcn_readfirstlane(t / kWave);
-    __syncthreads();
-    const uint32_t a = 2 * t < C ? cnt[2 * t] : 0u, b = 2 * t + 1 < C ? cnt[2 * t + 1] : 0u;
-    const uint32_t inc = wave_inclusive_add(a + b);
-    if (lane_id() == kWave - 1) wtmp[w] = inc;
-    __syncthreads();
-    uint32_t before = 0, all = 0;
-    #pragma unroll
-    for (int q = 0; q < kStBlock / kWave; ++q) {
-        before += q < w ? wtmp[q] : 0u;
-        all += wtmp[q];
-    }
-    const uint32_t x = before + inc - a - b;
-    if (2 * t < C) off[2 * t] = x;
-    if (2 * t + 1 < C) off[2 * t + 1] = x + a;
-    __syncthreads();
-    return all;
-}
-
-// Slots of the lane's elements in bucket order, two per word of at[], from
-// one counter atomic each (1 << cl counters per bucket, taken by lane); off[b
-// << cl] = first slot of bucket b.  Returns the number of elements that are
-// some; the others all get the last slot, which is then past them.
-template <int EPL>
-__device__ __forceinline__ uint32_t st_rank(uint32_t tid, uint32_t (&x)[EPL], uint32_t (&at)[EPL / 2], int shift,
-                                            uint32_t b0, int B, int cl, uint32_t* cnt, uint32_t* off, uint32_t* wtmp) {
-    for (int i = (int)tid; i < ((B + 1) << cl); i += kStBlock) cnt[i] = 0;
-    __syncthreads();
-    const uint32_t copy = tid & ((1u << cl) - 1u);
-    #pragma unroll
-    for (int e = 0; e < EPL / 2; ++e) {
-        const uint32_t r0 = __hip_atomic_fetch_add(cnt + (st_bucket(x[2 * e], shift, b0, (uint32_t)B) << cl) + copy,
-                                                   1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        const uint32_t r1 = __hip_atomic_fetch_add(cnt + (st_bucket(x[2 * e + 1], shift, b0, (uint32_t)B) << cl) + copy,
-                                                   1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        at[e] = r0 | (r1 << 16);
-    }
-    // Packed before the scan, and the buckets worked out again after it: held
-    // across it, ranks and counter addresses do not fit the registers of two
-    // workgroups per CU.
-    #pragma unroll
-    for (int e = 0; e < EPL / 2; ++e) asm volatile("" : "+v"(at[e]), "+v"(x[2 * e]), "+v"(x[2 * e + 1]));
-    constexpr uint32_t kLast = kStBlock * EPL - 1;
-    if (tid < (1u << cl)) off[(B << cl) + tid] = kLast;
-    const uint32_t m = st_scan(tid, cnt, off, B << cl, wtmp);
-    #pragma unroll
-    for (int e = 0; e < EPL / 2; ++e) {
-        const uint32_t o0 = off[(st_bucket(x[2 * e], shift, b0, (uint32_t)B) << cl) + copy];
-        const uint32_t o1 = off[(st_bucket(x[2 * e + 1], shift, b0, (uint32_t)B) << cl) + copy];
-        at[e] = std::min((at[e] & 0xFFFFu) + o0, kLast) | std::min((at[e] >> 16) + o1, kLast) << 16;
-    }
-    return m;
-}
-// v[e] to slot e's place in buf
-template <class V, int EPL>
-__device__ __forceinline__ void st_place(V* buf, const uint32_t (&at)[EPL / 2], const V (&v)[EPL]) {
-    #pragma unroll
-    for (int e = 0; e < EPL / 2; ++e) {
-        buf[at[e] & 0xFFFFu] = v[2 * e];
-        buf[at[e] >> 16] = v[2 * e + 1];
-    }
-}
 // The m slots' indices to their output positions d[] (slot + dlt[bucket]; past
 // the output, where the store is dropped, for the slots of no element)
 template <int EPL>
@@ -593,7 +281,7 @@ __device__ __forceinline__ void st_load_idx(const int32_t* __restrict__ idx, int
 }
 
 // Indices (and a scatter's values) of one tile to window order: sidx / sval
-// [gsum[w] + rows[w] ...].  A gather's element keeps its slot in the
+// [base[w] + gsum[w] + rows[w] ...].  A gather's element keeps its slot in the
 // window-ordered tile in slot[].
 template <class T, bool SC>
 __global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_split(const T* __restrict__ in,
@@ -609,17 +297,18 @@ __global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_split(const T* 
     uint32_t* cnt = reinterpret_cast<uint32_t*>(smem + (size_t)kStTile<T> * (SC ? sizeof(T) : 4));
     uint32_t* off = cnt + kStBuckets;
     __shared__ uint32_t wtmp[kStBlock / kWave];
-    if (g.base[g.W] == 0) return;
+    if (*g.open == 0) return;
+    const uint32_t tid = threadIdx.x;
+    if (blockIdx.x == 0) st_keep_bases<CH>(g, tid, wtmp, off);
     const int64_t tile = st_order(blockIdx.x, (uint32_t)g.tiles, g.xcds);
     const uint32_t mask = st_done<CH>(g, tile);
     if (mask == (1u << CH) - 1u) return;
-    const uint32_t tid = threadIdx.x;
     const int cl = st_copies_lg(g.W);
     uint32_t at[EPL / 2], m;
     {
         uint32_t x[EPL];
         st_load_idx<T>(idx, tile, g.n, mask, tid, x);
-        m = st_rank<EPL>(tid, x, at, g.shift, 0u, g.W, cl, cnt, off, wtmp);
+        m = st_rank<EPL>(tid, x, at, [&](int, uint32_t v) { return st_bucket(v, g.shift, 0u, (uint32_t)g.W); }, g.W, cl, cnt, off, wtmp);
         st_place<uint32_t, EPL>(buf, at, x);
     }
     if (!SC) {
@@ -634,10 +323,7 @@ __global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_split(const T* 
         }
     }
     __syncthreads();
-    // cnt[w] becomes the distance from slot to output position
-    const uint32_t* gs = g.gsum + tile / kStGroup * g.WP;
-    const uint32_t* rw = g.rows + tile * g.WP;
-    for (int i = (int)tid; i < g.W; i += kStBlock) cnt[i] = gs[i] + rw[i] - off[i << cl];
+    st_distances(g, tile, tid, cl, cnt, off, wtmp);
     T val[EPL];
     if (SC) st_load_tile<T, T>(in, tile, g.n, tid, val);
     __syncthreads();
@@ -674,7 +360,7 @@ template <class T>
 __global__ __launch_bounds__(kStBlock) void k_st_hist2(StGeom g, const uint32_t* __restrict__ sidx) {
     constexpr int S = kStTile<T>;
     __shared__ uint32_t cnt[kStBuckets];
-    if (g.base[g.W] == 0) return;
+    if (*g.open == 0) return;
     const uint32_t tiles = g.tile2[g.W];
     if (blockIdx.x >= tiles) return;
     const int B = 1 << g.lg_subs;
@@ -702,10 +388,29 @@ __global__ __launch_bounds__(kStBlock) void k_st_hist2(StGeom g, const uint32_t*
     }
 }
 
+// exclusive prefix over the workgroup's lanes of s, plus carry; carry grows by
+// the sum.  wt: one word per wave.  Two barriers.
+template <int BLOCK>
+__device__ __forceinline__ uint32_t st_block_prefix(uint32_t s, uint32_t* wt, uint32_t& carry) {
+    const int w = threadIdx.x / kWave;
+    const uint32_t inc = wave_inclusive_add(s);
+    if (lane_id() == kWave - 1) wt[w] = inc;
+    __syncthreads();
+    uint32_t before = carry, all = 0;
+    #pragma unroll
+    for (int q = 0; q < BLOCK / kWave; ++q) {
+        before += q < w ? wt[q] : 0u;
+        all += wt[q];
+    }
+    carry += all;
+    __syncthreads();
+    return before + inc - s;
+}
+
 // One window's bin counts become output positions; the bins' first positions
 __global__ __launch_bounds__(kStRowBlock) void k_st_rows2(StGeom g) {
     __shared__ uint32_t wt[kStRowBlock / kWave];
-    if (g.base[g.W] == 0) return;
+    if (*g.open == 0) return;
     const int w = blockIdx.x;
     const uint32_t nt = g.tile2[w + 1] - g.tile2[w];
     uint32_t* rows = g.rows2 + ((int64_t)g.tile2[w] << g.lg_subs);
@@ -747,7 +452,7 @@ __global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_split2(StGeom g
     uint32_t* cnt = reinterpret_cast<uint32_t*>(smem + (size_t)S * sizeof(T));
     uint32_t* off = cnt + kStBuckets;
     __shared__ uint32_t wtmp[kStBlock / kWave];
-    if (g.base[g.W] == 0) return;
+    if (*g.open == 0) return;
     const uint32_t tiles = g.tile2[g.W];
     if (blockIdx.x >= tiles) return;
     const int B = 1 << g.lg_subs;
@@ -765,7 +470,7 @@ __global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_split2(StGeom g
         for (int j = 0; j < EPL; ++j) x[j] = buf_load<uint32_t>(rs, tid * 4, j * kStBlock * 4);
         #pragma unroll
         for (int j = 0; j < EPL; ++j) x[j] = tid + j * kStBlock < have ? x[j] : kStNone;
-        st_rank<EPL>(tid, x, at, g.sub_shift, b0, B, cl, cnt, off, wtmp);
+        st_rank<EPL>(tid, x, at, [&](int, uint32_t v) { return st_bucket(v, g.sub_shift, b0, (uint32_t)B); }, B, cl, cnt, off, wtmp);
         st_place<uint32_t, EPL>(buf, at, x);
     }
     __syncthreads();
@@ -799,7 +504,7 @@ __global__ __launch_bounds__(kStBinBlock, kStBinBlock / 128) void k_st_bins(StGe
     extern __shared__ char smem[];
     T* win = reinterpret_cast<T*>(smem);                              // [E]
     uint32_t* cov = reinterpret_cast<uint32_t*>(smem + kStBin);       // [E / 32]
-    if (g.base[g.W] == 0) return;
+    if (*g.open == 0) return;
     st_close(g);
     for (uint32_t ob = blockIdx.x; ob < (uint32_t)nbins; ob += gridDim.x) {
     const int64_t bin = st_order(ob, (uint32_t)nbins, g.xcds);
@@ -854,7 +559,7 @@ template <class T>
 __global__ __launch_bounds__(256) void k_st_gather(const T* __restrict__ in, StGeom g,
                                                    const uint32_t* __restrict__ sidx, T* __restrict__ sval) {
     constexpr int E = kStE<T>;
-    if (g.base[g.W] == 0) return;
+    if (*g.open == 0) return;
     const int64_t m = std::min<int64_t>(g.base[g.W], g.n);
     const uint32_t parts = (uint32_t)((m + kStPart<T> - 1) / kStPart<T>);
     if (blockIdx.x >= parts) return;
@@ -897,7 +602,7 @@ __global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_return(T* __res
     uint32_t* dlt = end + kStBuckets;                                 // [W] slot starts, then slot to position
     uint16_t* first = reinterpret_cast<uint16_t*>(dlt + kStBuckets);  // [tile / kStStep]
     __shared__ uint32_t wtmp[kStBlock / kWave];
-    if (g.base[g.W] == 0) return;
+    if (*g.open == 0) return;
     st_close(g);
     const uint32_t nall = (uint32_t)g.n;
     const int64_t tile = st_order(blockIdx.x, (uint32_t)g.tiles, g.xcds);
@@ -928,7 +633,7 @@ __global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_return(T* __res
         const uint32_t a = dlt[i], e = std::min<uint32_t>(a + end[i], (uint32_t)kStTile<T>);
         for (uint32_t k = (a + kStStep - 1) / kStStep; k * kStStep < e; ++k) first[k] = (uint16_t)i;
         end[i] = e;
-        dlt[i] = g.gsum[tile / kStGroup * g.WP + i] + g.rows[tile * g.WP + i] - a;
+        dlt[i] = g.base[i] + g.gsum[tile / g.group * g.WP + i] + g.rows[tile * g.WP + i] - a;
     }
     __syncthreads();
     const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sval, g.n);
@@ -984,11 +689,9 @@ int run_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, const StGeo
     constexpr size_t l3 = st_split_lds<T, SC>();
     const size_t l1 = ((size_t)g.WP << st_copies_lg(g.W)) * 4;
     T* sval = static_cast<T*>(b.sval);
-    int lgp = 4;  // at most one part per tile
-    while ((2 << lgp) < g.WP) ++lgp;
     EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_split<T, SC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l3));
     hipLaunchKernelGGL((k_st_first<T, SC>), dim3((unsigned)g.chunks), dim3(kStFirstBlock<T>), l1, c->stream, in, out, idx, g);
-    hipLaunchKernelGGL((k_st_prefix<CH>), dim3((unsigned)g.groups), dim3(kStRowBlock), 0, c->stream, g, lgp);
+    launch_st_prefix<CH>(c->stream, g, nullptr);
     hipLaunchKernelGGL((k_st_split<T, SC>), dim3(grid), dim3(kStBlock), l3, c->stream, in, idx, g, b.sidx, sval, b.slot);
     if constexpr (SC) {
         const uint32_t* first = g.base;
@@ -1038,7 +741,8 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
     g.n = n;
     g.chunks = ceil_div(n, (int64_t)kStChunk);
     g.tiles = ceil_div(n, S);
-    g.groups = ceil_div(g.tiles, (int64_t)kStGroup);
+    g.group = st_group(g.tiles);
+    g.groups = ceil_div(g.tiles, (int64_t)g.group);
     g.xcds = c->xcds;
     g.near = (uint32_t)(kStWindow / (int64_t)sizeof(T));
     bool two = false;
@@ -1063,7 +767,7 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
         return p;
     };
     const size_t o_done = take((size_t)(g.tiles * S / kStChunk)), o_count = take((size_t)g.chunks * g.WP * 2),
-                 o_rows = take((size_t)g.tiles * g.WP * 4), o_gsum = take((size_t)g.groups * g.WP * 4), o_base = take(((size_t)g.WP + 1) * 4),
+                 o_rows = take((size_t)g.tiles * g.WP * 4), o_gsum = take((size_t)g.groups * g.WP * 4), o_total = take((size_t)g.WP * 4), o_open = take(4), o_base = take(((size_t)g.WP + 1) * 4),
                  o_tile2 = take(((size_t)g.WP + 1) * 4), o_win2 = take((size_t)tiles2 * 2), o_rows2 = take(((size_t)tiles2 << g.lg_subs) * 4),
                  o_bins = take(((size_t)g.W << g.lg_subs) * 4), o_sidx = take((size_t)n * 4),
                  o_sval = take((size_t)n * sizeof(T)), o_didx = take(two ? (size_t)n * 4 : 0),
@@ -1090,6 +794,8 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
     g.count = reinterpret_cast<uint16_t*>(p + o_count);
     g.rows = u32(o_rows);
     g.gsum = u32(o_gsum);
+    g.total = u32(o_total);
+    g.open = u32(o_open);
     g.base = u32(o_base);
     if (two) {
         g.tile2 = u32(o_tile2);
@@ -1099,7 +805,6 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
     }
     const StBufs b = {u32(o_sidx), u32(o_didx), p + o_sval, p + o_dval, reinterpret_cast<uint16_t*>(p + o_slot)};
     g.gate = c->gs_gate;
-    g.arrived = c->gs_gate + kStGates * kStGatePad;
     *ran = true;
     return scatter ? run_staged<T, true>(c, in, out, idx, g, b, nbins)
                    : run_staged<T, false>(c, in, out, idx, g, b, 0);

@@ -9,17 +9,23 @@
 //   sum over keys k of |{i: R[i] == k}| * |{j: S[j] == k}|.
 // Here the keys are replaced by a bijective mix of their bits (mix32), so that
 // the partitions stay balanced for structured keys; equal keys keep equal
-// mixes.  The split's first pass mixes each key as it loads it (MixOnLoad),
-// so the mixed keys are never written and read back by a pass of their own.
-// The partition width targets 4096 build keys (up to 16 partition bits); a
-// workgroup builds its table from the smaller side of its pair in chunks of at
-// most kJoinChunk keys (load factor <= 1/2), so any skew ends, at the cost of
-// re-probing.  Every
-// key is valid (no sentinel value, unlike the reference's -1).
+// mixes.  The partitioning mixes each key as it loads it, so the mixed keys
+// are never written and read back by a pass of their own.
+//
+// A count does not depend on the order inside a partition, so relations of up
+// to 2^24 keys (the smaller one) are partitioned by the mix's top bits into at
+// most 1024 windows in one pass, both in the same launches (k_jn_hist,
+// k_st_groups, k_st_totals, k_jn_split); longer ones by the stable split's two passes.
+// The partition pairs are then joined by persistent workgroups with a hash
+// table in LDS: 64-bit slots and 4096 build keys per partition (k_join_probe),
+// or, where partitions are fewer, 32-bit slots and 16 384 build keys
+// (k_jn_probe).  Every key is valid (no sentinel value, unlike the reference's
+// -1), and any skew ends, at the cost of re-probing.
 #include <algorithm>
 #include "ctx.hpp"
 #include "device.hpp"
 #include "split_tile.hpp"
+#include "window_tile.hpp"
 
 namespace edpp {
 
@@ -118,6 +124,20 @@ __device__ __forceinline__ void join_load(const JoinPair& jp, uint32_t (&bk)[kJo
     }
 }
 
+// Adds the workgroup's counts to *d_count: wave sums, then one lane per wave
+// through the table's first slots.
+__device__ __forceinline__ void join_add_up(unsigned long long local, uint64_t* table, unsigned long long* d_count) {
+    const uint64_t ws = wave_sum((uint64_t)local);
+    __syncthreads();
+    if (lane_id() == 0) table[threadIdx.x / kWave] = ws;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long total = 0;
+        for (int q = 0; q < kJoinBlock / kWave; ++q) total += table[q];
+        if (total) atomicAdd(d_count, total);
+    }
+}
+
 // Persistent: workgroup g (one per CU, as its table fills the CU's LDS)
 // takes partition pairs g, g + gridDim.x, ...  While a pair's table is
 // cleared, filled and probed, the next pair's offsets and (when both of its
@@ -189,27 +209,331 @@ __global__ __launch_bounds__(kJoinBlock) void k_join_probe(const uint32_t* __res
             pk[q] = npk[q];
         }
     }
-    // workgroup sum: wave sums, then one lane per wave into the table's first slots
-    const uint64_t ws = wave_sum((uint64_t)local);
+    join_add_up(local, table, d_count);
+}
+
+// ------------------------------------------------------------- one-pass partition
+constexpr int kJnEpl = 32;                        // keys per lane of a tile
+constexpr int kJnTile = kStBlock * kJnEpl;        // 16,384 keys
+constexpr int kJnCh = kJnTile / kStChunk;
+constexpr int kJnMaxBits = 10;                    // at most kStMaxWindows partitions
+struct JnRel {
+    const uint32_t* keys;
+    uint32_t* part;
+    StGeom g;
+};
+
+// chunk counts of both relations (grid.y); the count is cleared here
+__global__ __launch_bounds__(256) void k_jn_hist(JnRel r0, JnRel r1, unsigned long long* d_count) {
+    __shared__ uint32_t cnt[kStBuckets];
+    const JnRel& r = blockIdx.y ? r1 : r0;
+    const StGeom& g = r.g;
+    const int t = threadIdx.x;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) *d_count = 0ull;
+    if ((int64_t)blockIdx.x >= g.chunks) return;
+    const int64_t v0 = (int64_t)blockIdx.x * (kStChunk / 4) + t;
+    uint32_t x[16];
+    #pragma unroll
+    for (int u = 0; u < 4; ++u) st_load<uint32_t, 4>(r.keys, v0 + u * 256, g.n, 0u, x + 4 * u);
+    const int cl = st_copies_lg(g.W);
+    for (int i = t; i < (g.WP << cl); i += 256) cnt[i] = 0;
     __syncthreads();
-    if (lane_id() == 0) table[threadIdx.x / kWave] = ws;
+    const uint32_t copy = t & ((1u << cl) - 1u);
+    #pragma unroll
+    for (int e = 0; e < 16; ++e)
+        if (4 * (v0 + e / 4 * 256) + e % 4 < g.n)
+            __hip_atomic_fetch_add(cnt + ((mix32(x[e]) >> g.shift) << cl) + copy, 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long total = 0;
-        for (int q = 0; q < kJoinBlock / kWave; ++q) total += table[q];
-        if (total) atomicAdd(d_count, total);
+    uint32_t* row = reinterpret_cast<uint32_t*>(g.count + (int64_t)blockIdx.x * g.WP);
+    for (int i = t; i < g.WP / 2; i += 256) {
+        uint32_t a = 0, b = 0;
+        for (int c = 0; c < (1 << cl); ++c) {
+            a += cnt[((2 * i) << cl) + c];
+            b += cnt[((2 * i + 1) << cl) + c];
+        }
+        row[i] = a | (b << 16);
     }
+}
+
+constexpr size_t kJnSplitLds = (size_t)kJnTile * 4 + 8 * kStBuckets;
+// mixed keys of one tile to their partitions
+__global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_jn_split(JnRel r0, JnRel r1) {
+    extern __shared__ uint32_t buf[];  // [tile], then counts and offsets
+    uint32_t* cnt = buf + kJnTile;
+    uint32_t* off = cnt + kStBuckets;
+    __shared__ uint32_t wtmp[kStBlock / kWave];
+    const JnRel& r = blockIdx.y ? r1 : r0;
+    const StGeom& g = r.g;
+    if ((int64_t)blockIdx.x >= g.tiles) return;
+    const int64_t tile = st_order(blockIdx.x, (uint32_t)g.tiles, g.xcds);
+    const uint32_t tid = threadIdx.x;
+    if (blockIdx.x == 0) st_keep_bases<kJnCh>(g, tid, wtmp, off);
+    const int cl = st_copies_lg(g.W);
+    const int left = (int)std::min<int64_t>(g.n - tile * kJnTile, kJnTile) - (int)tid * 4;
+    uint32_t m;
+    {
+        uint32_t x[kJnEpl], at[kJnEpl / 2];
+        if (left + (int)tid * 4 == kJnTile) {
+            #pragma unroll
+            for (int u = 0; u < kJnEpl / 4; ++u) {
+                const v4u32 v = ld_stream(reinterpret_cast<const v4u32*>(r.keys) + tile * (kJnTile / 4) + u * kStBlock + tid);
+                #pragma unroll
+                for (int k = 0; k < 4; ++k) x[4 * u + k] = v[k];
+            }
+        } else {
+            const __amdgpu_buffer_rsrc_t rs = buf_rsrc(r.keys + tile * kJnTile, g.n - tile * kJnTile);
+            #pragma unroll
+            for (int e = 0; e < kJnEpl; ++e) x[e] = buf_load<uint32_t>(rs, tid * 16, (uint32_t)(e / 4 * kStBlock * 16 + e % 4 * 4));
+        }
+        #pragma unroll
+        for (int e = 0; e < kJnEpl; ++e) x[e] = mix32(x[e]);
+        m = st_rank<kJnEpl>(
+            tid, x, at,
+            [&](int e, uint32_t v) { return e / 4 * kStBlock * 4 + e % 4 < left ? v >> g.shift : (uint32_t)g.W; }, g.W, cl,
+            cnt, off, wtmp);
+        st_place<uint32_t, kJnEpl>(buf, at, x);
+    }
+    __syncthreads();
+    st_distances(g, tile, tid, cl, cnt, off, wtmp);
+    __syncthreads();
+    const BufSink<uint32_t> out = buf_sink(r.part, g.n);
+    #pragma unroll
+    for (int j = 0; j < kJnEpl; ++j) {
+        const uint32_t i = tid + j * kStBlock;
+        const uint32_t k = buf[i];
+        const uint32_t d = cnt[std::min(k >> g.shift, (uint32_t)g.W - 1u)] + i;  // a slot past m holds anything
+        out.put(i < m ? d : kStNone, k);
+    }
+}
+
+// ------------------------------------------------------------- 32-bit slots
+// Partitions of about 16,384 build keys whose mixes share their top `pbits`
+// bits: a slot holds the other bits and, above them, a count of up to
+// 2^pbits - 1; 0 is empty.  A key that occurs more often raises `over`, and
+// the pair is joined with 64-bit slots instead.
+//
+// Slots lie in buckets of four, read with one 16-byte LDS load; at a load of
+// 1/2 nearly every key ends in its first bucket.  2^24 x 2^24, 1024 pairs:
+// 173 us, VALU and LDS each busy for two fifths of it: a wave goes on until the
+// last of its lanes has found its slot.  As fast: one slot after the other; a
+// claim of the key's own slot first, four keys' claims in flight.
+constexpr int kJnSlots = 2 * kJoinSlots;   // the same 128 KiB
+constexpr int kJnBuckets = kJnSlots / 4;
+constexpr int kJnPre = 18;                 // keys per lane per side held in registers: a partition of 16,384
+                                           // expected keys has fewer than 18,432 but once in 10^50
+__device__ __forceinline__ void jn_insert(uint32_t* table, uint32_t k, int fb, uint32_t* over) {
+    const uint32_t fm = (1u << fb) - 1u, one = 1u << fb;
+    const uint32_t w = one | (k & fm);
+    uint32_t h = k & (uint32_t)(kJnBuckets - 1);
+    while (true) {
+        asm volatile("" ::: "memory");  // other lanes fill slots: read anew (a volatile read would be a flat load)
+        const v4u32 v = reinterpret_cast<const v4u32*>(table)[h];
+        // the key's slot, else the first empty one: slots fill in order and
+        // never empty, so lanes with one key meet in one slot
+        int at = -1;
+        #pragma unroll
+        for (int i = 3; i >= 0; --i) at = v[i] == 0u ? i : at;
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) at = v[i] != 0u && ((v[i] ^ k) & fm) == 0 ? i : at;
+        if (at < 0) {  // full
+            h = (h + 1) & (uint32_t)(kJnBuckets - 1);
+            continue;
+        }
+        uint32_t* slot = table + 4 * h + at;
+        uint32_t o = 0;
+        if (__hip_atomic_compare_exchange_strong(slot, &o, w, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP))
+            return;
+        if (((o ^ k) & fm) == 0) {
+            o = __hip_atomic_fetch_add(slot, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if ((o >> fb) == (0xFFFFFFFFu >> fb)) *over = 1u;
+            return;
+        }
+    }
+}
+__device__ __forceinline__ uint32_t jn_lookup(const uint32_t* table, uint32_t k, int fb) {
+    const uint32_t fm = (1u << fb) - 1u;
+    uint32_t h = k & (uint32_t)(kJnBuckets - 1);
+    while (true) {
+        const v4u32 v = reinterpret_cast<const v4u32*>(table)[h];
+        uint32_t c = 0;
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) c = v[i] != 0u && ((v[i] ^ k) & fm) == 0 ? v[i] >> fb : c;
+        if (c != 0 || v[3] == 0u) return c;  // slots fill in order
+        h = (h + 1) & (uint32_t)(kJnBuckets - 1);
+    }
+}
+
+__device__ __forceinline__ void jn_load(const uint32_t* __restrict__ p, int64_t lo, int64_t hi, uint32_t (&x)[kJnPre]) {
+    // one descriptor for the lane's keys; loads past the end read 0
+    const __amdgpu_buffer_rsrc_t r = buf_rsrc(p + lo, std::min<int64_t>(hi - lo, kJnPre * kJoinBlock));
+    #pragma unroll
+    for (int q = 0; q < kJnPre; ++q) x[q] = buf_load<uint32_t>(r, threadIdx.x * 4, q * kJoinBlock * 4);
+}
+
+// Persistent, as k_join_probe: the next pair's keys are loaded while the
+// current pair's table is filled and probed.  A build side past the registers
+// (heavy keys) takes chunked fills of 64-bit slots; a probe side past them is
+// read on from memory.
+__global__ __launch_bounds__(kJoinBlock) void k_jn_probe(const uint32_t* __restrict__ rk, int64_t rn,
+                                                         const int32_t* __restrict__ rs,
+                                                         const uint32_t* __restrict__ sk, int64_t sn,
+                                                         const int32_t* __restrict__ ss, int B, int pbits,
+                                                         unsigned long long* d_count) {
+    extern __shared__ uint64_t table64[];  // kJoinSlots
+    uint32_t* table = reinterpret_cast<uint32_t*>(table64);
+    __shared__ uint32_t over;
+    const int fb = 32 - pbits;
+    unsigned long long local = 0;
+    int b = blockIdx.x;
+    JoinPair cur = join_pair(b, rk, rn, rs, sk, sn, ss, B);
+    uint32_t bk[kJnPre], pk[kJnPre];
+    jn_load(cur.bkeys, cur.b0, cur.b1, bk);
+    jn_load(cur.pkeys, cur.p0, cur.p1, pk);
+    for (; b < B; b += gridDim.x) {
+        const int nb = b + (int)gridDim.x;
+        JoinPair nxt = cur;
+        if (nb < B) nxt = join_pair(nb, rk, rn, rs, sk, sn, ss, B);
+        uint32_t nbk[kJnPre], npk[kJnPre];
+        const bool any = cur.b1 > cur.b0 && cur.p1 > cur.p0;
+        const bool held = any && cur.b1 - cur.b0 <= kJnPre * kJoinBlock;
+        bool chunks = any && !held;
+        __syncthreads();  // the previous pair's lookups are done before the table is cleared
+        if (held) {
+            v4u32* t4 = reinterpret_cast<v4u32*>(table);
+            #pragma unroll
+            for (int i = 0; i < kJnSlots / 4 / kJoinBlock; ++i) t4[threadIdx.x + i * kJoinBlock] = v4u32{0u, 0u, 0u, 0u};
+            if (threadIdx.x == 0) over = 0u;
+        }
+        if (nb < B) {
+            jn_load(nxt.bkeys, nxt.b0, nxt.b1, nbk);
+            jn_load(nxt.pkeys, nxt.p0, nxt.p1, npk);
+        }
+        if (held) {
+            __syncthreads();
+            const int bn = (int)(cur.b1 - cur.b0);
+            #pragma unroll
+            for (int q = 0; q < kJnPre; ++q)
+                if ((int)threadIdx.x + q * kJoinBlock < bn) jn_insert(table, bk[q], fb, &over);
+            __syncthreads();
+            chunks = over != 0u;
+            if (!chunks) {
+                const int64_t pn = cur.p1 - cur.p0;
+                #pragma unroll
+                for (int q = 0; q < kJnPre; ++q)
+                    if (threadIdx.x + (int64_t)q * kJoinBlock < pn) local += jn_lookup(table, pk[q], fb);
+                for (int64_t i = cur.p0 + kJnPre * kJoinBlock + threadIdx.x; i < cur.p1; i += kJoinBlock)
+                    local += jn_lookup(table, cur.pkeys[i], fb);
+            }
+        }
+        if (chunks) {
+            for (int64_t c0 = cur.b0; c0 < cur.b1; c0 += kJoinChunk) {
+                const int64_t c1 = std::min<int64_t>(c0 + kJoinChunk, cur.b1);
+                __syncthreads();
+                for (int i = threadIdx.x; i < kJoinSlots; i += kJoinBlock) table64[i] = 0ull;
+                __syncthreads();
+                for (int64_t i = c0 + threadIdx.x; i < c1; i += kJoinBlock) join_insert(table64, cur.bkeys[i], 0);
+                __syncthreads();
+                for (int64_t i = cur.p0 + threadIdx.x; i < cur.p1; i += kJoinBlock)
+                    local += join_lookup(table64, cur.pkeys[i], 0);
+            }
+        }
+        cur = nxt;
+        #pragma unroll
+        for (int q = 0; q < kJnPre; ++q) {
+            bk[q] = nbk[q];
+            pk[q] = npk[q];
+        }
+    }
+    join_add_up(local, table64, d_count);
+}
+
+}  // namespace
+
+namespace {
+
+// Both relations partitioned into 2^pbits windows by the mix's top bits, then
+// joined.  `wide`: 32-bit slots.
+int run_one_pass(edpp_ctx* c, const uint32_t* rk, int64_t rn, const uint32_t* sk, int64_t sn, int pbits, bool wide,
+                 unsigned long long* d_count) {
+    const int W = 1 << pbits;
+    JnRel rel[2] = {};
+    size_t at = 0;
+    auto take = [&at](size_t bytes) {
+        const size_t p = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return p;
+    };
+    size_t o[2][6];
+    for (int i = 0; i < 2; ++i) {
+        StGeom& g = rel[i].g;
+        rel[i].keys = i ? sk : rk;
+        g.n = i ? sn : rn;
+        g.shift = 32 - pbits;
+        g.W = g.WP = W;
+        g.chunks = ceil_div(g.n, (int64_t)kStChunk);
+        g.tiles = ceil_div(g.n, (int64_t)kJnTile);
+        g.group = st_group(std::max(ceil_div(rn, (int64_t)kJnTile), ceil_div(sn, (int64_t)kJnTile)));
+        g.groups = ceil_div(g.tiles, (int64_t)g.group);
+        g.xcds = c->xcds;
+        o[i][0] = take((size_t)g.n * 4);
+        o[i][1] = take((size_t)g.chunks * W * 2);
+        o[i][2] = take((size_t)g.tiles * W * 4);
+        o[i][3] = take((size_t)g.groups * W * 4);
+        o[i][4] = take(((size_t)W + 1) * 4);
+        o[i][5] = take((size_t)W * 4);
+    }
+    void* w;
+    int rc = ws_outer_reserve(c, at, &w);
+    if (rc) return rc;
+    char* p = static_cast<char*>(w);
+    for (int i = 0; i < 2; ++i) {
+        StGeom& g = rel[i].g;
+        rel[i].part = reinterpret_cast<uint32_t*>(p + o[i][0]);
+        g.count = reinterpret_cast<uint16_t*>(p + o[i][1]);
+        g.rows = reinterpret_cast<uint32_t*>(p + o[i][2]);
+        g.gsum = reinterpret_cast<uint32_t*>(p + o[i][3]);
+        g.base = reinterpret_cast<uint32_t*>(p + o[i][4]);
+        g.total = reinterpret_cast<uint32_t*>(p + o[i][5]);
+    }
+    const StGeom &g0 = rel[0].g, &g1 = rel[1].g;
+    auto both = [](int64_t a, int64_t b) { return dim3((unsigned)std::max(a, b), 2); };
+    hipLaunchKernelGGL(k_jn_hist, both(g0.chunks, g1.chunks), dim3(256), 0, c->stream, rel[0], rel[1], d_count);
+    launch_st_prefix<kJnCh>(c->stream, g0, &g1);
+    EDPP_HIP(c, hipFuncSetAttribute((const void*)k_jn_split, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kJnSplitLds));
+    hipLaunchKernelGGL(k_jn_split, both(g0.tiles, g1.tiles), dim3(kStBlock), kJnSplitLds, c->stream, rel[0], rel[1]);
+    const size_t lds = (size_t)kJoinSlots * 8;
+    const unsigned grid = (unsigned)std::max(1, std::min(W, std::max(c->cus, 1)));
+    const int32_t *rs = reinterpret_cast<const int32_t*>(g0.base), *ss = reinterpret_cast<const int32_t*>(g1.base);
+    const auto probe = wide ? k_jn_probe : k_join_probe;
+    EDPP_HIP(c, hipFuncSetAttribute((const void*)probe, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    // the partition is the mix's top bits: k_join_probe finds its slots in the low ones
+    hipLaunchKernelGGL(probe, dim3(grid), dim3(kJoinBlock), lds, c->stream, rel[0].part, rn, rs, rel[1].part, sn, ss, W,
+                       wide ? pbits : 0, d_count);
+    EDPP_HIP(c, hipGetLastError());
+    return EDPP_OK;
 }
 
 }  // namespace
 
 int launch_join_count(edpp_ctx* c, const uint32_t* rk, int64_t rn, const uint32_t* sk, int64_t sn,
                       unsigned long long* d_count) {
+    const int64_t small = std::min(rn, sn), large = std::max(rn, sn);
+    // One pass: 32-bit slots need 8 partition bits or more for their counts, and
+    // from 2^22 keys on 16,384 build keys per partition ask for that many; with
+    // fewer keys 64-bit slots and 4096 build keys per partition.  Byte offsets
+    // of 31 bits and whole vectors.
+    if (small > 0 && small <= (1ll << (kJnMaxBits + 14)) && large < (1ll << 29) && aligned16(rk) && aligned16(sk)) {
+        const bool wide = small >= (1ll << 22);
+        int bits = wide ? 8 : 1;
+        while (bits < kJnMaxBits && (small >> bits) > (wide ? 16384 : kJoinTargetBuild)) ++bits;
+        return run_one_pass(c, rk, rn, sk, sn, bits, wide, d_count);
+    }
     hipLaunchKernelGGL(k_join_zero, dim3(1), dim3(64), 0, c->stream, d_count);
     EDPP_HIP(c, hipGetLastError());
-    if (rn == 0 || sn == 0) return EDPP_OK;
+    if (small == 0) return EDPP_OK;
     // partition bits: about kJoinTargetBuild keys of the smaller side per partition
-    const int64_t small = std::min(rn, sn);
     int pbits = 0;
     while (pbits < kJoinMaxBits && (small >> pbits) > kJoinTargetBuild) ++pbits;
     const int B = 1 << pbits;
