@@ -171,6 +171,146 @@ __global__ __launch_bounds__(BLOCK, (BLOCK > kSplitBlock ? 2 * BLOCK / (4 * kWav
     }
 }
 
+// ------------------------------------------------------------- short inputs
+// Two launches instead of four: each scatter workgroup adds up the tiles'
+// counts itself, so no scan and no start kernel run, and every tile is one
+// sub-tile of 2048 keys, so that as many CUs as possible work.  Such calls are
+// bound by latency: 100,000 pairs into 256 buckets take 10.8 us, and 20.2 with
+// a scan between (histogram 4.9, scan 3.8, start 1.4, scatter 11.5 with two
+// sub-tiles per workgroup, and the gaps); 131,072 keys sorted 43.1 and 73.3.
+// The line: tiles x buckets up to kShortOne, which the lanes read at once, and
+// up to kShortTiles tiles (2^21 keys, 2 buckets: 18.1 and 18.3 us, 16: 18.1
+// and 21.3); or up to kShortCounts while every workgroup has a CU of its own
+// (500,000 pairs into 256 buckets 18.4 and 22.4 us, with more workgroups than
+// CUs 2^21 pairs into 64 buckets 55 and 21).
+constexpr int64_t kShortCounts = 65536;
+constexpr int kShortWords = 32;  // words a lane reads at a time, of two counts each
+constexpr int64_t kShortOne = 2 * kShortWords * kSplitBlock;
+constexpr int64_t kShortTiles = 1024;
+constexpr int kShortIpt = 8;
+constexpr int kShortTile = kSplitBlock * kShortIpt;
+
+// counts[tile][B] in 16 bits (B >= 2)
+template <class K, int REGW>
+__global__ __launch_bounds__(kSplitBlock) void k_short_hist(const K* __restrict__ kin, SplitGeom g,
+                                                            uint32_t* __restrict__ counts) {
+    __shared__ uint32_t whist[kSplitWaves * 256];
+    const int B = 1 << g.lg;
+    for (int b = threadIdx.x; b < kSplitWaves * B; b += kSplitBlock) whist[b] = 0;
+    __syncthreads();
+    count_tiles<K, kShortIpt, 1, REGW>(kin, (int64_t)blockIdx.x * kShortTile, g.n, g.lg, g.shift, 1, whist, g.flip);
+    __syncthreads();
+    for (int i = threadIdx.x; i < B / 2; i += kSplitBlock) {
+        uint32_t a = 0, b = 0;
+        #pragma unroll
+        for (int q = 0; q < kSplitWaves; ++q) {
+            a += whist[q * B + 2 * i];
+            b += whist[q * B + 2 * i + 1];
+        }
+        counts[(int64_t)blockIdx.x * (B / 2) + i] = a | (b << 16);
+    }
+}
+
+// place_and_store hook: the output positions from the tiles' counts.  Lane t
+// has added up the buckets 2p and 2p + 1, p = t % (B/2), of every parts-th
+// tile: in all, and in the tiles before this one.
+struct ShortPrefix {
+    static constexpr bool kSync = true;
+    uint32_t before0, before1, total0, total1;
+    int B;
+    uint32_t *run, *tot, *start, *wtmp;
+    int32_t* d_start;
+    __device__ __forceinline__ void publish() const {}
+    __device__ __forceinline__ void keys_placed() const {}
+    __device__ __forceinline__ void resolve() const {
+        // run[] and tot[] are zero since before the ranking
+        const int p = threadIdx.x & (B / 2 - 1);
+        __hip_atomic_fetch_add(run + 2 * p, before0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add(run + 2 * p + 1, before1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add(tot + 2 * p, total0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add(tot + 2 * p + 1, total1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();
+        scan_buckets<kSplitBlock>(tot, start, B, wtmp);
+        __syncthreads();
+        for (int b = threadIdx.x; b < B; b += kSplitBlock) {
+            run[b] += start[b];
+            if (d_start && blockIdx.x == 0) d_start[b] = (int32_t)start[b];
+        }
+    }
+};
+
+// ONE: one batch of words covers the counts; it waits in registers until the
+// keys are ranked.
+template <class K, bool KV, bool BALLOT, bool ONE>
+__global__ __launch_bounds__(kSplitBlock) void k_short_scatter(const K* __restrict__ kin, K* __restrict__ kout,
+                                                               const int32_t* __restrict__ vin,
+                                                               int32_t* __restrict__ vout, SplitGeom g,
+                                                               const uint32_t* __restrict__ counts,
+                                                               int32_t* __restrict__ d_start) {
+    extern __shared__ uint32_t lds[];  // the WG scatter's layout
+    __shared__ uint32_t tot[256], start[256];
+    constexpr int W = kSplitWaves;
+    const int B = 1 << g.lg;
+    uint64_t* wmask = reinterpret_cast<uint64_t*>(lds);
+    uint32_t* whist = lds + whist_word_offset(B, W);
+    uint32_t* run = whist + W * B;
+    uint32_t* sub = run + B;
+    uint32_t* off = sub + B;
+    uint32_t* wtmp = off + B;
+    K* kbuf = reinterpret_cast<K*>(lds + kbuf_word_offset(B, W));
+    int32_t* vbuf = reinterpret_cast<int32_t*>(kbuf + kShortTile);
+    const int tile = blockIdx.x;
+    const int64_t s = (int64_t)tile * kShortTile;
+    const int64_t tend = std::min<int64_t>(s + kShortTile, g.n);
+    const int w = threadIdx.x / kWave;
+    ShortPrefix hook = {0u, 0u, 0u, 0u, B, run, tot, start, wtmp, d_start};
+    const int P = B / 2, parts = kSplitBlock / P;
+    const uint32_t* q = counts + (threadIdx.x & (P - 1));
+    int t0 = threadIdx.x / P;
+    uint32_t c[kShortWords];
+    auto read = [&]() {
+        #pragma unroll
+        for (int i = 0; i < kShortWords; ++i) c[i] = t0 + i * parts < (int)g.tiles ? q[(t0 + i * parts) * P] : 0u;
+    };
+    auto add = [&]() {
+        #pragma unroll
+        for (int i = 0; i < kShortWords; ++i) {
+            const uint32_t lo = c[i] & 0xFFFFu, hi = c[i] >> 16;
+            const bool b = t0 + i * parts < tile;
+            hook.before0 += b ? lo : 0u;
+            hook.before1 += b ? hi : 0u;
+            hook.total0 += lo;
+            hook.total1 += hi;
+        }
+    };
+    read();
+    if (!ONE) {
+        add();
+        #pragma unroll 1
+        for (int r = kShortWords * parts; r < (int)g.tiles; r += kShortWords * parts) {  // the same in the whole workgroup
+            t0 += kShortWords * parts;
+            read();
+            add();
+        }
+    }
+    for (int b = threadIdx.x; b < B; b += kSplitBlock) run[b] = tot[b] = 0;
+    for (int b = threadIdx.x; b < W * B; b += kSplitBlock) {
+        wmask[b] = 0ull;
+        whist[b] = 0;
+    }
+    __syncthreads();
+    uint32_t bk[kShortIpt], rk[kShortIpt];
+    K key[kShortIpt];
+    int32_t val[kShortIpt];
+    rank_subtile<K, kShortIpt, BALLOT, true>(kin, KV ? vin : nullptr, s, tend, g.lg, g.shift, whist + w * B,
+                                             wmask + w * B, bk, rk, key, val, g.flip);
+    if (ONE) add();
+    __syncthreads();
+    place_and_store_to<K, kShortIpt, KV, kSplitBlock, false>(whist, run, sub, off, wtmp, kbuf, vbuf, bk, rk, key, val, B,
+                                                             g.shift, (int)(tend - s), buf_sink(kout, g.n),
+                                                             buf_sink(vout, g.n), g.flip, hook);
+}
+
 // d_start[b] = scanned[b*tiles] (opencl/kernels/split_kernel.cl:320-332)
 __global__ void k_split_start(const int32_t* scanned, int64_t tiles, int B, int32_t* d_start) {
     for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < B; b += gridDim.x * blockDim.x)
@@ -701,13 +841,50 @@ int wg_block(edpp_ctx* c, int lg) {
 template <class K>
 int64_t his_len(edpp_ctx* c, int strategy, int64_t n, int lg) {
     const int64_t B = (int64_t)1 << lg;
-    if (strategy == EDPP_SPLIT_WG) return B * ceil_div(n, wg_tile(c, lg, wg_block<K>(c, lg) * wg_ipt<K>(c, lg)));
+    // the short form's counts are 16-bit, and need their room whatever the tile
+    if (strategy == EDPP_SPLIT_WG)
+        return std::max(B * ceil_div(n, wg_tile(c, lg, wg_block<K>(c, lg) * wg_ipt<K>(c, lg))), kShortCounts / 2);
     if (strategy == EDPP_SPLIT_WI) return B * ceil_div(n, wi_colen(c, lg, 16));
     return B * single_lanes(c, n, lg);
 }
 
+// The short form of a WG pass
+template <class K, bool BALLOT>
+int run_short(edpp_ctx* c, const SplitCall<K>& a, int32_t* his) {
+    SplitGeom g;
+    g.n = a.n;
+    g.lg = a.lg;
+    g.shift = a.shift;
+    g.tile = kShortTile;
+    g.tiles = ceil_div(a.n, (int64_t)kShortTile);
+    g.xcds = c->xcds;
+    g.flip = a.flip;
+    uint32_t* counts = reinterpret_cast<uint32_t*>(his);
+    const dim3 grid((unsigned)g.tiles), block(kSplitBlock);
+    switch (a.lg <= kRegCountBits ? reg_count_words(a.lg) : 0) {
+        case 1: hipLaunchKernelGGL((k_short_hist<K, 1>), grid, block, 0, c->stream, a.kin, g, counts); break;
+        case 2: hipLaunchKernelGGL((k_short_hist<K, 2>), grid, block, 0, c->stream, a.kin, g, counts); break;
+        case 4: hipLaunchKernelGGL((k_short_hist<K, 4>), grid, block, 0, c->stream, a.kin, g, counts); break;
+        default: hipLaunchKernelGGL((k_short_hist<K, 0>), grid, block, 0, c->stream, a.kin, g, counts);
+    }
+    const size_t ls = wg_lds_bytes<kShortIpt, K>(1 << a.lg);
+    const bool one = g.tiles << g.lg <= kShortOne;
+    const auto scatter = a.vin ? (one ? k_short_scatter<K, true, BALLOT, true> : k_short_scatter<K, true, BALLOT, false>)
+                               : (one ? k_short_scatter<K, false, BALLOT, true> : k_short_scatter<K, false, BALLOT, false>);
+    EDPP_HIP(c, hipFuncSetAttribute((const void*)scatter, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ls));
+    hipLaunchKernelGGL(scatter, grid, block, ls, c->stream, a.kin, a.kout, a.vin, a.vout, g, (const uint32_t*)counts,
+                       a.d_start);
+    EDPP_HIP(c, hipGetLastError());
+    return EDPP_OK;
+}
+
 template <class K, int IPT, bool BALLOT, int BLOCK, int RO = kReorderVaried>
 int run_wg(edpp_ctx* c, const SplitCall<K>& a, int32_t* his) {
+    if constexpr (IPT == kShortIpt && BLOCK == kSplitBlock && RO == kReorderVaried && !std::is_same_v<K, MixOnLoad>) {
+        const int64_t tiles = ceil_div(a.n, (int64_t)kShortTile);
+        const int64_t most = tiles <= c->cus ? kShortCounts : tiles <= kShortTiles ? kShortOne : 0;
+        if (a.lg >= 1 && tiles << a.lg <= most) return run_short<K, BALLOT>(c, a, his);
+    }
     const int B = 1 << a.lg;
     constexpr int S = BLOCK * IPT;         // scatter sub-tile
     constexpr int SH = kSplitBlock * IPT;  // histogram sub-tile
