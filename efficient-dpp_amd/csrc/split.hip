@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <type_traits>
 #include "ctx.hpp"
+#include "sort_local.hpp"
 #include "split_tile.hpp"
 #include "tile_scan.hpp"
 
@@ -34,6 +35,11 @@ template <class K, int IPT, int TPW, int REGW>
 __global__ __launch_bounds__(kSplitBlock) void k_split_hist(const K* __restrict__ kin, SplitGeom g, int spt,
                                                             int32_t* __restrict__ his) {
     extern __shared__ uint32_t lds[];
+    if (g.gate.flag) {
+        const bool set = *g.gate.flag != 0;
+        if (!set && !g.gate.other) return;
+        if (set && g.gate.other) kin = static_cast<const K*>(g.gate.k);
+    }
     const int B = 1 << g.lg;
     constexpr int S = kSplitBlock * IPT;
     const int tpw = TPW > 1 ? TPW / spt : 1;  // whole tiles per workgroup
@@ -109,6 +115,14 @@ __global__ __launch_bounds__(BLOCK, (BLOCK > kSplitBlock ? 2 * BLOCK / (4 * kWav
                                                          const int32_t* __restrict__ vin, int32_t* __restrict__ vout,
                                                          SplitGeom g, const int32_t* __restrict__ scanned) {
     extern __shared__ uint32_t lds[];
+    if (g.gate.flag) {
+        const bool set = *g.gate.flag != 0;
+        if (!set && !g.gate.other) return;
+        if (set && g.gate.other) {
+            kin = static_cast<const K*>(g.gate.k);
+            vin = g.gate.v;
+        }
+    }
     constexpr int W = BLOCK / kWave;
     constexpr bool SEP = KV && BLOCK > kSplitBlock;
     static_assert(RO == kReorderVaried || BLOCK == kSplitBlock, "the none and fixed variants use 256 lanes");
@@ -773,6 +787,7 @@ struct SplitCall {
     int64_t n;
     int lg, shift;
     uint32_t flip;     // WG strategy only: bucket bits inverted (signed top digit of a radix sort)
+    SplitGate gate = {};  // WG strategy only, beyond the short form
 };
 
 int64_t wg_tile(edpp_ctx* c, int lg, int S) {
@@ -896,6 +911,7 @@ int run_wg(edpp_ctx* c, const SplitCall<K>& a, int32_t* his) {
     g.tiles = ceil_div(a.n, g.tile);
     g.xcds = c->xcds;
     g.flip = a.flip;
+    g.gate = a.gate;
     const int64_t hlen = (int64_t)B * g.tiles;
     // histogram: register counters up to 16 buckets; above, LDS atomics with
     // four histogram sub-tiles per workgroup where they make whole tiles and
@@ -1286,6 +1302,14 @@ int launch_split(edpp_ctx* c, const K* kin, K* kout, const int32_t* vin, int32_t
 // Signed keys order as int32: the digit holding bit 31 has its top bit
 // flipped.  Passes alternate between the output and workspace copies, so the
 // last one lands in the output; keys_in may equal keys_out.
+// From kLocalSortMin keys on, ordered by all 32 bits: sort_local.hpp's kernels
+// end the sort after the passes over the top 16 bits, and the first two passes
+// run only where the top bits are uneven.  2^26 even keys take 870 us (991
+// before), pairs 1030 (1272).  2^25 would gain as much (447 and 515, 600 and
+// 711), but uneven keys would lose 6 % there.  Up to 2^16 segments of
+// kLocalSortMean keys: more would need a third pass.
+constexpr int64_t kLocalSortMin = 1 << 26;
+constexpr int64_t kLocalSortMean = kSlCap - kSlCap / 16;  // mean segment: room for five deviations of even ones
 int launch_sort_u32(edpp_ctx* c, const uint32_t* kin, uint32_t* kout, const int32_t* vin, int32_t* vout, int64_t n,
                     int begin_bit, int end_bit, bool is_signed) {
     if (n == 0) return EDPP_OK;
@@ -1316,7 +1340,14 @@ int launch_sort_u32(edpp_ctx* c, const uint32_t* kin, uint32_t* kout, const int3
     const bool need_a = passes > 1 || (alias && first_out);
     const bool need_b = alias && first_out && passes > 1;
     const bool chained = c->tune.sort_strategy == EDPP_SPLIT_CHAINED;
-    const size_t hbytes = chained ? kChainSmallBytes : ((size_t)hlen * 4 + 255) & ~(size_t)255;
+    // samples before the passes, segment starts and list after them, share the counts' room
+    int lg_segs = 14;
+    while (n >> lg_segs > kLocalSortMean) ++lg_segs;
+    const bool local = n >= kLocalSortMin && lg_segs <= 16 && bits == 32 && !chained;
+    const size_t cbytes = chained ? kChainSmallBytes
+                          : local ? std::max((size_t)hlen * 4, ((size_t)2 << lg_segs) * 4 + 256)
+                                  : (size_t)hlen * 4;
+    const size_t hbytes = ((cbytes + 255) & ~(size_t)255) + (local ? 256 : 0);
     const size_t kb = ((size_t)n * 4 + 255) & ~(size_t)255;
     const size_t vb = vin ? kb : 0;
     const size_t copies = (need_a ? 1 : 0) + (need_b ? 1 : 0);
@@ -1357,16 +1388,38 @@ int launch_sort_u32(edpp_ctx* c, const uint32_t* kin, uint32_t* kout, const int3
         }
         rc = launch_chain<uint32_t>(c, n, passes, st, nullptr, reinterpret_cast<uint32_t*>(his));
     }
+    SlGeom sl = {};
+    if (local) {
+        sl.n = n;
+        sl.segs = 1 << lg_segs;
+        sl.flip = is_signed ? 0x80000000u : 0u;
+        sl.sample = reinterpret_cast<uint16_t*>(base);
+        sl.start = reinterpret_cast<uint32_t*>(base);
+        sl.list = sl.start + sl.segs + 64;
+        sl.gate = reinterpret_cast<uint32_t*>(base + hbytes - 256);
+        rc = launch_sort_sample(c, kin, sl);
+    }
     for (int p = 0; p < passes && rc == EDPP_OK && !chained; ++p) {
         const int lo = begin_bit + p * per, hi = std::min(end_bit, lo + per), lg = hi - lo;
         const uint32_t flip = (is_signed && hi == 32) ? (1u << (lg - 1)) : 0u;
         SplitCall<uint32_t> a = {sk, const_cast<uint32_t*>(dk[p]), sv, const_cast<int32_t*>(dv[p]), nullptr, n, lg, lo,
                                  flip};
+        if (local && p <= 2) {
+            a.gate.flag = sl.gate;
+            if (p == 2) {  // the first pass, or the third
+                a.gate.other = true;
+                a.gate.k = sk;
+                a.gate.v = sv;
+                a.kin = kin;
+                a.vin = vin;
+            }
+        }
         rc = run_pass<uint32_t>(c, EDPP_SPLIT_WG, a, his);
         sk = dk[p];
         sv = dv[p];
     }
     c->tune = saved;
+    if (local && rc == EDPP_OK) rc = launch_sort_local(c, kout, vin ? vout : nullptr, ak, av, sl);
     if (rc == EDPP_OK && sk != kout) {  // single in-place pass: copy A to the output
         EDPP_HIP(c, hipMemcpyAsync(kout, sk, (size_t)n * 4, hipMemcpyDeviceToDevice, c->stream));
         if (vin) EDPP_HIP(c, hipMemcpyAsync(vout, sv, (size_t)n * 4, hipMemcpyDeviceToDevice, c->stream));

@@ -67,6 +67,14 @@ __host__ __device__ constexpr int kbuf_word_offset(int B, int waves = kSplitWave
 // [w*64*IPT, (w+1)*64*IPT) and item j of lane l is element w*64*IPT + j*64 + l,
 // so ranks follow input order: sub-tile, wave, item, lane.
 
+// A pass that a flag in device memory decides about
+struct SplitGate {
+    const uint32_t* flag = nullptr;
+    bool other = false;         // flag set: read k and v; or else: leave unless the flag is set
+    const void* k = nullptr;
+    const int32_t* v = nullptr;
+};
+
 struct SplitGeom {
     int64_t n;
     int lg;          // log2 B
@@ -75,6 +83,7 @@ struct SplitGeom {
     int64_t tiles;
     int xcds;
     uint32_t flip;   // 0, or the top bucket bit: buckets of a signed top digit in order
+    SplitGate gate;
 };
 
 // Bucket of a key: bits [shift, shift + log2 B) of its low 32 bits, with the
