@@ -18,8 +18,8 @@
 // k_st_groups, k_st_totals, k_jn_split); longer ones by the stable split's two passes.
 // The partition pairs are then joined by persistent workgroups with a hash
 // table in LDS: 64-bit slots and 4096 build keys per partition (k_join_probe),
-// or, where partitions are fewer, 32-bit slots and 16 384 build keys
-// (k_jn_probe).  Every key is valid (no sentinel value, unlike the reference's
+// or, where partitions are fewer, 16 384 build keys in bucket order or in
+// 32-bit slots (k_jn_probe).  Every key is valid (no sentinel value, unlike the reference's
 // -1), and any skew ends, at the cost of re-probing.
 #include <algorithm>
 #include "ctx.hpp"
@@ -314,10 +314,10 @@ __global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_jn_split(JnRel r0,
 // the pair is joined with 64-bit slots instead.
 //
 // Slots lie in buckets of four, read with one 16-byte LDS load; at a load of
-// 1/2 nearly every key ends in its first bucket.  2^24 x 2^24, 1024 pairs:
-// 173 us, VALU and LDS each busy for two fifths of it: a wave goes on until the
-// last of its lanes has found its slot.  As fast: one slot after the other; a
-// claim of the key's own slot first, four keys' claims in flight.
+// 1/2 nearly every key ends in its first bucket.  2^24 x 2^24 distinct keys in
+// 1024 pairs took 173 us so, VALU and LDS each busy for two fifths of it: a
+// wave goes on until the last of its lanes has found its slot.  Such keys now
+// take the bucket order below; these slots are for keys that repeat.
 constexpr int kJnSlots = 2 * kJoinSlots;   // the same 128 KiB
 constexpr int kJnBuckets = kJnSlots / 4;
 constexpr int kJnPre = 18;                 // keys per lane per side held in registers: a partition of 16,384
@@ -372,18 +372,97 @@ __device__ __forceinline__ void jn_load(const uint32_t* __restrict__ p, int64_t 
     for (int q = 0; q < kJnPre; ++q) x[q] = buf_load<uint32_t>(r, threadIdx.x * 4, q * kJoinBlock * 4);
 }
 
-// Persistent, as k_join_probe: the next pair's keys are loaded while the
-// current pair's table is filled and probed.  A build side past the registers
-// (heavy keys) takes chunked fills of 64-bit slots; a probe side past them is
-// read on from memory.
+// Build keys in bucket order: bucket h's are keys[first .. first + len), from
+// index[h] = first | len << 16.  An insertion is one counter atomic, with no
+// claim that can fail, and a lookup reads the bucket's keys only.  2^24 x 2^24
+// keys: 104 us instead of 173; one workgroup per CU, whose LDS operations and
+// barriers bound it.
+constexpr int kJnHeads = 16384;
+// Keys that repeat make buckets long, and slots with counts are then the
+// better table: a bucket of more than kJnEarly among the first keys of every
+// lane, or of more than kJnDeep in the end.  2^24 x 2^24 keys that occur 4, 8
+// and 16 times: 248, 243 and 242 us, and 270 to 280 where only the end tells.
+constexpr int kJnFirst = 6;
+constexpr uint32_t kJnEarly = 9, kJnDeep = 24;
+constexpr int kJnBatch = 3;  // probes that go on together
+static_assert(kJnPre % kJnBatch == 0 && kJnPre % 2 == 0);
+constexpr size_t kJnLds = ((size_t)kJnHeads + kJnPre * kJoinBlock) * 4;
+static_assert(kJnLds >= (size_t)kJnSlots * 4);
+
+// index[] from counts to {first, len}.  Barriers around it.
+__device__ __forceinline__ void jn_index(uint32_t* index, uint32_t* wtmp) {
+    constexpr int R = kJnHeads / 4 / kJoinBlock, W = kJoinBlock / kWave;
+    static_assert(R * W <= kWave);
+    v4u32* v = reinterpret_cast<v4u32*>(index) + threadIdx.x;
+    const int w = threadIdx.x / kWave;
+    v4u32 c[R];
+    uint32_t at[R];
+    #pragma unroll
+    for (int j = 0; j < R; ++j) c[j] = v[j * kJoinBlock];
+    #pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const uint32_t sum = c[j][0] + c[j][1] + c[j][2] + c[j][3], inc = wave_inclusive_add(sum);
+        if (lane_id() == kWave - 1) wtmp[j * W + w] = inc;
+        at[j] = inc - sum;
+    }
+    __syncthreads();
+    // every wave scans all the row sums for itself
+    const uint32_t sum = lane_id() < R * W ? wtmp[lane_id()] : 0u, before = wave_inclusive_add(sum) - sum;
+    #pragma unroll
+    for (int j = 0; j < R; ++j) {
+        uint32_t f = at[j] + read_lane(before, j * W + __builtin_amdgcn_readfirstlane(w));
+        v4u32 y;
+        #pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            y[k] = f | (c[j][k] << 16);
+            f += c[j][k];
+        }
+        v[j * kJoinBlock] = y;
+    }
+    __syncthreads();
+}
+
+// Build keys that equal the batch's probe keys (ok: the lane has one)
+__device__ __forceinline__ uint32_t jn_matches(const uint32_t* index, const uint32_t* keys,
+                                               const uint32_t (&k)[kJnBatch], const bool (&ok)[kJnBatch]) {
+    uint32_t at[kJnBatch], end[kJnBatch], found = 0;
+    #pragma unroll
+    for (int q = 0; q < kJnBatch; ++q) {
+        const uint32_t x = ok[q] ? index[k[q] & (uint32_t)(kJnHeads - 1)] : 0u;
+        at[q] = x & 0xFFFFu;
+        end[q] = at[q] + (x >> 16);
+    }
+    bool more = true;
+    while (more) {
+        uint32_t y[kJnBatch];
+        #pragma unroll
+        for (int q = 0; q < kJnBatch; ++q) y[q] = at[q] < end[q] ? keys[at[q]] : ~k[q];
+        more = false;
+        #pragma unroll
+        for (int q = 0; q < kJnBatch; ++q) {
+            found += y[q] == k[q] ? 1u : 0u;
+            ++at[q];
+            more = more || at[q] < end[q];
+        }
+    }
+    return found;
+}
+
+// Persistent, as k_join_probe; a side's keys of the next pair are loaded into
+// the registers that this pair is done with, so the probes hide the one load
+// and the next pair's counting the other.  Build keys that repeat take 32-bit
+// slots with counts instead, a build side past the registers (heavy keys)
+// chunked fills of 64-bit slots; a probe side past them is read on from memory.
 __global__ __launch_bounds__(kJoinBlock) void k_jn_probe(const uint32_t* __restrict__ rk, int64_t rn,
                                                          const int32_t* __restrict__ rs,
                                                          const uint32_t* __restrict__ sk, int64_t sn,
                                                          const int32_t* __restrict__ ss, int B, int pbits,
                                                          unsigned long long* d_count) {
-    extern __shared__ uint64_t table64[];  // kJoinSlots
+    extern __shared__ uint64_t table64[];  // kJnLds bytes
     uint32_t* table = reinterpret_cast<uint32_t*>(table64);
-    __shared__ uint32_t over;
+    uint32_t* keys = table + kJnHeads;
+    v4u32* t4 = reinterpret_cast<v4u32*>(table) + threadIdx.x;
+    __shared__ uint32_t over, wtmp[kWave];
     const int fb = 32 - pbits;
     unsigned long long local = 0;
     int b = blockIdx.x;
@@ -395,31 +474,78 @@ __global__ __launch_bounds__(kJoinBlock) void k_jn_probe(const uint32_t* __restr
         const int nb = b + (int)gridDim.x;
         JoinPair nxt = cur;
         if (nb < B) nxt = join_pair(nb, rk, rn, rs, sk, sn, ss, B);
-        uint32_t nbk[kJnPre], npk[kJnPre];
         const bool any = cur.b1 > cur.b0 && cur.p1 > cur.p0;
         const bool held = any && cur.b1 - cur.b0 <= kJnPre * kJoinBlock;
-        bool chunks = any && !held;
+        const int bn = held ? (int)(cur.b1 - cur.b0) : 0;
+        const int64_t pn = cur.p1 - cur.p0;
+        bool slots = false, chunks = any && !held;
         __syncthreads();  // the previous pair's lookups are done before the table is cleared
         if (held) {
-            v4u32* t4 = reinterpret_cast<v4u32*>(table);
             #pragma unroll
-            for (int i = 0; i < kJnSlots / 4 / kJoinBlock; ++i) t4[threadIdx.x + i * kJoinBlock] = v4u32{0u, 0u, 0u, 0u};
+            for (int i = 0; i < kJnHeads / 4 / kJoinBlock; ++i) t4[i * kJoinBlock] = v4u32{0u, 0u, 0u, 0u};
             if (threadIdx.x == 0) over = 0u;
+            __syncthreads();
+            uint32_t rank[kJnPre / 2];  // two to a word
+            uint32_t most = 0;
+            #pragma unroll
+            for (int q = 0; q < kJnPre / 2; ++q) {
+                if (q == kJnFirst / 2) slots = __syncthreads_or(most >= kJnEarly);
+                if (slots) continue;
+                uint32_t r[2];
+                #pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    r[h] = (int)threadIdx.x + (2 * q + h) * kJoinBlock < bn
+                               ? __hip_atomic_fetch_add(table + (bk[2 * q + h] & (uint32_t)(kJnHeads - 1)), 1u,
+                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
+                               : 0u;
+                most = std::max(most, std::max(r[0], r[1]));
+                rank[q] = r[0] | (r[1] << 16);
+            }
+            slots = __syncthreads_or(slots || most >= kJnDeep);
+            if (!slots) {
+                jn_index(table, wtmp);
+                #pragma unroll
+                for (int q = 0; q < kJnPre; ++q)
+                    if ((int)threadIdx.x + q * kJoinBlock < bn)
+                        keys[(table[bk[q] & (uint32_t)(kJnHeads - 1)] & 0xFFFFu) +
+                             (q % 2 ? rank[q / 2] >> 16 : rank[q / 2] & 0xFFFFu)] = bk[q];
+            } else {
+                #pragma unroll
+                for (int i = 0; i < kJnSlots / 4 / kJoinBlock; ++i) t4[i * kJoinBlock] = v4u32{0u, 0u, 0u, 0u};
+                if (threadIdx.x == 0) over = 0u;
+                __syncthreads();
+                #pragma unroll
+                for (int q = 0; q < kJnPre; ++q)
+                    if ((int)threadIdx.x + q * kJoinBlock < bn) jn_insert(table, bk[q], fb, &over);
+            }
         }
-        if (nb < B) {
-            jn_load(nxt.bkeys, nxt.b0, nxt.b1, nbk);
-            jn_load(nxt.pkeys, nxt.p0, nxt.p1, npk);
-        }
+        if (nb < B) jn_load(nxt.bkeys, nxt.b0, nxt.b1, bk);
         if (held) {
             __syncthreads();
-            const int bn = (int)(cur.b1 - cur.b0);
-            #pragma unroll
-            for (int q = 0; q < kJnPre; ++q)
-                if ((int)threadIdx.x + q * kJoinBlock < bn) jn_insert(table, bk[q], fb, &over);
-            __syncthreads();
-            chunks = over != 0u;
-            if (!chunks) {
-                const int64_t pn = cur.p1 - cur.p0;
+            chunks = over != 0u && slots;
+            if (!slots) {
+                #pragma unroll
+                for (int q = 0; q < kJnPre; q += kJnBatch) {
+                    uint32_t k[kJnBatch];
+                    bool ok[kJnBatch];
+                    #pragma unroll
+                    for (int i = 0; i < kJnBatch; ++i) {
+                        k[i] = pk[q + i];
+                        ok[i] = threadIdx.x + (int64_t)(q + i) * kJoinBlock < pn;
+                    }
+                    local += jn_matches(table, keys, k, ok);
+                }
+                for (int64_t i = cur.p0 + kJnPre * kJoinBlock + threadIdx.x; i < cur.p1; i += kJnBatch * kJoinBlock) {
+                    uint32_t k[kJnBatch];
+                    bool ok[kJnBatch];
+                    #pragma unroll
+                    for (int q = 0; q < kJnBatch; ++q) {
+                        ok[q] = i + (int64_t)q * kJoinBlock < cur.p1;
+                        k[q] = ok[q] ? cur.pkeys[i + (int64_t)q * kJoinBlock] : 0u;
+                    }
+                    local += jn_matches(table, keys, k, ok);
+                }
+            } else if (!chunks) {
                 #pragma unroll
                 for (int q = 0; q < kJnPre; ++q)
                     if (threadIdx.x + (int64_t)q * kJoinBlock < pn) local += jn_lookup(table, pk[q], fb);
@@ -427,6 +553,7 @@ __global__ __launch_bounds__(kJoinBlock) void k_jn_probe(const uint32_t* __restr
                     local += jn_lookup(table, cur.pkeys[i], fb);
             }
         }
+        if (nb < B) jn_load(nxt.pkeys, nxt.p0, nxt.p1, pk);
         if (chunks) {
             for (int64_t c0 = cur.b0; c0 < cur.b1; c0 += kJoinChunk) {
                 const int64_t c1 = std::min<int64_t>(c0 + kJoinChunk, cur.b1);
@@ -440,11 +567,6 @@ __global__ __launch_bounds__(kJoinBlock) void k_jn_probe(const uint32_t* __restr
             }
         }
         cur = nxt;
-        #pragma unroll
-        for (int q = 0; q < kJnPre; ++q) {
-            bk[q] = nbk[q];
-            pk[q] = npk[q];
-        }
     }
     join_add_up(local, table64, d_count);
 }
@@ -503,7 +625,7 @@ int run_one_pass(edpp_ctx* c, const uint32_t* rk, int64_t rn, const uint32_t* sk
     launch_st_prefix<kJnCh>(c->stream, g0, &g1);
     EDPP_HIP(c, hipFuncSetAttribute((const void*)k_jn_split, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kJnSplitLds));
     hipLaunchKernelGGL(k_jn_split, both(g0.tiles, g1.tiles), dim3(kStBlock), kJnSplitLds, c->stream, rel[0], rel[1]);
-    const size_t lds = (size_t)kJoinSlots * 8;
+    const size_t lds = wide ? kJnLds : (size_t)kJoinSlots * 8;
     const unsigned grid = (unsigned)std::max(1, std::min(W, std::max(c->cus, 1)));
     const int32_t *rs = reinterpret_cast<const int32_t*>(g0.base), *ss = reinterpret_cast<const int32_t*>(g1.base);
     const auto probe = wide ? k_jn_probe : k_join_probe;

@@ -64,3 +64,24 @@ def test_join_of_keys_repeated_past_a_slots_count(torch_gpu, ctx, repeats):
     ctx.join_count(r, s, cnt)
     ctx.sync()
     assert int(cnt.item()) == want
+
+
+@pytest.mark.parametrize("repeats", [2, 4, 8, 12, 30])
+@pytest.mark.parametrize("n", [(1 << 22) + 5, (1 << 23) - 1])
+def test_join_of_keys_repeated_a_few_times(torch_gpu, ctx, repeats, n):
+    """Partitions on both sides of the bucket lengths at which a pair goes over to slots with counts."""
+    torch = torch_gpu
+    g = torch.Generator(device="cuda").manual_seed(repeats)
+    r = torch.randint(-2**31, 2**31, (n // repeats,), device="cuda", dtype=torch.int32, generator=g).repeat(repeats)
+    s = torch.randint(-2**31, 2**31, (2 * n,), device="cuda", dtype=torch.int32, generator=g)
+    s[:r.numel()] = r.flip(0)
+    r = torch.cat([r, s[-(n - r.numel()):]]) if r.numel() < n else r
+    r = r[torch.randperm(r.numel(), device="cuda", generator=g)].contiguous()
+    keys, count = torch.unique(r, return_counts=True)
+    at = torch.searchsorted(keys, s).clamp_(max=keys.numel() - 1)
+    want = int(torch.where(keys[at] == s, count[at], 0).sum())
+    cnt = torch.full((1,), -1, dtype=torch.int64, device="cuda")
+    for a, b in ((r, s), (s, r)):
+        ctx.join_count(a, b, cnt)
+        ctx.sync()
+        assert int(cnt.item()) == want
