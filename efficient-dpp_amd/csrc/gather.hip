@@ -7,8 +7,8 @@
 // set of one pass is n/P elements and can stay in L2 / Infinity Cache while
 // the sequential index stream is re-read every pass.
 //
-// MI355X layout: each lane owns U groups of 4 consecutive positions; the
-// index (and, for scatter, value) groups are read as 16-byte vectors with
+// MI355X layout: each lane owns U groups of 2 or 4 consecutive positions; the
+// index (and, for scatter, value) groups are read as vectors with
 // non-temporal hints so the streaming side does not evict the random side.
 #include <algorithm>
 #include "ctx.hpp"
@@ -16,33 +16,38 @@
 
 namespace edpp {
 
-constexpr int kGsBlock = 256;
+// A lane's step is a group of consecutive positions, and a workgroup's 1024
+// positions.  Scatters: 256 lanes of 4.  Gathers: 256 lanes of 4 4-byte values
+// or 512 of 2 8-byte ones, so that the CU has 32 waves beside LDS windows of 32
+// KiB, not 16, and a wave's 16-byte vectors are contiguous: local, 2^21 and
+// 2^22 positions, 6.2 and 11.2 us, with 256 lanes of 4 9.1 and 18.2; random
+// ones the same.  (Scatters gained a tenth where they are local, but random
+// ones of 2^24 took 340 us instead of 303.)
+template <class T, bool SC>
+constexpr int kGsE = SC ? 4 : 16 / (int)sizeof(T);
+template <class T, bool SC>
+constexpr int kGsBlock = 1024 / kGsE<T, SC>;
 
-template <class T>
-__device__ __forceinline__ void load4(const T* p, T (&v)[4]) {
-    if (sizeof(T) == 4) {
-        v4u32 x = ld_stream(reinterpret_cast<const v4u32*>(p));
+// group g of E consecutive elements, by vectors of 16 bytes or less
+template <class T, int E>
+__device__ __forceinline__ void load_group(const T* p, int64_t g, T (&v)[E]) {
+    constexpr int N = 16 / (int)sizeof(T) < E ? 16 / (int)sizeof(T) : E;
+    typedef T vec __attribute__((ext_vector_type(N)));
+    #pragma unroll
+    for (int h = 0; h < E / N; ++h) {
+        const vec y = ld_stream(reinterpret_cast<const vec*>(p) + g * (E / N) + h);
         #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = (T)x[k];
-    } else {
-        v2u64 a = ld_stream(reinterpret_cast<const v2u64*>(p));
-        v2u64 b = ld_stream(reinterpret_cast<const v2u64*>(p) + 1);
-        v[0] = (T)a[0]; v[1] = (T)a[1]; v[2] = (T)b[0]; v[3] = (T)b[1];
+        for (int k = 0; k < N; ++k) v[h * N + k] = y[k];
     }
 }
-template <class T>
-__device__ __forceinline__ void store4(T* p, const T (&v)[4]) {
-    if (sizeof(T) == 4) {
-        v4u32 x;
-        #pragma unroll
-        for (int k = 0; k < 4; ++k) x[k] = (uint32_t)v[k];
-        st_stream(x, reinterpret_cast<v4u32*>(p));
-    } else {
-        v2u64 a, b;
-        a[0] = v[0]; a[1] = v[1]; b[0] = v[2]; b[1] = v[3];
-        st_stream(a, reinterpret_cast<v2u64*>(p));
-        st_stream(b, reinterpret_cast<v2u64*>(p) + 1);
-    }
+template <class T, int E>
+__device__ __forceinline__ void store_group(T* p, int64_t g, const T (&v)[E]) {
+    static_assert(sizeof(T) * E == 16);
+    typedef T vec __attribute__((ext_vector_type(E)));
+    vec y;
+    #pragma unroll
+    for (int k = 0; k < E; ++k) y[k] = v[k];
+    st_stream(y, reinterpret_cast<vec*>(p) + g);
 }
 
 // Window staging.  A workgroup's chunk is 1024*U consecutive positions.  When
@@ -64,15 +69,15 @@ enum GsPhase { kGsOnly = 0, kGsFirst = 1, kGsLater = 2 };
 
 // Smallest and largest index in [0, nall) of the workgroup's chunk (lo > hi
 // when there is none), the same in every lane.  Ends with a barrier.
-template <int U>
-__device__ __forceinline__ void chunk_window(const uint32_t (&pos)[U][4], uint32_t nall, uint32_t* wlo, uint32_t* whi,
+template <int U, int E, int BLOCK>
+__device__ __forceinline__ void chunk_window(const uint32_t (&pos)[U][E], uint32_t nall, uint32_t* wlo, uint32_t* whi,
                                              uint32_t& lo, uint32_t& hi) {
     lo = 0xFFFFFFFFu;
     hi = 0;
     #pragma unroll
     for (int u = 0; u < U; ++u)
         #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < E; ++k)
             if (pos[u][k] < nall) {
                 lo = std::min(lo, pos[u][k]);
                 hi = std::max(hi, pos[u][k]);
@@ -89,7 +94,7 @@ __device__ __forceinline__ void chunk_window(const uint32_t (&pos)[U][4], uint32
     }
     __syncthreads();
     #pragma unroll
-    for (int q = 0; q < kGsBlock / kWave; ++q) {
+    for (int q = 0; q < BLOCK / kWave; ++q) {
         lo = std::min(lo, wlo[q]);
         hi = std::max(hi, whi[q]);
     }
@@ -97,15 +102,15 @@ __device__ __forceinline__ void chunk_window(const uint32_t (&pos)[U][4], uint32
 
 // out[i] = in[idx[i]] for idx[i] in [from, from+span).  The host clamps
 // from+span to n, so an index outside [0,n) is skipped instead of read.
-// Chunks of the first pass (kGsBlock*UF index vectors each) that its window
+// Chunks of the first pass (kGsBlock*UF groups each) that its window
 // path finished, from done[]: skip[u] for the workgroup's u-th slice of
-// kGsBlock index vectors, the same in the whole workgroup.  Returns whether
+// kGsBlock groups, the same in the whole workgroup.  Returns whether
 // every slice is skipped.  A later pass may run with more vectors per lane
 // (U > UF) than the first.
 // ufs = log2 of the first pass's vectors per lane, which divides U; nchunk =
 // the first pass's chunks (flags).  Shifts only: the test runs in every
 // workgroup of every later pass.
-template <int U>
+template <int U, int BLOCK>
 __device__ __forceinline__ bool later_skips(const uint8_t* __restrict__ done, int64_t ngrp, int ufs, uint32_t nchunk,
                                             bool (&skip)[U]) {
     // the workgroup's slices belong to the U >> ufs consecutive first-pass
@@ -118,49 +123,52 @@ __device__ __forceinline__ bool later_skips(const uint8_t* __restrict__ done, in
     bool all = true;
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-        const int64_t slice = (int64_t)blockIdx.x * U + u;  // its first vector: slice * kGsBlock
-        skip[u] = slice * kGsBlock >= ngrp || ((mask >> (u >> ufs)) & 1u) != 0;
+        const int64_t slice = (int64_t)blockIdx.x * U + u;  // its first group: slice * BLOCK
+        skip[u] = slice * BLOCK >= ngrp || ((mask >> (u >> ufs)) & 1u) != 0;
         all = all && skip[u];
     }
     return all;
 }
 
 template <class T, int U, bool RNT>
-__global__ __launch_bounds__(kGsBlock) void k_gather(const T* __restrict__ in, T* __restrict__ out,
+__global__ __launch_bounds__((kGsBlock<T, false>)) void k_gather(const T* __restrict__ in, T* __restrict__ out,
                                                      const int32_t* __restrict__ idx, int64_t ngrp, uint32_t from,
                                                      uint32_t span, uint32_t nall, uint8_t* __restrict__ done,
                                                      int phase, int ufs, uint32_t nchunk) {
+    constexpr int E = kGsE<T, false>, BLOCK = kGsBlock<T, false>;
     __shared__ T win[kGsWin];
-    __shared__ uint32_t wlo[kGsBlock / kWave], whi[kGsBlock / kWave];
+    __shared__ uint32_t wlo[BLOCK / kWave], whi[BLOCK / kWave];
     // a gather's later passes use the first pass's vectors per lane: one flag
     // per workgroup
     (void)ufs;
     (void)nchunk;
     if (phase == kGsLater && done[blockIdx.x]) return;  // the same in the whole workgroup
-    const int64_t g0 = (int64_t)blockIdx.x * kGsBlock * U + threadIdx.x;
-    uint32_t pos[U][4];
+    const int64_t g0 = (int64_t)blockIdx.x * BLOCK * U + threadIdx.x;
+    uint32_t pos[U][E];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-        int64_t g = g0 + (int64_t)u * kGsBlock;
-        v4u32 x = {nall, nall, nall, nall};  // out of range
-        if (g < ngrp) x = ld_stream(reinterpret_cast<const v4u32*>(idx) + g);
-        #pragma unroll
-        for (int k = 0; k < 4; ++k) pos[u][k] = x[k];
+        int64_t g = g0 + (int64_t)u * BLOCK;
+        if (g < ngrp) {
+            load_group<uint32_t, E>(reinterpret_cast<const uint32_t*>(idx), g, pos[u]);
+        } else {
+            #pragma unroll
+            for (int k = 0; k < E; ++k) pos[u][k] = nall;  // out of range
+        }
     }
-    T val[U][4];
+    T val[U][E];
     bool window = false;
     if (phase != kGsLater) {
         uint32_t lo, hi;
-        chunk_window<U>(pos, nall, wlo, whi, lo, hi);
+        chunk_window<U, E, BLOCK>(pos, nall, wlo, whi, lo, hi);
         window = lo <= hi && hi - lo < (uint32_t)kGsWin;  // the same in the whole workgroup
         if (phase == kGsFirst && threadIdx.x == 0) done[blockIdx.x] = window ? 1 : 0;
         if (window) {
-            for (uint32_t o = threadIdx.x; o <= hi - lo; o += kGsBlock) win[o] = in[lo + o];
+            for (uint32_t o = threadIdx.x; o <= hi - lo; o += BLOCK) win[o] = in[lo + o];
             __syncthreads();
             #pragma unroll
             for (int u = 0; u < U; ++u)
                 #pragma unroll
-                for (int k = 0; k < 4; ++k) val[u][k] = pos[u][k] < nall ? win[pos[u][k] - lo] : T(0);
+                for (int k = 0; k < E; ++k) val[u][k] = pos[u][k] < nall ? win[pos[u][k] - lo] : T(0);
             // every index of the chunk is done: the slice of this pass is all of [0, n)
             from = 0;
             span = nall;
@@ -170,22 +178,22 @@ __global__ __launch_bounds__(kGsBlock) void k_gather(const T* __restrict__ in, T
         #pragma unroll
         for (int u = 0; u < U; ++u)
             #pragma unroll
-            for (int k = 0; k < 4; ++k)
+            for (int k = 0; k < E; ++k)
                 val[u][k] = (pos[u][k] - from < span) ? (RNT ? ld_stream(in + pos[u][k]) : in[pos[u][k]]) : T(0);
     }
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-        int64_t g = g0 + (int64_t)u * kGsBlock;
+        int64_t g = g0 + (int64_t)u * BLOCK;
         if (g < ngrp) {
             bool all = true;
             #pragma unroll
-            for (int k = 0; k < 4; ++k) all = all && (pos[u][k] - from < span);
+            for (int k = 0; k < E; ++k) all = all && (pos[u][k] - from < span);
             if (all) {
-                store4(out + 4 * g, val[u]);
+                store_group<T, E>(out, g, val[u]);
             } else {
                 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (pos[u][k] - from < span) out[4 * g + k] = val[u][k];
+                for (int k = 0; k < E; ++k)
+                    if (pos[u][k] - from < span) out[E * g + k] = val[u][k];
             }
         }
     }
@@ -193,50 +201,49 @@ __global__ __launch_bounds__(kGsBlock) void k_gather(const T* __restrict__ in, T
 
 // out[idx[i]] = in[i] for idx[i] in [from, from+span)
 template <class T, int U, bool RNT>
-__global__ __launch_bounds__(kGsBlock) void k_scatter(const T* __restrict__ in, T* __restrict__ out,
+__global__ __launch_bounds__((kGsBlock<T, true>)) void k_scatter(const T* __restrict__ in, T* __restrict__ out,
                                                       const int32_t* __restrict__ idx, int64_t ngrp, uint32_t from,
                                                       uint32_t span, uint32_t nall, uint8_t* __restrict__ done,
                                                       int phase, int ufs, uint32_t nchunk) {
+    constexpr int E = kGsE<T, true>, BLOCK = kGsBlock<T, true>;
     __shared__ T win[kGsWin];
     __shared__ uint32_t cov[kGsWin / 32];  // positions of the window this chunk writes
-    __shared__ uint32_t wlo[kGsBlock / kWave], whi[kGsBlock / kWave];
+    __shared__ uint32_t wlo[BLOCK / kWave], whi[BLOCK / kWave];
     bool skip[U] = {};
-    if (phase == kGsLater && later_skips<U>(done, ngrp, ufs, nchunk, skip)) return;
-    for (int i = threadIdx.x; i < kGsWin / 32; i += kGsBlock) cov[i] = 0;
-    const int64_t g0 = (int64_t)blockIdx.x * kGsBlock * U + threadIdx.x;
-    uint32_t pos[U][4];
-    T val[U][4];
+    if (phase == kGsLater && later_skips<U, BLOCK>(done, ngrp, ufs, nchunk, skip)) return;
+    for (int i = threadIdx.x; i < kGsWin / 32; i += BLOCK) cov[i] = 0;
+    const int64_t g0 = (int64_t)blockIdx.x * BLOCK * U + threadIdx.x;
+    uint32_t pos[U][E];
+    T val[U][E];
     #pragma unroll
     for (int u = 0; u < U; ++u) {
-        int64_t g = g0 + (int64_t)u * kGsBlock;
+        int64_t g = g0 + (int64_t)u * BLOCK;
         if (g < ngrp && !skip[u]) {
-            v4u32 x = ld_stream(reinterpret_cast<const v4u32*>(idx) + g);
-            #pragma unroll
-            for (int k = 0; k < 4; ++k) pos[u][k] = x[k];
-            load4(in + 4 * g, val[u]);
+            load_group<uint32_t, E>(reinterpret_cast<const uint32_t*>(idx), g, pos[u]);
+            load_group<T, E>(in, g, val[u]);
         } else {
             #pragma unroll
-            for (int k = 0; k < 4; ++k) { pos[u][k] = nall; val[u][k] = 0; }
+            for (int k = 0; k < E; ++k) { pos[u][k] = nall; val[u][k] = 0; }
         }
     }
     bool window = false;
     if (phase != kGsLater) {
         uint32_t lo, hi;
-        chunk_window<U>(pos, nall, wlo, whi, lo, hi);  // its barrier also orders the cov clearing
+        chunk_window<U, E, BLOCK>(pos, nall, wlo, whi, lo, hi);  // its barrier also orders the cov clearing
         window = lo <= hi && hi - lo < (uint32_t)kGsWin;  // the same in the whole workgroup
         if (phase == kGsFirst && threadIdx.x == 0) done[blockIdx.x] = window ? 1 : 0;
         if (window) {
             #pragma unroll
             for (int u = 0; u < U; ++u)
                 #pragma unroll
-                for (int k = 0; k < 4; ++k)
+                for (int k = 0; k < E; ++k)
                     if (pos[u][k] < nall) {
                         const uint32_t o = pos[u][k] - lo;
                         win[o] = val[u][k];
                         atomicOr(cov + (o >> 5), 1u << (o & 31));
                     }
             __syncthreads();
-            for (uint32_t o = threadIdx.x; o <= hi - lo; o += kGsBlock)
+            for (uint32_t o = threadIdx.x; o <= hi - lo; o += BLOCK)
                 if ((cov[o >> 5] >> (o & 31)) & 1u) out[lo + o] = win[o];
         }
     }
@@ -244,7 +251,7 @@ __global__ __launch_bounds__(kGsBlock) void k_scatter(const T* __restrict__ in, 
         #pragma unroll
         for (int u = 0; u < U; ++u)
             #pragma unroll
-            for (int k = 0; k < 4; ++k)
+            for (int k = 0; k < E; ++k)
                 if (pos[u][k] - from < span) {
                     if (RNT) st_stream(val[u][k], out + pos[u][k]);
                     else out[pos[u][k]] = val[u][k];
@@ -270,20 +277,17 @@ struct GsPass {
     uint32_t from, span, nall;
     uint8_t* done;  // one flag per workgroup chunk, written by the first of several passes
     int phase;
-    int ufs;          // log2 of the first pass's index vectors per lane (one done flag per kGsBlock << ufs)
+    int ufs;          // log2 of the first pass's groups per lane (one done flag per 1024 << ufs positions)
     uint32_t nchunk;  // done flags (workgroups of the first pass)
 };
 
 template <class T, int U, bool RNT>
 static void launch_gs_kernel(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t ngrp, const GsPass& q,
                              bool scatter) {
-    const unsigned grid = (unsigned)ceil_div(ngrp, (int64_t)kGsBlock * U);
-    if (scatter)
-        hipLaunchKernelGGL((k_scatter<T, U, RNT>), dim3(grid), dim3(kGsBlock), 0, c->stream, in, out, idx, ngrp,
-                           q.from, q.span, q.nall, q.done, q.phase, q.ufs, q.nchunk);
-    else
-        hipLaunchKernelGGL((k_gather<T, U, RNT>), dim3(grid), dim3(kGsBlock), 0, c->stream, in, out, idx, ngrp,
-                           q.from, q.span, q.nall, q.done, q.phase, q.ufs, q.nchunk);
+    const int block = scatter ? kGsBlock<T, true> : kGsBlock<T, false>;
+    const unsigned grid = (unsigned)ceil_div(ngrp, (int64_t)block * U);
+    hipLaunchKernelGGL((scatter ? k_scatter<T, U, RNT> : k_gather<T, U, RNT>), dim3(grid), dim3(block), 0, c->stream, in,
+                       out, idx, ngrp, q.from, q.span, q.nall, q.done, q.phase, q.ufs, q.nchunk);
 }
 
 template <class T, bool RNT>
@@ -308,11 +312,12 @@ int launch_gather(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t 
     }
     if (passes < 1 || passes > n) passes = passes < 1 ? 1 : (int)n;
     const bool vec = aligned16(in) && aligned16(out) && aligned16(idx);
-    const int64_t ngrp = vec ? n / 4 : 0;
+    const int e = scatter ? kGsE<T, true> : kGsE<T, false>, block = 1024 / e;
+    const int64_t ngrp = vec ? n / e : 0;
     const int64_t len = ceil_div(n, passes);  // gatherImpl.cpp:37
     uint8_t* done = nullptr;
     if (ngrp && passes > 1) {
-        const int64_t grid = ceil_div(ngrp, (int64_t)kGsBlock * c->tune.gs_unroll);
+        const int64_t grid = ceil_div(ngrp, (int64_t)block * c->tune.gs_unroll);
         void* w;
         int rc = ws_reserve(c, (size_t)grid, &w);
         if (rc) return rc;
@@ -329,7 +334,7 @@ int launch_gather(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t 
         q.phase = passes == 1 ? kGsOnly : (p == 0 ? kGsFirst : kGsLater);
         const int uf = c->tune.gs_unroll;  // 1, 2, 4 or 8
         q.ufs = uf == 1 ? 0 : uf == 2 ? 1 : uf == 4 ? 2 : 3;
-        q.nchunk = (uint32_t)ceil_div(ngrp, (int64_t)kGsBlock * uf);
+        q.nchunk = (uint32_t)ceil_div(ngrp, (int64_t)block * uf);
         const uint32_t from = q.from, span = q.span;
         // scatter passes after the first skip the window test, so for 4-byte
         // values they take 8 index vectors per lane: half the workgroups
@@ -342,10 +347,10 @@ int launch_gather(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t 
             else
                 dispatch_unroll<T, false>(c, u, in, out, idx, ngrp, q, scatter);
         }
-        if (ngrp * 4 < n) {
-            int64_t rest = n - ngrp * 4;
+        if (ngrp * e < n) {
+            int64_t rest = n - ngrp * e;
             unsigned g = (unsigned)(rest < 256 * 4096 ? ceil_div(rest, 256) : 4096);
-            hipLaunchKernelGGL((k_gs_scalar<T>), dim3(g), dim3(256), 0, c->stream, in, out, idx, ngrp * 4, n, from,
+            hipLaunchKernelGGL((k_gs_scalar<T>), dim3(g), dim3(256), 0, c->stream, in, out, idx, ngrp * e, n, from,
                                span, scatter);
         }
     }
