@@ -44,7 +44,7 @@ struct DJob {
     int32_t* vout;
     void* aux;
     uint64_t* status;  // u32 scan: 1 word per tile; u64 scan: 2 per tile; split: 1 per histogram-scan tile
-    uint64_t* his;     // split: [B][tiles] tagged words {tag:32 | value:32}
+    uint64_t* his;     // split: [tiles][B] tagged words {tag:32 | value:32}
 };
 
 constexpr int kMaxQueues = 8;
@@ -149,35 +149,49 @@ __device__ void scan_tile(const T* in, T* out, int64_t n, int64_t t, typename Lo
     ts.store(out, base, n, sm.prefix);
 }
 
-// In-place scan of a split job's histogram words: tile t of the bucket-major
-// matrix waits for the count words of its entries, scans them with the
-// look-back over the job's histogram-scan tiles, and rewrites them as
-// scanned words.  Only this tile reads or writes its entries' count words.
+// In-place scan of a split job's histogram words, in bucket-major order: tile
+// t waits for the count words of its entries, scans them with the look-back
+// over the job's histogram-scan tiles, and rewrites them as scanned words.
+// Only this tile reads or writes its entries' count words.  The words lie tile
+// by tile, so that a histogram tile writes its counts, and a scatter tile reads
+// its offsets, as whole lines: an agent-scope word is a request of its own
+// where its neighbours in the wave lie elsewhere.
 template <int BLOCK>
 __device__ void hist_scan_tile(const DJob& J, int64_t t, char* smem, uint32_t spin_limit, int32_t* err) {
     typedef TileScan<uint32_t, BLOCK, 4> TS;
     typename TS::Smem& sm = *reinterpret_cast<typename TS::Smem*>(smem);
-    const int64_t hlen = ((int64_t)1 << J.lg) * J.tiles;
-    const int64_t base = t * TS::TILE;
+    const uint32_t tiles = (uint32_t)J.tiles, hlen = tiles << J.lg;
+    const uint32_t base = (uint32_t)t * TS::TILE;
     TS ts;
     // all 16 words are read at once; only those whose count has not arrived
     // yet are polled again
+    uint32_t at[4][TS::EPV];
     uint64_t w[4][TS::EPV];
     #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t e = base + j * TS::SUB + threadIdx.x * TS::EPV;
+        uint32_t b = e / tiles, c = e - b * tiles;
         #pragma unroll
         for (int k = 0; k < TS::EPV; ++k) {
-            const int64_t e = base + (int64_t)j * TS::SUB + (int64_t)threadIdx.x * TS::EPV + k;
-            w[j][k] = e < hlen ? ld_relaxed(J.his + e) : tagged(kTagCount, 0u);
+            at[j][k] = e + k < hlen ? (c << J.lg) + b : 0xFFFFFFFFu;
+            if (++c == tiles) {
+                c = 0;
+                ++b;
+            }
         }
+    }
     #pragma unroll
     for (int j = 0; j < 4; ++j)
         #pragma unroll
-        for (int k = 0; k < TS::EPV; ++k) {
-            const int64_t e = base + (int64_t)j * TS::SUB + (int64_t)threadIdx.x * TS::EPV + k;
-            ts.v[j][k] = (uint32_t)(w[j][k] >> 32) == kTagCount ? (uint32_t)w[j][k]
-                                                                 : wait_tagged(J.his + e, kTagCount, spin_limit, err);
-        }
+        for (int k = 0; k < TS::EPV; ++k)
+            w[j][k] = at[j][k] != 0xFFFFFFFFu ? ld_relaxed(J.his + at[j][k]) : tagged(kTagCount, 0u);
+    #pragma unroll
+    for (int j = 0; j < 4; ++j)
+        #pragma unroll
+        for (int k = 0; k < TS::EPV; ++k)
+            ts.v[j][k] = (uint32_t)(w[j][k] >> 32) == kTagCount
+                             ? (uint32_t)w[j][k]
+                             : wait_tagged(J.his + at[j][k], kTagCount, spin_limit, err);
     ts.scan(sm);
     LookbackState32 st;
     st.status = J.status;
@@ -199,9 +213,67 @@ __device__ void hist_scan_tile(const DJob& J, int64_t t, char* smem, uint32_t sp
         uint32_t x = sm.prefix + ts.off[j];
         #pragma unroll
         for (int k = 0; k < TS::EPV; ++k) {
-            const int64_t e = base + (int64_t)j * TS::SUB + (int64_t)threadIdx.x * TS::EPV + k;
-            if (e < hlen) st_relaxed(J.his + e, tagged(kTagScanned, x));
+            if (at[j][k] != 0xFFFFFFFFu) st_relaxed(J.his + at[j][k], tagged(kTagScanned, x));
             x += ts.v[j][k];
+        }
+    }
+}
+
+// The same for a job of at most kColumnTiles tiles, by one workgroup: a lane
+// takes a bucket (BLOCK >> lg lanes a range of the tiles each), so that every
+// access of a wave is whole lines, and nothing is looked back for.  (With
+// bucket-major lanes, the scans of the 10,000-job mix, 11 M words, took 174 us
+// by themselves, a request for almost every word; the mix took 1.79 ms, and
+// 1.67 ms so.  From about 256 tiles on one workgroup's chain of reads would be
+// the longest of the launch.)
+constexpr int64_t kColumnTiles = 256;
+template <int BLOCK>
+__device__ void hist_column_scan(const DJob& J, char* smem, uint32_t spin_limit, int32_t* err) {
+    constexpr int R = 16;  // words in flight
+    uint32_t* sums = reinterpret_cast<uint32_t*>(smem);  // [bucket][range]
+    uint32_t* wtmp = sums + BLOCK;
+    const uint32_t B = 1u << J.lg, tiles = (uint32_t)J.tiles;
+    const uint32_t ranges = std::min<uint32_t>(BLOCK >> J.lg, tiles), per = (tiles + ranges - 1) / ranges;
+    const uint32_t b = threadIdx.x & (B - 1), r = threadIdx.x >> J.lg;
+    const uint32_t t0 = std::min(r * per, tiles), t1 = r < ranges ? std::min(t0 + per, tiles) : t0;
+    uint64_t* col = J.his + b;
+    uint32_t c[R];
+    auto counts = [&](uint32_t t) {
+        uint64_t w[R];
+        #pragma unroll
+        for (int i = 0; i < R; ++i)
+            w[i] = t + i < t1 ? ld_relaxed(col + ((int64_t)(t + i) << J.lg)) : tagged(kTagCount, 0u);
+        #pragma unroll
+        for (int i = 0; i < R; ++i)
+            c[i] = (uint32_t)(w[i] >> 32) == kTagCount
+                       ? (uint32_t)w[i]
+                       : wait_tagged(col + ((int64_t)(t + i) << J.lg), kTagCount, spin_limit, err);
+    };
+    uint32_t sum = 0;
+    for (uint32_t t = t0; t < t1; t += R) {
+        counts(t);
+        #pragma unroll
+        for (int i = 0; i < R; ++i) sum += c[i];
+    }
+    sums[threadIdx.x] = 0;
+    __syncthreads();
+    if (r < ranges) sums[b * ranges + r] = sum;
+    __syncthreads();
+    const uint32_t mine = sums[threadIdx.x], inc = wave_inclusive_add(mine);
+    if (lane_id() == kWave - 1) wtmp[threadIdx.x / kWave] = inc;
+    __syncthreads();
+    uint32_t x = inc - mine;
+    #pragma unroll
+    for (int q = 0; q < BLOCK / kWave; ++q) x += q < (int)threadIdx.x / kWave ? wtmp[q] : 0u;
+    sums[threadIdx.x] = x;
+    __syncthreads();
+    x = r < ranges ? sums[b * ranges + r] : 0u;
+    for (uint32_t t = t0; t < t1; t += R) {
+        if (per > R) counts(t);
+        #pragma unroll
+        for (int i = 0; i < R; ++i) {
+            if (t + i < t1) st_relaxed(col + ((int64_t)(t + i) << J.lg), tagged(kTagScanned, x));
+            x += c[i];
         }
     }
 }
@@ -223,7 +295,7 @@ __device__ void split_hist_tile(const DJob& J, int64_t t, uint32_t* lds) {
     for (int b = threadIdx.x; b < B; b += BLOCK) {
         uint32_t a = 0;
         for (int q = 0; q < W; ++q) a += whist[q * B + b];
-        st_relaxed(J.his + (int64_t)b * J.tiles + t, tagged(kTagCount, a));
+        st_relaxed(J.his + (t << J.lg) + b, tagged(kTagCount, a));
     }
 }
 
@@ -265,7 +337,7 @@ __device__ void split_scatter_tile(const DJob& J, int64_t t, uint32_t* lds, uint
     const bool single = J.tiles == 1;
     if (!single) {
         for (int b = threadIdx.x; b < B; b += BLOCK) {
-            const uint32_t r = wait_tagged(J.his + (int64_t)b * J.tiles + t, kTagScanned, spin_limit, err);
+            const uint32_t r = wait_tagged(J.his + (t << J.lg) + b, kTagScanned, spin_limit, err);
             run[b] = r;
             if (t == 0 && J.aux) static_cast<int32_t*>(J.aux)[b] = (int32_t)r;
         }
@@ -307,47 +379,49 @@ __device__ void split_scatter_tile(const DJob& J, int64_t t, uint32_t* lds, uint
 }
 
 // ---------------------------------------------------------------- gather tiles
-// A tile of BLOCK*4*U elements: U rounds of one 16-byte index vector per lane
+// A tile of BLOCK*4*U elements, in steps of one 16-byte vector of output per
+// lane (4 or 2 elements), so that a wave's stores are whole lines for both
+// widths
 template <class T, int BLOCK, int U>
 __device__ void gather_tile(const DJob& J, int64_t t) {
+    typedef typename vec16<T>::type V;
+    constexpr int E = vec16<T>::n, S = 4 * U / E;
+    typedef uint32_t vidx __attribute__((ext_vector_type(E)));
     const T* in = static_cast<const T*>(J.in);
     T* out = static_cast<T*>(J.out);
     const uint32_t n = (uint32_t)J.n;
     const int64_t base = t * (int64_t)BLOCK * 4 * U;
     if (base + (int64_t)BLOCK * 4 * U <= J.n) {
         // a whole tile: every index vector, then every random read, then the
-        // stores, so that each group of loads is in flight at once; four
-        // valid indices leave as one 16-byte store per 16 bytes of output
-        // (batch buffers are 16-byte aligned)
-        v4u32 x[U];
+        // stores, so that each group of loads is in flight at once; a step's
+        // valid indices leave as one 16-byte store (batch buffers are 16-byte
+        // aligned)
+        vidx x[S];
         #pragma unroll
-        for (int u = 0; u < U; ++u)
-            x[u] = ld_stream(reinterpret_cast<const v4u32*>(J.idx + base + (int64_t)u * BLOCK * 4 + threadIdx.x * 4));
+        for (int u = 0; u < S; ++u)
+            x[u] = ld_stream(reinterpret_cast<const vidx*>(J.idx + base + (int64_t)u * BLOCK * E + threadIdx.x * E));
         __builtin_amdgcn_sched_barrier(0);
-        T v[U][4];
+        T v[S][E];
         #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < S; ++u)
             #pragma unroll
-            for (int k = 0; k < 4; ++k) v[u][k] = (uint32_t)x[u][k] < n ? in[(uint32_t)x[u][k]] : T(0);
+            for (int k = 0; k < E; ++k) v[u][k] = (uint32_t)x[u][k] < n ? in[(uint32_t)x[u][k]] : T(0);
         __builtin_amdgcn_sched_barrier(0);
         #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t e0 = base + (int64_t)u * BLOCK * 4 + threadIdx.x * 4;
-            const bool all = (uint32_t)x[u][0] < n && (uint32_t)x[u][1] < n && (uint32_t)x[u][2] < n &&
-                             (uint32_t)x[u][3] < n;
+        for (int u = 0; u < S; ++u) {
+            const int64_t e0 = base + (int64_t)u * BLOCK * E + threadIdx.x * E;
+            bool all = true;
+            V o;
+            #pragma unroll
+            for (int k = 0; k < E; ++k) {
+                all = all && (uint32_t)x[u][k] < n;
+                o[k] = v[u][k];
+            }
             if (all) {
-                typedef typename vec16<T>::type V;
-                constexpr int EPV = vec16<T>::n;
-                #pragma unroll
-                for (int h = 0; h < 4 / EPV; ++h) {
-                    V o;
-                    #pragma unroll
-                    for (int k = 0; k < EPV; ++k) o[k] = v[u][h * EPV + k];
-                    st_stream(o, reinterpret_cast<V*>(out + e0 + h * EPV));
-                }
+                st_stream(o, reinterpret_cast<V*>(out + e0));
             } else {
                 #pragma unroll
-                for (int k = 0; k < 4; ++k)
+                for (int k = 0; k < E; ++k)
                     if ((uint32_t)x[u][k] < n) out[e0 + k] = v[u][k];
             }
         }
@@ -421,7 +495,8 @@ __global__ __launch_bounds__(BLOCK) void k_batch(const DJob* __restrict__ jobs, 
             if (J.wide) split_hist_tile<uint64_t, IPT, BLOCK>(J, t, lds);
             else split_hist_tile<uint32_t, IPT, BLOCK>(J, t, lds);
         } else if (phase == kPhaseHistScan) {
-            hist_scan_tile<BLOCK>(J, t, smem, spin_limit, err);
+            if (J.tiles <= kColumnTiles) hist_column_scan<BLOCK>(J, smem, spin_limit, err);
+            else hist_scan_tile<BLOCK>(J, t, smem, spin_limit, err);
         } else if (phase == kPhaseScatter) {
             if (J.wide) split_scatter_tile<uint64_t, IPT, BLOCK>(J, t, lds, spin_limit, err);
             else split_scatter_tile<uint32_t, IPT, BLOCK>(J, t, lds, spin_limit, err);
@@ -453,7 +528,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch(const DJob* __restrict__ jobs, 
 constexpr size_t shape_lds(const BatchShape& s) {
     return std::max<size_t>((size_t)kbuf_word_offset(256, s.block / kWave) * 4 +
                                 (size_t)s.block * s.split_ipt * (sizeof(uint64_t) + sizeof(int32_t)),
-                            1024);
+                            4096);
 }
 
 typedef void (*BatchKernel)(const DJob*, const uint64_t*, QTable, uint32_t*, uint32_t, int32_t*);
@@ -579,7 +654,7 @@ static int plan(edpp_batch* b) {
         } else if (q.kind == EDPP_JOB_SPLIT && d.tiles > 1) {
             // (a job of one tile takes its offsets from its own counts)
             const int64_t hlen = ((int64_t)1 << d.lg) * d.tiles;
-            d.hscan_tiles = ceil_div(hlen, hscan_tile_elems(sh));
+            d.hscan_tiles = d.tiles <= kColumnTiles ? 1 : ceil_div(hlen, hscan_tile_elems(sh));
             words += 2 * d.hscan_tiles + 2 * hlen;  // u64 status, then u64 histogram words
         }
         words = (words + 3) & ~(int64_t)3;  // 16-byte alignment of every job's state
