@@ -171,10 +171,10 @@ __device__ __forceinline__ uint32_t sl_prefix(uint32_t x, uint32_t* wtmp) {
 
 // hist[w][b] = elements of smaller digits, and of digit b in earlier waves.
 // Barriers around it.
-template <int BITS>
+template <int BITS, int BLOCK = kSlBlock>
 __device__ __forceinline__ void sl_scan(uint16_t* hist, uint32_t* wtmp) {
-    constexpr int B = 1 << BITS, W = kSlBlock / kWave;
-    static_assert(B <= kSlBlock);
+    constexpr int B = 1 << BITS, W = BLOCK / kWave;
+    static_assert(B <= BLOCK);
     const int t = threadIdx.x;
     __syncthreads();
     uint32_t c[W], sum = 0;
@@ -346,6 +346,72 @@ __global__ __launch_bounds__(kSlBlock) void k_sort_longer(uint32_t* keys, int32_
         if (cnt <= kSlLongCap) continue;
         sl_long_pass<KV, BITS1, 0>(keys + s, vals + s, tkeys + s, tvals + s, cnt, hist, run, wtmp);
         sl_long_pass<KV, BITS2, BITS1>(tkeys + s, tvals + s, keys + s, vals + s, cnt, hist, run, wtmp);
+    }
+}
+
+// A whole sort by one workgroup: the passes of the long form, with the keys
+// and values in registers and LDS between them.  A short sort is bound by
+// latency.  Pairs, us, so and with two launches per pass: 1000 7.5 and 35, 4000
+// 13 and 40, 8192 21 and 40, 12,000 28 and 42; with one pass of 8 bits, 8192
+// 6.8 and 9.6.  At 16,384 the one CU is as slow (41 and 43).  Up to 8192 keys
+// eight per lane: the longer kernel takes 3 us more at any length.
+constexpr int kOneBlock = 1024, kOneRows = 8, kOneCap = 12 * kOneBlock;
+struct OneSort {
+    int n, begin, end, per;  // per: bits of a pass, at most 8
+    uint32_t sign;           // flips the key's top bit
+};
+template <bool KV, int ROWS>
+__global__ __launch_bounds__(kOneBlock) void k_sort_one(const uint32_t* kin, uint32_t* kout, const int32_t* vin,
+                                                        int32_t* vout, OneSort g) {
+    constexpr int W = kOneBlock / kWave;
+    __shared__ uint32_t keys[ROWS * kOneBlock];
+    __shared__ int32_t vals[KV ? ROWS * kOneBlock : 1];
+    __shared__ uint16_t hist[W << 8];
+    __shared__ uint32_t wtmp[W];
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int all = (g.n + kWave - 1) / kWave, per = all / W, rem = all % W;
+    const int rows = per + (w < rem ? 1 : 0);
+    const int e0 = (w * per + std::min(w, rem)) * kWave + lane_id();
+    uint32_t x[ROWS], d[ROWS], old[ROWS], below[ROWS];
+    int32_t v[ROWS];
+    #pragma unroll
+    for (int j = 0; j < ROWS; ++j) {
+        const int e = e0 + j * kWave;
+        const bool ok = j < rows && e < g.n;
+        x[j] = ok ? kin[e] : 0u;
+        if constexpr (KV) v[j] = ok ? vin[e] : 0;
+    }
+    for (int lo = g.begin; lo < g.end; lo += g.per) {
+        const int bits = std::min(g.per, g.end - lo);
+        // the last row's lanes past the end take the last digit: they stay the last ones
+        #pragma unroll
+        for (int j = 0; j < ROWS; ++j)
+            d[j] = e0 + j * kWave < g.n ? __builtin_amdgcn_ubfe(x[j] ^ g.sign, lo, bits) : 255u;
+        uint16_t* row = hist + (w << 8);
+        sl_rank<8, 0, ROWS>(d, rows, row, old, below);
+        sl_scan<8, kOneBlock>(hist, wtmp);
+        #pragma unroll
+        for (int j = 0; j < ROWS; ++j)
+            if (j < rows) {
+                const uint32_t p = row[d[j]] + old[j] + below[j];
+                keys[p] = x[j];
+                if constexpr (KV) vals[p] = v[j];
+            }
+        __syncthreads();
+        #pragma unroll
+        for (int j = 0; j < ROWS; ++j)
+            if (j < rows) {
+                x[j] = keys[e0 + j * kWave];
+                if constexpr (KV) v[j] = vals[e0 + j * kWave];
+            }
+    }
+    #pragma unroll
+    for (int j = 0; j < ROWS; ++j) {
+        const int e = e0 + j * kWave;
+        if (j < rows && e < g.n) {
+            kout[e] = x[j];
+            if constexpr (KV) vout[e] = v[j];
+        }
     }
 }
 

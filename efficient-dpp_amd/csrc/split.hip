@@ -1322,6 +1322,14 @@ int launch_sort_u32(edpp_ctx* c, const uint32_t* kin, uint32_t* kout, const int3
     const int bits = end_bit - begin_bit;
     const int passes = (bits + kMaxSplitBitsPerPass - 1) / kMaxSplitBitsPerPass;
     const int per = (bits + passes - 1) / passes;  // balanced digits of at most 8 bits
+    if (n <= kOneCap && c->tune.sort_strategy != EDPP_SPLIT_CHAINED) {
+        const OneSort g = {(int)n, begin_bit, end_bit, per, is_signed && end_bit == 32 ? 0x80000000u : 0u};
+        const auto one = n <= kOneRows * kOneBlock ? (vin ? k_sort_one<true, kOneRows> : k_sort_one<false, kOneRows>)
+                                                   : (vin ? k_sort_one<true, 12> : k_sort_one<false, 12>);
+        hipLaunchKernelGGL(one, dim3(1), dim3(kOneBlock), 0, c->stream, kin, kout, vin, vout, g);
+        EDPP_HIP(c, hipGetLastError());
+        return EDPP_OK;
+    }
     const edpp_tuning saved = c->tune;
     default_split_shape(c, n, 1 << per, 4, &c->tune.split_ipt, &c->tune.split_tile_mult);
     int64_t hlen = 0;
