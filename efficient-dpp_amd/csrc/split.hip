@@ -31,14 +31,14 @@ namespace edpp {
 // TPW), so that every lane has TPW*IPT loads in flight and the workgroup's
 // fixed costs (LDS clearing, barriers, the column writes) are shared; that
 // pays where the per-key LDS atomics dominate (many buckets).
-template <class K, int IPT, int TPW, int REGW>
+template <class K, int IPT, int TPW, int REGW, bool GATED = false>
 __global__ __launch_bounds__(kSplitBlock) void k_split_hist(const K* __restrict__ kin, SplitGeom g, int spt,
-                                                            int32_t* __restrict__ his) {
+                                                            int32_t* __restrict__ his, SplitGate gate) {
     extern __shared__ uint32_t lds[];
-    if (g.gate.flag) {
-        const bool set = *g.gate.flag != 0;
-        if (!set && !g.gate.other) return;
-        if (set && g.gate.other) kin = static_cast<const K*>(g.gate.k);
+    if constexpr (GATED) {
+        const bool set = *gate.flag != 0;
+        if (!set && !gate.other) return;
+        if (set && gate.other) kin = static_cast<const K*>(gate.k);
     }
     const int B = 1 << g.lg;
     constexpr int S = kSplitBlock * IPT;
@@ -110,17 +110,18 @@ struct LateValues {
 // 256 lanes.  Keys and values are loaded through raw buffer descriptors
 // (no branch per load); BST: the varied variant also stores through them,
 // for outputs whose byte offsets fit 31 bits.
-template <class K, int IPT, bool KV, bool BALLOT, int BLOCK, int RO = kReorderVaried, bool BST = false>
+template <class K, int IPT, bool KV, bool BALLOT, int BLOCK, int RO = kReorderVaried, bool BST = false, bool GATED = false>
 __global__ __launch_bounds__(BLOCK, (BLOCK > kSplitBlock ? 2 * BLOCK / (4 * kWave) : 1)) void k_split_scatter(const K* __restrict__ kin, K* __restrict__ kout,
                                                          const int32_t* __restrict__ vin, int32_t* __restrict__ vout,
-                                                         SplitGeom g, const int32_t* __restrict__ scanned) {
+                                                         SplitGeom g, const int32_t* __restrict__ scanned,
+                                                         SplitGate gate) {
     extern __shared__ uint32_t lds[];
-    if (g.gate.flag) {
-        const bool set = *g.gate.flag != 0;
-        if (!set && !g.gate.other) return;
-        if (set && g.gate.other) {
-            kin = static_cast<const K*>(g.gate.k);
-            vin = g.gate.v;
+    if constexpr (GATED) {
+        const bool set = *gate.flag != 0;
+        if (!set && !gate.other) return;
+        if (set && gate.other) {
+            kin = static_cast<const K*>(gate.k);
+            vin = gate.v;
         }
     }
     constexpr int W = BLOCK / kWave;
@@ -787,7 +788,7 @@ struct SplitCall {
     int64_t n;
     int lg, shift;
     uint32_t flip;     // WG strategy only: bucket bits inverted (signed top digit of a radix sort)
-    SplitGate gate = {};  // WG strategy only, beyond the short form
+    SplitGate gate = {};  // WG strategy and 32-bit keys only, more than 16 buckets, beyond the short form
 };
 
 int64_t wg_tile(edpp_ctx* c, int lg, int S) {
@@ -911,7 +912,6 @@ int run_wg(edpp_ctx* c, const SplitCall<K>& a, int32_t* his) {
     g.tiles = ceil_div(a.n, g.tile);
     g.xcds = c->xcds;
     g.flip = a.flip;
-    g.gate = a.gate;
     const int64_t hlen = (int64_t)B * g.tiles;
     // histogram: register counters up to 16 buckets; above, LDS atomics with
     // four histogram sub-tiles per workgroup where they make whole tiles and
@@ -933,20 +933,25 @@ int run_wg(edpp_ctx* c, const SplitCall<K>& a, int32_t* his) {
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)ls));
     const unsigned hgrid = (unsigned)ceil_div(g.tiles, (int64_t)tpw);
     const int ispt = (int)spt;
+    // a gated pass (of a long sort) has 32-bit keys, more than 16 buckets and
+    // outputs within a buffer descriptor
+    constexpr bool kGates = std::is_same_v<K, uint32_t> && RO == kReorderVaried && !BALLOT;
+    const bool gated = kGates && a.gate.flag;
     switch (regw) {
-        case 1: hipLaunchKernelGGL((k_split_hist<K, IPT, 1, 1>), dim3(hgrid), dim3(kSplitBlock), lh, c->stream, a.kin, g, 1, his); break;
-        case 2: hipLaunchKernelGGL((k_split_hist<K, IPT, 1, 2>), dim3(hgrid), dim3(kSplitBlock), lh, c->stream, a.kin, g, 1, his); break;
-        case 4: hipLaunchKernelGGL((k_split_hist<K, IPT, 1, 4>), dim3(hgrid), dim3(kSplitBlock), lh, c->stream, a.kin, g, 1, his); break;
+        case 1: hipLaunchKernelGGL((k_split_hist<K, IPT, 1, 1>), dim3(hgrid), dim3(kSplitBlock), lh, c->stream, a.kin, g, 1, his, a.gate); break;
+        case 2: hipLaunchKernelGGL((k_split_hist<K, IPT, 1, 2>), dim3(hgrid), dim3(kSplitBlock), lh, c->stream, a.kin, g, 1, his, a.gate); break;
+        case 4: hipLaunchKernelGGL((k_split_hist<K, IPT, 1, 4>), dim3(hgrid), dim3(kSplitBlock), lh, c->stream, a.kin, g, 1, his, a.gate); break;
         default:
             if (multi && hsub == 2)
-                hipLaunchKernelGGL((k_split_hist<K, IPT, 2, 0>), dim3(hgrid), dim3(kSplitBlock), lh,
-                                   c->stream, a.kin, g, ispt, his);
+                hipLaunchKernelGGL((gated ? k_split_hist<K, IPT, 2, 0, kGates> : k_split_hist<K, IPT, 2, 0>), dim3(hgrid),
+                                   dim3(kSplitBlock), lh, c->stream, a.kin, g, ispt, his, a.gate);
             else if (multi)
-                hipLaunchKernelGGL((k_split_hist<K, IPT, kHistTilesPerWG, 0>), dim3(hgrid), dim3(kSplitBlock), lh,
-                                   c->stream, a.kin, g, ispt, his);
+                hipLaunchKernelGGL((gated ? k_split_hist<K, IPT, kHistTilesPerWG, 0, kGates>
+                                          : k_split_hist<K, IPT, kHistTilesPerWG, 0>), dim3(hgrid), dim3(kSplitBlock), lh,
+                                   c->stream, a.kin, g, ispt, his, a.gate);
             else
-                hipLaunchKernelGGL((k_split_hist<K, IPT, 1, 0>), dim3(hgrid), dim3(kSplitBlock), lh, c->stream, a.kin,
-                                   g, 1, his);
+                hipLaunchKernelGGL((gated ? k_split_hist<K, IPT, 1, 0, kGates> : k_split_hist<K, IPT, 1, 0>), dim3(hgrid),
+                                   dim3(kSplitBlock), lh, c->stream, a.kin, g, 1, his, a.gate);
     }
     EDPP_HIP(c, hipGetLastError());
     int rc = launch_scan<uint32_t>(c, (const uint32_t*)his, (uint32_t*)his, hlen, EDPP_SCAN_LOOKBACK, nullptr);
@@ -957,26 +962,24 @@ int run_wg(edpp_ctx* c, const SplitCall<K>& a, int32_t* his) {
     if constexpr (RO == kReorderVaried) {
         // buffer stores while every output offset fits the descriptor's 31 bits
         if ((uint64_t)a.n * sizeof(K) < (1ull << 31)) {
-            EDPP_HIP(c, hipFuncSetAttribute((const void*)k_split_scatter<K, IPT, true, BALLOT, BLOCK, RO, true>,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)ls));
-            EDPP_HIP(c, hipFuncSetAttribute((const void*)k_split_scatter<K, IPT, false, BALLOT, BLOCK, RO, true>,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)ls));
-            if (a.vin)
-                hipLaunchKernelGGL((k_split_scatter<K, IPT, true, BALLOT, BLOCK, RO, true>), dim3((unsigned)g.tiles),
-                                   dim3(BLOCK), ls, c->stream, a.kin, a.kout, a.vin, a.vout, g, (const int32_t*)his);
-            else
-                hipLaunchKernelGGL((k_split_scatter<K, IPT, false, BALLOT, BLOCK, RO, true>), dim3((unsigned)g.tiles),
-                                   dim3(BLOCK), ls, c->stream, a.kin, a.kout, a.vin, a.vout, g, (const int32_t*)his);
+            const auto scatter =
+                a.vin ? (gated ? k_split_scatter<K, IPT, true, BALLOT, BLOCK, RO, true, kGates>
+                               : k_split_scatter<K, IPT, true, BALLOT, BLOCK, RO, true>)
+                      : (gated ? k_split_scatter<K, IPT, false, BALLOT, BLOCK, RO, true, kGates>
+                               : k_split_scatter<K, IPT, false, BALLOT, BLOCK, RO, true>);
+            EDPP_HIP(c, hipFuncSetAttribute((const void*)scatter, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ls));
+            hipLaunchKernelGGL(scatter, dim3((unsigned)g.tiles), dim3(BLOCK), ls, c->stream, a.kin, a.kout, a.vin, a.vout, g,
+                               (const int32_t*)his, a.gate);
             EDPP_HIP(c, hipGetLastError());
             return EDPP_OK;
         }
     }
     if (a.vin)
         hipLaunchKernelGGL((k_split_scatter<K, IPT, true, BALLOT, BLOCK, RO>), dim3((unsigned)g.tiles), dim3(BLOCK),
-                           ls, c->stream, a.kin, a.kout, a.vin, a.vout, g, (const int32_t*)his);
+                           ls, c->stream, a.kin, a.kout, a.vin, a.vout, g, (const int32_t*)his, a.gate);
     else
         hipLaunchKernelGGL((k_split_scatter<K, IPT, false, BALLOT, BLOCK, RO>), dim3((unsigned)g.tiles), dim3(BLOCK),
-                           ls, c->stream, a.kin, a.kout, a.vin, a.vout, g, (const int32_t*)his);
+                           ls, c->stream, a.kin, a.kout, a.vin, a.vout, g, (const int32_t*)his, a.gate);
     EDPP_HIP(c, hipGetLastError());
     return EDPP_OK;
 }
@@ -1351,7 +1354,8 @@ int launch_sort_u32(edpp_ctx* c, const uint32_t* kin, uint32_t* kout, const int3
     // samples before the passes, segment starts and list after them, share the counts' room
     int lg_segs = 14;
     while (n >> lg_segs > kLocalSortMean) ++lg_segs;
-    const bool local = n >= kLocalSortMin && lg_segs <= 16 && bits == 32 && !chained;
+    const bool varied = c->tune.split_reorder != EDPP_REORDER_NONE && c->tune.split_reorder != EDPP_REORDER_FIXED;
+    const bool local = n >= kLocalSortMin && lg_segs <= 16 && bits == 32 && !chained && varied;  // gated passes are varied
     const size_t cbytes = chained ? kChainSmallBytes
                           : local ? std::max((size_t)hlen * 4, ((size_t)2 << lg_segs) * 4 + 256)
                                   : (size_t)hlen * 4;

@@ -83,7 +83,6 @@ struct SplitGeom {
     int64_t tiles;
     int xcds;
     uint32_t flip;   // 0, or the top bucket bit: buckets of a signed top digit in order
-    SplitGate gate;
 };
 
 // Bucket of a key: bits [shift, shift + log2 B) of its low 32 bits, with the
