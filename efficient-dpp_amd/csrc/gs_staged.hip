@@ -30,10 +30,11 @@
 // elements, where whole lines are 17 M, and took 2.9 ms against 1.7 ms for the
 // second split and the bins.)
 //
-// 2^28 4-byte elements, random permutation, us per kernel: gather 185 + 62 +
-// 518 + 1420 + 587 (k_st_gather: 290 M L2 requests, 204 G/s; the others move
-// 10 to 12 B per element at 4.6 to 5 TB/s); scatter 170 + 37 + 885 + 255 + 14
-// + 885 + 579.
+// 2^28 4-byte elements, random permutation, us per kernel: gather 186 (first)
+// + 31 (prefixes) + 522 (split) + 1430 (gather: 290 M L2 requests, 204 G/s) +
+// 587 (return); the others move 10 to 12 B per element at 4.6 to 5 TB/s;
+// scatter 163 + 31 + 874 (split) + 254 (hist2) + 14 (rows2) + 880 (split2) +
+// 580 (bins).
 #include <algorithm>
 #include "ctx.hpp"
 #include "device.hpp"
