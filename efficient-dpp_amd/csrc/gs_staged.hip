@@ -737,6 +737,16 @@ template <class T>
 int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t n, bool scatter, bool* ran) {
     *ran = false;
     if (!gs_staged_applies(in, out, idx, n, (int)sizeof(T), scatter)) return EDPP_OK;
+    // A graph keeps the pointers it was captured with, and may be replayed when
+    // the workspace has been given back for a larger one, or beside other work
+    // on the context's gate words.  So a stream under capture takes the direct
+    // passes, of which a single one holds nothing but the caller's buffers.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();  // some other capture forbids the question
+        return EDPP_OK;
+    }
+    if (cap != hipStreamCaptureStatusNone) return EDPP_OK;
     constexpr int64_t S = kStTile<T>;
     StGeom g = {};
     g.n = n;
@@ -773,15 +783,6 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
                  o_bins = take(((size_t)g.W << g.lg_subs) * 4), o_sidx = take((size_t)n * 4),
                  o_sval = take((size_t)n * sizeof(T)), o_didx = take(two ? (size_t)n * 4 : 0),
                  o_dval = take(two ? (size_t)n * sizeof(T) : 0), o_slot = take(scatter ? 0 : (size_t)g.tiles * S * 2);
-    if (at > c->ws_bytes) {
-        // a stream under capture must not allocate: the direct passes then run
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess) {
-            (void)hipGetLastError();  // some other capture forbids the question
-            return EDPP_OK;
-        }
-        if (cap != hipStreamCaptureStatusNone) return EDPP_OK;
-    }
     void* w;
     int rc = ws_reserve(c, at, &w);
     if (rc == EDPP_ENOMEM) {  // the direct passes need no copies

@@ -120,7 +120,12 @@ typedef struct edpp_ctx edpp_ctx;
  * what torch reports for its default stream.  The context owns a
  * device workspace that grows on demand (hipMalloc outside the timed
  * kernels, as the reference allocates its temporaries per call,
- * opencl/primitives/scanImpl.cpp:39, splitImpl.cpp:76).                    */
+ * opencl/primitives/scanImpl.cpp:39, splitImpl.cpp:76).
+ * A captured call needs a workspace that is large enough already (make the
+ * call once before), and its graph holds the workspace it was captured with:
+ * replay it on the context's stream, and no more once a later call of the
+ * context has needed a larger one, or the context is gone.  Gathers and
+ * scatters in a single pass use no workspace.                              */
 int  edpp_ctx_create(int device, void* stream, edpp_ctx** out);
 int  edpp_ctx_destroy(edpp_ctx* ctx);
 int  edpp_ctx_sync(edpp_ctx* ctx);
@@ -149,8 +154,9 @@ int edpp_stream_i32(edpp_ctx* ctx, int op, const int32_t* a, const int32_t* b,
  * calls on large tables (512 MiB to 2 GiB; gathers of 8-byte elements from
  * 64 MiB) then order their indices by windows of the random side in the
  * context's workspace instead (up to 24 bytes per element), unless that
- * memory is not to be had or the stream is under capture and the workspace
- * too small; the output is the same.
+ * memory is not to be had or the stream is under capture; the output is the
+ * same.  Under capture a gather in one pass uses the caller's buffers only;
+ * see edpp_ctx for the calls that use the workspace.
  * idx must hold values in [0,n); for scatter it must be a permutation.      */
 int edpp_gather_i32 (edpp_ctx* ctx, const int32_t* in, int32_t* out, const int32_t* idx,
                      int64_t n, int passes, double* ms);
