@@ -13,8 +13,10 @@
 // after window, each from the L2 of the XCD that works on it, and brings the
 // values back into index order; a scatter moves its values along, down to
 // bins of 64 KiB of output, which it assembles in LDS.
-//   k_st_first   one read of the indices: chunks that are local are done at
-//                once; the others' elements are counted per window
+//   gather:      k_st_probe     whether the indices are scattered at all
+//   k_st_first   one read of the indices: chunks that are local, and a
+//                gather's if they are not scattered, are done at once; the
+//                others' elements are counted per window
 //   k_st_groups, k_st_totals   prefixes of the counts
 //   k_st_split   indices (scatter: and values) to window order, tile by tile
 //                through LDS; a gather keeps each element's slot in its tile
@@ -78,6 +80,8 @@ __device__ __forceinline__ int64_t st_vec(int64_t tile, int u, uint32_t tid) {
 __device__ __forceinline__ bool st_skip(uint32_t mask, int h, uint32_t tid) {
     return (mask >> (h * (kStBlock / 256) + (int)(tid >> 8))) & 1u;
 }
+// lg bits of a line's number
+__device__ __forceinline__ uint32_t st_line_hash(uint32_t line, int lg) { return (line * 0x9E3779B1u) >> (32 - lg); }
 // finished chunks of a tile as bits (the last tile's missing ones among them)
 template <int CH>
 __device__ __forceinline__ uint32_t st_done(const StGeom& g, int64_t tile) {
@@ -87,13 +91,96 @@ __device__ __forceinline__ uint32_t st_done(const StGeom& g, int64_t tile) {
     return m;
 }
 
+// Whether a gather's indices are scattered enough for the window order to pay.
+// It takes 2750 us for 2^28 4-byte elements almost whatever the indices are,
+// and a direct gather about 550 + 4900 d us, where d is the share of the
+// elements that fetch a line of their own: two interleaved halves take 520 us,
+// rows of 32 elements 530, 1000 distinct indices 910, a transposed 16384 x
+// 16384 table 1700, random indices within 4 MiB 1800 (3360, 2080, 1720, 2080
+// and 3410 in window order).  So d is measured: a workgroup takes
+// kStProbeRows chunks that follow each other on one XCD (every kStProbeStep-th
+// is on it), so that lines which its L2 keeps from one chunk to the next count
+// once, as in the transposition, and counts their distinct lines in a bitmap
+// of hashed line numbers, a quarter of the lines: 8192 elements in 2^16 bits,
+// of which random ones set 0.94 each.  8 us.
+constexpr int kStProbes = kWave;  // workgroups, spread evenly over the indices
+constexpr int kStProbeRows = 8, kStProbeStep = 16, kStProbeLg = 16;
+constexpr int kStProbeBlock = kStChunk / 4;
+__global__ __launch_bounds__(kStProbeBlock) void k_st_probe(const int32_t* __restrict__ idx, StGeom g, int lg_line) {
+    __shared__ uint32_t seen[1 << (kStProbeLg - 5)];
+    __shared__ uint32_t wd[kStProbeBlock / kWave], wm[kStProbeBlock / kWave];
+    const int t = threadIdx.x;
+    const uint32_t nall = (uint32_t)g.n;
+    constexpr int kSpan = (kStProbeRows - 1) * kStProbeStep + 1;
+    const int64_t first = std::max<int64_t>(g.chunks - kSpan, 0) * blockIdx.x / (kStProbes - 1);
+    uint32_t pos[kStProbeRows * 4];
+    #pragma unroll
+    for (int r = 0; r < kStProbeRows; ++r)
+        st_load<uint32_t, 4>(reinterpret_cast<const uint32_t*>(idx), (first + r * kStProbeStep) * (kStChunk / 4) + t, g.n,
+                             kStNone, pos + 4 * r);
+    for (int i = t; i < (1 << (kStProbeLg - 5)); i += kStProbeBlock) seen[i] = 0;
+    __syncthreads();
+    uint32_t m = 0, d = 0;
+    #pragma unroll
+    for (int e = 0; e < kStProbeRows * 4; ++e)
+        if (pos[e] < nall) {
+            ++m;
+            const uint32_t h = st_line_hash(pos[e] >> lg_line, kStProbeLg + 2);
+            if ((h & 3u) == 0) atomicOr(seen + (h >> 7), 1u << ((h >> 2) & 31));
+        }
+    __syncthreads();
+    for (int i = t; i < (1 << (kStProbeLg - 5)); i += kStProbeBlock) d += __popc(seen[i]);
+    d = wave_sum(d);
+    m = wave_sum(m);
+    if (lane_id() == 0) {
+        wd[t / kWave] = d;
+        wm[t / kWave] = m;
+    }
+    __syncthreads();
+    if (t < kWave) {
+        d = wave_sum(t < kStProbeBlock / kWave ? wd[t] : 0u);
+        m = wave_sum(t < kStProbeBlock / kWave ? wm[t] : 0u);
+        if (t == 0) {
+            g.probe[2 * blockIdx.x] = 4 * d;
+            g.probe[2 * blockIdx.x + 1] = m;
+        }
+    }
+}
+// The line lies where the window order is the faster one for certain: random
+// indices within 16 MiB (d = 0.87, direct 3700, in window order 2790 us) and
+// Zipf(0.8) ones (4710, 2730) are above it; below it, random ones within 8 MiB
+// (0.76: 2700, 3000), and Zipf(1) ones (0.6: 2930 and 2600, but 8-byte values
+// 1490 and 1770).  The same in every wave.
+__device__ __forceinline__ bool st_scattered(const StGeom& g) {
+    const uint2 y = reinterpret_cast<const uint2*>(g.probe)[lane_id()];
+    return wave_sum(y.x) * 16u > wave_sum(y.y) * 13u;
+}
+
 // One chunk per workgroup, of as many lanes as give a CU 32 waves beside the
-// LDS windows.  A chunk whose indices fall inside
-// kStLocal elements (a block-local permutation) goes through an LDS window: a
-// gather loads the window with consecutive loads and reads its values from
-// LDS; a scatter writes its values into the window and stores the covered
-// positions as runs.  One whose indices fall inside g.near elements is
-// addressed directly, as L2 holds that many.  The others are counted.
+// LDS windows.  A chunk whose indices fall inside kStLocal elements (a
+// block-local permutation) goes through an LDS window: a gather loads the
+// window with consecutive loads and reads its values from LDS; a scatter
+// writes its values into the window and stores the covered positions as runs.
+// A gather addresses a chunk directly if its indices fall inside g.near
+// elements, as L2 holds that many, and every chunk if the indices are not
+// scattered.  A scatter does so with a chunk that writes at least kStCover
+// sixteenths of the lines it touches, or whole 32-byte sectors by neighbouring
+// lanes, as most of that leaves L2 as whole lines or sectors.  The others are
+// counted.
+//
+// Scatters of 2^28 4-byte elements, us in one direct pass / in four / in
+// window order: two interleaved streams 590 / 1610 / 2690, 64 of them 1150 /
+// 1880 / 2680, rows of 32 elements 670 / 1910 / 2610, every second element
+// 1310 / 2160 / 2700, rows of 8 1950 / 2610 / 2740; but every eighth element
+// 6710 / 5480 / 2690, rows of 2 5620 / 3560 / 2770, 256 streams of random
+// lengths 3210 / 2530 / 2730.  The lines of a chunk are counted by hash in
+// bytes of LDS (k_st_first of a random scatter 166 us without, 202 so, 213 by
+// atomics on a bitmap).  Its lanes take 4 elements per step also of 8-byte
+// values, so that the lanes of one store touch fewer streams (128 streams 1240
+// us, by steps of 2 2040); a gather's stores have to be consecutive (470, by
+// steps of 4 820).
+constexpr uint32_t kStCover = 7;
+constexpr int kStLineLg = 12;
 template <class T>
 constexpr int kStFirstBlock = 64 * (int)sizeof(T);  // 256 or 512
 template <class T, bool SC>
@@ -102,23 +189,28 @@ __global__ __launch_bounds__(kStFirstBlock<T>) void k_st_first(const T* __restri
     constexpr int E = kStE<T>;
     constexpr int BL = kStFirstBlock<T>;
     constexpr int NW = BL / kWave;
-    constexpr int N = kStChunk / BL;  // elements per lane
+    constexpr int N = kStChunk / BL;  // elements per lane, in steps of P
+    constexpr int P = SC ? 4 : E;
     extern __shared__ uint32_t cnt[];  // [W << cl]
-    __shared__ T win[kStLocal];
-    __shared__ uint32_t wlo[NW], whi[NW];
+    __shared__ __attribute__((aligned(16))) T win[kStLocal];
+    uint8_t* seen = reinterpret_cast<uint8_t*>(win);  // [1 << kStLineLg] of a scatter that fills no window
+    __shared__ uint32_t wlo[NW], whi[NW], wsw[SC ? NW : 1];
     __shared__ uint32_t cov[SC ? kStLocal / 32 : 1];
     const int t = threadIdx.x, w = t / kWave;
-    const int64_t v0 = (int64_t)blockIdx.x * (kStChunk / E) + t;
+    const int64_t v0 = (int64_t)blockIdx.x * (kStChunk / P) + t;
     const uint32_t nall = (uint32_t)g.n;
     uint32_t pos[N];
     T val[N];
     #pragma unroll
-    for (int u = 0; u < N / E; ++u)
-        st_load<uint32_t, E>(reinterpret_cast<const uint32_t*>(idx), v0 + u * BL, g.n, kStNone, pos + E * u);
+    for (int u = 0; u < N / P; ++u)
+        st_load<uint32_t, P>(reinterpret_cast<const uint32_t*>(idx), v0 + u * BL, g.n, kStNone, pos + P * u);
+    const bool scattered = SC || st_scattered(g);
     const int cl = st_copies_lg(g.W);
     for (int i = t; i < (g.WP << cl); i += BL) cnt[i] = 0;
-    if (SC)
+    if (SC) {
         for (int i = t; i < kStLocal / 32; i += BL) cov[i] = 0;
+        for (int i = t; i < (1 << kStLineLg) / 4; i += BL) reinterpret_cast<uint32_t*>(win)[i] = 0;
+    }
     uint32_t lo = kStNone, hi = 0;
     #pragma unroll
     for (int e = 0; e < N; ++e)
@@ -131,9 +223,22 @@ __global__ __launch_bounds__(kStFirstBlock<T>) void k_st_first(const T* __restri
         lo = std::min(lo, (uint32_t)__shfl_xor((int)lo, o));
         hi = std::max(hi, (uint32_t)__shfl_xor((int)hi, o));
     }
+    constexpr int kLgLine = sizeof(T) == 4 ? 5 : 4;
+    uint32_t broken = 0;  // the wave's lane steps (4-byte elements: pairs of lanes) that touch more than one sector
+    if constexpr (SC) {
+        #pragma unroll
+        for (int u = 0; u < N / P; ++u) {
+            uint32_t x = 0;
+            #pragma unroll
+            for (int k = 1; k < P; ++k) x |= pos[P * u] ^ pos[P * u + k];
+            if (sizeof(T) == 4) x |= pos[P * u] ^ (uint32_t)__builtin_amdgcn_mov_dpp((int)pos[P * u], 0xB1, 0xf, 0xf, true);
+            broken += __popcll(ballot(x >> (kLgLine - 2) != 0));
+        }
+    }
     if (lane_id() == 0) {
         wlo[w] = lo;
         whi[w] = hi;
+        if (SC) wsw[w] = broken;
     }
     __syncthreads();
     #pragma unroll
@@ -143,8 +248,31 @@ __global__ __launch_bounds__(kStFirstBlock<T>) void k_st_first(const T* __restri
     }
     // the same in the whole workgroup from here on
     const bool some = lo <= hi;
-    const bool near = !some || hi - lo < g.near;
     const bool window = some && hi - lo < (uint32_t)kStLocal;
+    bool near = !some || window;
+    if constexpr (SC) {
+        broken = 0;
+        #pragma unroll
+        for (int x = 0; x < NW; ++x) broken += wsw[x];
+        near = near || 8 * broken <= kStChunk / P;
+        if (!near) {
+            // distinct lines, by hash (a few hundred where it matters)
+            #pragma unroll
+            for (int e = 0; e < N; ++e)
+                if (pos[e] < nall) seen[st_line_hash(pos[e] >> kLgLine, kStLineLg)] = 1;
+            __syncthreads();
+            uint32_t lines = 0;
+            #pragma unroll
+            for (int i = 0; i < (1 << kStLineLg) / 16 / kWave; ++i) {
+                const v4u32 y = reinterpret_cast<const v4u32*>(seen)[i * kWave + lane_id()];
+                lines += __popc(y[0]) + __popc(y[1]) + __popc(y[2]) + __popc(y[3]);
+            }
+            const uint32_t m = (uint32_t)std::min<int64_t>(g.n - (int64_t)blockIdx.x * kStChunk, kStChunk);
+            near = (wave_sum(lines) << kLgLine) * kStCover <= 16u * m;  // every wave sums all of them
+        }
+    } else {
+        near = near || hi - lo < g.near || !scattered;
+    }
     if (t == 0) {
         g.done[blockIdx.x] = near ? 1 : 0;
         // read first, and many words: one address that every workgroup stores
@@ -173,7 +301,8 @@ __global__ __launch_bounds__(kStFirstBlock<T>) void k_st_first(const T* __restri
     }
     if constexpr (SC) {
         #pragma unroll
-        for (int u = 0; u < N / E; ++u) st_load<T, E>(in, v0 + u * BL, g.n, T(0), val + E * u);
+        for (int u = 0; u < N / E; ++u)
+            st_load<T, E>(in, (v0 + u / (P / E) * BL) * (P / E) + u % (P / E), g.n, T(0), val + E * u);
         if (window) {
             #pragma unroll
             for (int e = 0; e < N; ++e)
@@ -690,6 +819,8 @@ int run_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, const StGeo
     constexpr size_t l3 = st_split_lds<T, SC>();
     const size_t l1 = ((size_t)g.WP << st_copies_lg(g.W)) * 4;
     T* sval = static_cast<T*>(b.sval);
+    if (!SC)
+        hipLaunchKernelGGL(k_st_probe, dim3(kStProbes), dim3(kStProbeBlock), 0, c->stream, idx, g, sizeof(T) == 4 ? 5 : 4);
     EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_split<T, SC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l3));
     hipLaunchKernelGGL((k_st_first<T, SC>), dim3((unsigned)g.chunks), dim3(kStFirstBlock<T>), l1, c->stream, in, out, idx, g);
     launch_st_prefix<CH>(c->stream, g, nullptr);
@@ -782,7 +913,8 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
                  o_tile2 = take(((size_t)g.WP + 1) * 4), o_win2 = take((size_t)tiles2 * 2), o_rows2 = take(((size_t)tiles2 << g.lg_subs) * 4),
                  o_bins = take(((size_t)g.W << g.lg_subs) * 4), o_sidx = take((size_t)n * 4),
                  o_sval = take((size_t)n * sizeof(T)), o_didx = take(two ? (size_t)n * 4 : 0),
-                 o_dval = take(two ? (size_t)n * sizeof(T) : 0), o_slot = take(scatter ? 0 : (size_t)g.tiles * S * 2);
+                 o_dval = take(two ? (size_t)n * sizeof(T) : 0), o_slot = take(scatter ? 0 : (size_t)g.tiles * S * 2),
+                 o_probe = take(scatter ? 0 : (size_t)kStProbes * 8);
     void* w;
     int rc = ws_reserve(c, at, &w);
     if (rc == EDPP_ENOMEM) {  // the direct passes need no copies
@@ -798,6 +930,7 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
     g.gsum = u32(o_gsum);
     g.total = u32(o_total);
     g.open = u32(o_open);
+    g.probe = u32(o_probe);
     g.base = u32(o_base);
     if (two) {
         g.tile2 = u32(o_tile2);
@@ -812,29 +945,32 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
                    : run_staged<T, false>(c, in, out, idx, g, b, 0);
 }
 
-// A call whose chunks all turn out local pays for the kernels behind the first
-// one, which return at once (2 to 9 us each with their dispatch), but not for
-// the later passes of the direct schedule.  us, direct / staged:
-//                      random permutation    4096-element blocks
-//   gather  4 B  2^26      1297 /  657           113 / 127
-//   gather  4 B  2^27      2581 / 1332           292 / 311
-//   gather  4 B  2^28      5464 / 2780           567 / 598
-//   scatter 4 B  2^26      1245 /  670           128 / 135
-//   scatter 4 B  2^27      2277 / 1376           347 / 331
-//   scatter 4 B  2^28      4485 / 2810           690 / 657
-//   gather  8 B  2^23       162 /  119            35 /  31
-//   gather  8 B  2^26      1327 /  870           283 / 247
-//   gather  8 B  2^27      2922 / 1822           554 / 484
-//   scatter 8 B  2^24       302 /  247            58 /  62
-//   scatter 8 B  2^26      1398 / 1021           286 / 279
-//   scatter 8 B  2^27      2798 / 2106           570 / 549
+// A call whose chunks are all done directly pays for the kernels around the
+// first one (the probe 8 us, those that return at once 2 to 8 us each), but
+// not for the later passes of the direct schedule.  us, direct schedule / by
+// this path:
+//                     random permutation   4096-element blocks   two halves
+//   gather  4 B  2^26     1281 /  666          112 / 135           97 / 123
+//   gather  4 B  2^27     2564 / 1337          289 / 317          257 / 285
+//   gather  4 B  2^28     5455 / 2766          562 / 606          518 / 551
+//   scatter 4 B  2^26     1241 /  682          127 / 137          218 / 143
+//   scatter 4 B  2^27     2276 / 1385          345 / 332          811 / 317
+//   scatter 4 B  2^28     4475 / 2826          684 / 650         1601 / 625
+//   gather  8 B  2^24      329 /  221           44 /  61           43 /  62
+//   gather  8 B  2^25      663 /  455           84 / 106           80 / 103
+//   gather  8 B  2^26     1317 /  890          226 / 258          222 / 247
+//   gather  8 B  2^27     2931 / 1832          451 / 495          462 / 495
+//   scatter 8 B  2^25      586 /  517          109 / 123          179 / 127
+//   scatter 8 B  2^26     1396 / 1022          286 / 289          620 / 290
+//   scatter 8 B  2^27     2795 / 2109          570 / 569         1216 / 558
 // So calls start at 512 MiB, from where a local gather and scatter together
-// take no longer than before (4 B, 2^26: 262 against 241 us), and gathers of
-// 8-byte elements, whose local chunks got faster, at 64 MiB.  The upper bound
-// is 1024 windows, and byte offsets of 31 bits.
+// take no longer than by the direct schedule or little more (4 B, 2^26: 272
+// against 239 us, 2^27: 649 and 634); a direct gather of smaller tables loses
+// a fifth or more where its indices are in streams.  The upper bound is 1024
+// windows, and byte offsets of 31 bits.
 bool gs_staged_applies(const void* in, const void* out, const int32_t* idx, int64_t n, int elem_bytes, bool scatter) {
     const int64_t bytes = n * elem_bytes;
-    const int64_t least = (elem_bytes == 8 && !scatter ? 64ll : 512ll) << 20;
+    const int64_t least = 512ll << 20;
     return aligned16(in) && aligned16(out) && aligned16(idx) && bytes >= least && bytes <= kStWindow * kStMaxWindows &&
            bytes < (1ll << 31);
 }

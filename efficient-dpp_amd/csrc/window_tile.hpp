@@ -63,7 +63,8 @@ struct StGeom {
     int64_t chunks, tiles, groups;
     int group;          // tiles per group, a power of two up to kStMaxGroup
     int xcds;
-    uint32_t near;      // a chunk whose indices span fewer elements is done directly
+    uint32_t near;      // a gather's chunk whose indices span fewer elements is done directly
+    uint32_t* probe;    // [2 * workgroup] distinct lines and elements that a gather's k_st_probe saw
     uint8_t* done;      // [chunks] chunk is finished (null: none is)
     uint16_t* count;    // [chunk][WP] elements per window of the chunks that are not
     uint32_t* rows;     // [tile][WP] elements of the window in the group's earlier tiles

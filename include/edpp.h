@@ -151,12 +151,12 @@ int edpp_stream_i32(edpp_ctx* ctx, int op, const int32_t* a, const int32_t* b,
  * opencl/primitives/gatherImpl.cpp:7-55, scatterImpl.cpp:9-54.  Pass k of
  * `passes` touches only indices in [k*ceil(n/passes), (k+1)*ceil(n/passes)).
  * passes == 0 picks the count from the context's schedule (tuner or model);
- * calls on large tables (512 MiB to 2 GiB; gathers of 8-byte elements from
- * 64 MiB) then order their indices by windows of the random side in the
- * context's workspace instead (up to 24 bytes per element), unless that
- * memory is not to be had or the stream is under capture; the output is the
- * same.  Under capture a gather in one pass uses the caller's buffers only;
- * see edpp_ctx for the calls that use the workspace.
+ * calls on large tables (512 MiB to 2 GiB) whose indices are scattered over
+ * them then order these by windows of the random side in the context's
+ * workspace instead (up to 24 bytes per element), unless that memory is not to
+ * be had or the stream is under capture; the output is the same.  Under
+ * capture a gather in one pass uses the caller's buffers only; see edpp_ctx
+ * for the calls that use the workspace.
  * idx must hold values in [0,n); for scatter it must be a permutation.      */
 int edpp_gather_i32 (edpp_ctx* ctx, const int32_t* in, int32_t* out, const int32_t* idx,
                      int64_t n, int passes, double* ms);
