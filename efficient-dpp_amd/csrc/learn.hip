@@ -656,6 +656,10 @@ int edpp_default_candidate(edpp_ctx* c, const edpp_call* q, int32_t* cand) {
     if (rc) return rc;
     const int fam = family_of(q->op);
     int scheme = 0, a = 0, b = 0;
+    *cand = -1;
+    // large gathers and scatters go by windows or in one pass, as their
+    // indices ask: no candidate does
+    if (fam == 1 && gs_staged_applies(q->in, q->out, q->idx, q->n, q->elem_bytes, q->op == EDPP_OP_SCATTER)) return EDPP_OK;
     if (fam == 0) {
         scheme = default_scan_scheme(c, q->n, q->elem_bytes);
         if (scheme == EDPP_SCAN_LOOKBACK) default_scan_shape(c, q->n, &a, &b);
@@ -667,7 +671,6 @@ int edpp_default_candidate(edpp_ctx* c, const edpp_call* q, int32_t* cand) {
         scheme = default_split_strategy(c, q->n, q->buckets);
         default_split_shape(c, q->n, q->buckets, q->elem_bytes, &a, &b);
     }
-    *cand = -1;
     for (int k = 0; k < K; ++k) {
         const Cand& d = kCands[k];
         if (d.family != fam || d.scheme != scheme) continue;

@@ -64,7 +64,8 @@ int edpp_call_run(edpp_ctx* ctx, const edpp_call* call, int32_t cand, double* ms
  * of other families.  times has EDPP_MAX_CANDIDATES entries. */
 int edpp_autotune(edpp_ctx* ctx, const edpp_call* call, int32_t reps, double* times);
 /* The candidate the built-in schedule (no model) gives this call, or -1 when
- * that schedule is none of the candidates. */
+ * that schedule is none of the candidates (gathers and scatters of 512 MiB or
+ * more, which edpp.h describes). */
 int edpp_default_candidate(edpp_ctx* ctx, const edpp_call* call, int32_t* cand);
 /* Features of a call, computed on the device from samples of its inputs. */
 int edpp_call_features(edpp_ctx* ctx, const edpp_call* call, float* d_features);
@@ -100,7 +101,8 @@ int edpp_ctx_set_model(edpp_ctx* ctx, edpp_mlp* m);
  * either setting forgets the remembered choices. */
 int edpp_mlp_memo(edpp_mlp* m, int32_t enabled);
 /* The candidate the context's model picks for the call (through the memo), as
- * an AUTO call would; EDPP_EINVAL when no model is set. */
+ * an AUTO call would where it asks the model (not for gathers and scatters
+ * that edpp.h says may go by windows); EDPP_EINVAL when no model is set. */
 int edpp_model_choice(edpp_ctx* ctx, const edpp_call* call, int32_t* cand);
 
 #ifdef __cplusplus
