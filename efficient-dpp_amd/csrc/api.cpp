@@ -49,6 +49,31 @@ static int grow(edpp_ctx* c, void** ws, size_t* ws_bytes, size_t bytes, void** o
     return EDPP_OK;
 }
 int ws_reserve(edpp_ctx* c, size_t bytes, void** out) { return grow(c, &c->ws, &c->ws_bytes, bytes, out); }
+// The new block is taken before the old one is given back, so that a refusal
+// changes nothing; a size that was refused is not asked for again.
+int ws_try_reserve(edpp_ctx* c, size_t bytes, void** out) {
+    *out = nullptr;
+    bytes = (bytes + 255) & ~(size_t)255;
+    if (bytes > c->ws_bytes) {
+        if (c->ws_refused && bytes >= c->ws_refused) return EDPP_OK;
+        void* p = nullptr;
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            c->ws_refused = bytes;
+            return EDPP_OK;
+        }
+        hipError_t e = c->ws ? hipStreamSynchronize(c->stream) : hipSuccess;  // earlier kernels may still use it
+        if (e == hipSuccess && c->ws) e = hipFree(c->ws);
+        if (e != hipSuccess) {
+            hipFree(p);
+            return hip_fail(c, e, "workspace");
+        }
+        c->ws = p;
+        c->ws_bytes = bytes;
+    }
+    *out = c->ws;
+    return EDPP_OK;
+}
 int ws_outer_reserve(edpp_ctx* c, size_t bytes, void** out) {
     return grow(c, &c->ws_outer, &c->ws_outer_bytes, bytes, out);
 }
@@ -386,9 +411,12 @@ static int gs_common(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
     if (n > 0 && (const void*)in == (const void*)out) return fail(c, EDPP_EINVAL, "in and out must differ");
     int rc = timing_begin(c, ms);
     if (!rc) {
-        // the staged path is faster than every pass count where it applies, so
-        // the model, which chooses among pass counts, is not asked there
-        if (passes == 0 && c->model && n > 0 && !gs_staged_applies(in, out, idx, n, (int)sizeof(T), scatter)) {
+        // The window order looks at the indices itself; the model, which
+        // chooses among pass counts, is asked where it does not take the call.
+        bool ran = false;
+        if (passes == 0) rc = launch_gs_staged<T>(c, in, out, idx, n, scatter, &ran);
+        if (rc || ran) {
+        } else if (passes == 0 && c->model && n > 0) {
             edpp_call q = {};
             q.op = scatter ? EDPP_OP_SCATTER : EDPP_OP_GATHER;
             q.elem_bytes = (int32_t)sizeof(T);

@@ -18,6 +18,7 @@ struct edpp_ctx {
     // grow-only scratch for per-call temporaries (histograms, partials)
     void* ws = nullptr;
     size_t ws_bytes = 0;
+    size_t ws_refused = 0;  // size of the last ws_try_reserve that was refused, 0: none
     // scratch of composite calls (hash join) that hold buffers across the
     // primitives they call, which use ws
     void* ws_outer = nullptr;
@@ -71,6 +72,9 @@ int hip_fail(edpp_ctx* c, hipError_t e, const char* what);
 // workspace of at least `bytes` (256-byte aligned); may synchronise to grow
 int ws_reserve(edpp_ctx* c, size_t bytes, void** out);
 int ws_outer_reserve(edpp_ctx* c, size_t bytes, void** out);
+// the same for a caller that can do without: *out is null, with EDPP_OK, where
+// the memory is not to be had
+int ws_try_reserve(edpp_ctx* c, size_t bytes, void** out);
 int zero_fill(edpp_ctx* c, void* p, size_t bytes);  // kernel, graph-capturable
 // look-back state for at least `tiles` tiles; returns the epoch for this call
 int scan_state_acquire(edpp_ctx* c, int64_t tiles, uint32_t* epoch_out);
@@ -94,7 +98,7 @@ int launch_scan(edpp_ctx* c, const T* in, T* out, int64_t n, int scheme, T* d_to
 template <class T>
 int launch_gather(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t n, int passes, bool scatter);
 // gather / scatter through L2-sized windows of the random side; *ran says
-// whether it took the call (launch_gather's passes run otherwise)
+// whether it took the call (a pass count is to be chosen otherwise)
 template <class T>
 int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t n, bool scatter, bool* ran);
 bool gs_staged_applies(const void* in, const void* out, const int32_t* idx, int64_t n, int elem_bytes, bool scatter);

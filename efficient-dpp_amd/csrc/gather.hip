@@ -304,12 +304,7 @@ static void dispatch_unroll(edpp_ctx* c, int u, const T* in, T* out, const int32
 template <class T>
 int launch_gather(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64_t n, int passes, bool scatter) {
     if (n == 0) return EDPP_OK;
-    if (passes == 0) {
-        bool ran = false;
-        int rc = launch_gs_staged<T>(c, in, out, idx, n, scatter, &ran);
-        if (rc || ran) return rc;
-        passes = default_passes(c, n, (int)sizeof(T), scatter);
-    }
+    if (passes == 0) passes = default_passes(c, n, (int)sizeof(T), scatter);
     if (passes < 1 || passes > n) passes = passes < 1 ? 1 : (int)n;
     const bool vec = aligned16(in) && aligned16(out) && aligned16(idx);
     const int e = scatter ? kGsE<T, true> : kGsE<T, false>, block = 1024 / e;

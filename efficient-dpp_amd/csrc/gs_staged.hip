@@ -916,12 +916,8 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
                  o_dval = take(two ? (size_t)n * sizeof(T) : 0), o_slot = take(scatter ? 0 : (size_t)g.tiles * S * 2),
                  o_probe = take(scatter ? 0 : (size_t)kStProbes * 8);
     void* w;
-    int rc = ws_reserve(c, at, &w);
-    if (rc == EDPP_ENOMEM) {  // the direct passes need no copies
-        (void)hipGetLastError();
-        return EDPP_OK;
-    }
-    if (rc) return rc;
+    int rc = ws_try_reserve(c, at, &w);
+    if (rc || !w) return rc;  // the direct passes need no copies
     char* p = static_cast<char*>(w);
     auto u32 = [p](size_t o) { return reinterpret_cast<uint32_t*>(p + o); };
     g.done = reinterpret_cast<uint8_t*>(p + o_done);

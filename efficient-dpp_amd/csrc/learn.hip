@@ -596,9 +596,15 @@ int edpp_call_run(edpp_ctx* c, const edpp_call* q, int32_t cand, double* ms) {
     if (rc) return rc;
     if (q->n > 0) {
         if (cand < 0) {
-            const bool staged = (q->op == EDPP_OP_GATHER || q->op == EDPP_OP_SCATTER) &&
-                                gs_staged_applies(q->in, q->out, q->idx, q->n, q->elem_bytes, q->op == EDPP_OP_SCATTER);
-            if (c->model && !staged) {
+            bool ran = false;
+            if (q->op == EDPP_OP_GATHER || q->op == EDPP_OP_SCATTER)
+                rc = q->elem_bytes == 8
+                         ? launch_gs_staged<uint64_t>(c, (const uint64_t*)q->in, (uint64_t*)q->out, q->idx, q->n,
+                                                      q->op == EDPP_OP_SCATTER, &ran)
+                         : launch_gs_staged<uint32_t>(c, (const uint32_t*)q->in, (uint32_t*)q->out, q->idx, q->n,
+                                                      q->op == EDPP_OP_SCATTER, &ran);
+            if (rc || ran) {
+            } else if (c->model) {
                 int k;
                 rc = model_choose(c, *q, &k);
                 if (!rc) rc = run_candidate(c, *q, k, nullptr);
