@@ -22,8 +22,8 @@
 //                through LDS; a gather keeps each element's slot in its tile
 //   gather:      k_st_gather    values, window after window
 //                k_st_return    values back to their tiles and into order
-//   scatter:     k_st_hist2, k_st_rows2, k_st_split2   a second split, above
-//                               1024 bins
+//   scatter:     k_st_hist2, k_st_rows2, k_st_split2   a second split, of
+//                               windows into bins
 //                k_st_bins      every bin of the output through LDS
 // The order of a window's elements is free, so ranks come from LDS counters
 // (one atomic with return per element) and need no matching of lanes.
@@ -49,8 +49,6 @@ namespace {
 
 constexpr int64_t kStWindow = 2 << 20;    // bytes of the random side per window (an XCD's L2 holds 4 MiB)
 constexpr int kStBin = 64 << 10;          // bytes of the output a scatter's workgroup assembles in LDS
-constexpr int kStOneLevel = 1024;         // bins up to which a scatter splits once (2^24 4-byte elements: 151 against
-                                          // 167 us in two, with 32 windows of 32 bins)
 constexpr int kStLocal = 4096;            // elements of a local chunk's LDS window
 
 // Elements per 16-byte vector of T: 4 or 2.  A lane's step is one such vector
@@ -625,8 +623,7 @@ __global__ __launch_bounds__(kStBlock, kStBlock / 128) void k_st_split2(StGeom g
 // LDS: every covered line leaves whole
 constexpr int kStBinBlock = 1024;
 template <class T>
-__global__ __launch_bounds__(kStBinBlock, kStBinBlock / 128) void k_st_bins(StGeom g, const uint32_t* __restrict__ first,
-                                                                            int64_t nbins,
+__global__ __launch_bounds__(kStBinBlock, kStBinBlock / 128) void k_st_bins(StGeom g, int64_t nbins,
                                                                             const uint32_t* __restrict__ didx,
                                                                             const T* __restrict__ dval,
                                                                             T* __restrict__ out) {
@@ -639,7 +636,7 @@ __global__ __launch_bounds__(kStBinBlock, kStBinBlock / 128) void k_st_bins(StGe
     for (uint32_t ob = blockIdx.x; ob < (uint32_t)nbins; ob += gridDim.x) {
     const int64_t bin = st_order(ob, (uint32_t)nbins, g.xcds);
     const uint32_t m = std::min<uint32_t>(g.base[g.W], (uint32_t)g.n);
-    const uint32_t lo = std::min(first[bin], m), hi = bin + 1 < nbins ? std::min(first[bin + 1], m) : m;
+    const uint32_t lo = std::min(g.bins[bin], m), hi = bin + 1 < nbins ? std::min(g.bins[bin + 1], m) : m;
     if (lo >= hi) continue;  // the same in the whole workgroup
     const uint32_t o0 = (uint32_t)bin * (uint32_t)E;
     for (int i = threadIdx.x; i < E / 32; i += kStBinBlock) cov[i] = 0;
@@ -826,24 +823,17 @@ int run_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, const StGeo
     launch_st_prefix<CH>(c->stream, g, nullptr);
     hipLaunchKernelGGL((k_st_split<T, SC>), dim3(grid), dim3(kStBlock), l3, c->stream, in, idx, g, b.sidx, sval, b.slot);
     if constexpr (SC) {
-        const uint32_t* first = g.base;
-        const uint32_t* fidx = b.sidx;
-        const T* fval = sval;
-        if (g.tile2) {
-            const unsigned grid2 = (unsigned)(g.tiles + g.W);  // a window's last tile may be short
-            EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_split2<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l3));
-            hipLaunchKernelGGL((k_st_hist2<T>), dim3(grid2), dim3(kStBlock), 0, c->stream, g, (const uint32_t*)b.sidx);
-            hipLaunchKernelGGL(k_st_rows2, dim3((unsigned)g.W), dim3(kStRowBlock), 0, c->stream, g);
-            hipLaunchKernelGGL((k_st_split2<T>), dim3(grid2), dim3(kStBlock), l3, c->stream, g, (const uint32_t*)b.sidx,
-                               (const T*)sval, b.didx, static_cast<T*>(b.dval));
-            first = g.bins;
-            fidx = b.didx;
-            fval = static_cast<const T*>(b.dval);
-        }
+        const unsigned grid2 = (unsigned)(g.tiles + g.W);  // a window's last tile may be short
+        T* dval = static_cast<T*>(b.dval);
+        EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_split2<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l3));
+        hipLaunchKernelGGL((k_st_hist2<T>), dim3(grid2), dim3(kStBlock), 0, c->stream, g, (const uint32_t*)b.sidx);
+        hipLaunchKernelGGL(k_st_rows2, dim3((unsigned)g.W), dim3(kStRowBlock), 0, c->stream, g);
+        hipLaunchKernelGGL((k_st_split2<T>), dim3(grid2), dim3(kStBlock), l3, c->stream, g, (const uint32_t*)b.sidx,
+                           (const T*)sval, b.didx, dval);
         constexpr size_t l6 = kStBin + kStBin / sizeof(T) / 8;
         EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_bins<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l6));
         hipLaunchKernelGGL((k_st_bins<T>), dim3((unsigned)std::min<int64_t>(nbins, (int64_t)std::max(c->cus, 1) * 4)),
-                           dim3(kStBinBlock), l6, c->stream, g, first, nbins, fidx, fval, out);
+                           dim3(kStBinBlock), l6, c->stream, g, nbins, (const uint32_t*)b.didx, (const T*)dval, out);
     } else {
         constexpr size_t l5 = st_return_lds<T>();
         EDPP_HIP(c, hipFuncSetAttribute((const void*)k_st_return<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l5));
@@ -887,20 +877,18 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
     g.groups = ceil_div(g.tiles, (int64_t)g.group);
     g.xcds = c->xcds;
     g.near = (uint32_t)(kStWindow / (int64_t)sizeof(T));
-    bool two = false;
     int64_t nbins = 0;
     if (!scatter) {
         g.shift = st_ceil_lg(kStWindow / (int64_t)sizeof(T));
-    } else {
+    } else {  // 128 to 256 windows of 64 or 128 bins
         g.sub_shift = st_ceil_lg(kStBin / (int64_t)sizeof(T));
         nbins = ceil_div(n, 1ll << g.sub_shift);
-        two = nbins > kStOneLevel;
-        g.lg_subs = two ? st_ceil_lg(nbins) / 2 : 0;
+        g.lg_subs = st_ceil_lg(nbins) / 2;
         g.shift = g.sub_shift + g.lg_subs;
     }
     g.W = (int)ceil_div(n, 1ll << g.shift);
     g.WP = (g.W + 1) & ~1;
-    const int64_t tiles2 = two ? g.tiles + g.W : 0;
+    const int64_t tiles2 = scatter ? g.tiles + g.W : 0;
     // workspace, in this order
     size_t at = 0;
     auto take = [&at](size_t bytes) {
@@ -912,8 +900,8 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
                  o_rows = take((size_t)g.tiles * g.WP * 4), o_gsum = take((size_t)g.groups * g.WP * 4), o_total = take((size_t)g.WP * 4), o_open = take(4), o_base = take(((size_t)g.WP + 1) * 4),
                  o_tile2 = take(((size_t)g.WP + 1) * 4), o_win2 = take((size_t)tiles2 * 2), o_rows2 = take(((size_t)tiles2 << g.lg_subs) * 4),
                  o_bins = take(((size_t)g.W << g.lg_subs) * 4), o_sidx = take((size_t)n * 4),
-                 o_sval = take((size_t)n * sizeof(T)), o_didx = take(two ? (size_t)n * 4 : 0),
-                 o_dval = take(two ? (size_t)n * sizeof(T) : 0), o_slot = take(scatter ? 0 : (size_t)g.tiles * S * 2),
+                 o_sval = take((size_t)n * sizeof(T)), o_didx = take(scatter ? (size_t)n * 4 : 0),
+                 o_dval = take(scatter ? (size_t)n * sizeof(T) : 0), o_slot = take(scatter ? 0 : (size_t)g.tiles * S * 2),
                  o_probe = take(scatter ? 0 : (size_t)kStProbes * 8);
     void* w;
     int rc = ws_try_reserve(c, at, &w);
@@ -928,7 +916,7 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
     g.open = u32(o_open);
     g.probe = u32(o_probe);
     g.base = u32(o_base);
-    if (two) {
+    if (scatter) {
         g.tile2 = u32(o_tile2);
         g.win2 = reinterpret_cast<uint16_t*>(p + o_win2);
         g.rows2 = u32(o_rows2);
