@@ -35,7 +35,8 @@ namespace {
 constexpr int kPhaseHist = 0, kPhaseHistScan = 1, kPhaseMain = 2, kPhaseScatter = 3;
 
 struct DJob {
-    int32_t kind, wide, lg, pad;
+    int32_t kind, wide, lg;
+    int32_t column;  // split: one workgroup scans his, a lane per bucket
     int64_t n, tiles, hscan_tiles;
     const void* in;
     void* out;
@@ -219,17 +220,18 @@ __device__ void hist_scan_tile(const DJob& J, int64_t t, char* smem, uint32_t sp
     }
 }
 
-// The same for a job of at most kColumnTiles tiles, by one workgroup: a lane
-// takes a bucket (BLOCK >> lg lanes a range of the tiles each), so that every
-// access of a wave is whole lines, and nothing is looked back for.  (With
+// The same for a job of at most kColumnTiles tiles by one workgroup, where
+// column_scan says so: a lane takes a bucket (BLOCK >> lg lanes a range of the
+// tiles each), so that every access of a wave is whole lines, and nothing is
+// looked back for.  (With
 // bucket-major lanes, the scans of the 10,000-job mix, 11 M words, took 174 us
 // by themselves, a request for almost every word; the mix took 1.79 ms, and
-// 1.67 ms so.  From about 256 tiles on one workgroup's chain of reads would be
-// the longest of the launch.)
+// 1.67 ms so.)
 constexpr int64_t kColumnTiles = 256;
+constexpr int kColumnRows = 16;  // words of a lane in flight
 template <int BLOCK>
 __device__ void hist_column_scan(const DJob& J, char* smem, uint32_t spin_limit, int32_t* err) {
-    constexpr int R = 16;  // words in flight
+    constexpr int R = kColumnRows;
     uint32_t* sums = reinterpret_cast<uint32_t*>(smem);  // [bucket][range]
     uint32_t* wtmp = sums + BLOCK;
     const uint32_t B = 1u << J.lg, tiles = (uint32_t)J.tiles;
@@ -495,7 +497,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch(const DJob* __restrict__ jobs, 
             if (J.wide) split_hist_tile<uint64_t, IPT, BLOCK>(J, t, lds);
             else split_hist_tile<uint32_t, IPT, BLOCK>(J, t, lds);
         } else if (phase == kPhaseHistScan) {
-            if (J.tiles <= kColumnTiles) hist_column_scan<BLOCK>(J, smem, spin_limit, err);
+            if (J.column) hist_column_scan<BLOCK>(J, smem, spin_limit, err);
             else hist_scan_tile<BLOCK>(J, t, smem, spin_limit, err);
         } else if (phase == kPhaseScatter) {
             if (J.wide) split_scatter_tile<uint64_t, IPT, BLOCK>(J, t, lds, spin_limit, err);
@@ -621,6 +623,20 @@ static int validate_jobs(edpp_ctx* c, const edpp_job* jobs, int32_t njobs) {
     return EDPP_OK;
 }
 
+// Whether one workgroup scans a split job's counts (hist_column_scan): where
+// the words of a lane are in flight at once, and else where the launch is long
+// enough to hide the workgroup's chain of readings, about 6 us for each
+// kColumnRows words of a lane; 3 times that, as the job's own tiles wait for it.
+// 256 buckets, us, by column / by look-back: 1 job of 40,000 keys 33 / 31, of
+// 100,000 44 / 34, of 524,288 165 / 49; 16 jobs of 524,288 172 / 115, 64 of
+// them 382 / 357, 128 of them 665 / 700; 128 jobs of 100,000 126 / 146.
+static int column_scan(const BatchShape& sh, const DJob& d, double batch_us) {
+    if (d.tiles > kColumnTiles) return 0;
+    const int64_t ranges = std::min<int64_t>(sh.block >> d.lg, d.tiles);
+    const int64_t rounds = ceil_div(ceil_div(d.tiles, ranges), (int64_t)kColumnRows);
+    return rounds == 1 || 18.0 * (double)rounds <= batch_us ? 1 : 0;
+}
+
 // Builds the work queue and state of b->jobs for b->shape and uploads them.
 static int plan(edpp_batch* b) {
     edpp_ctx* c = b->ctx;
@@ -632,6 +648,12 @@ static int plan(edpp_batch* b) {
     // its look-back status words and, for a split, its tagged histogram words
     int64_t words = (int64_t)kMaxQueues * kTicketStride;
     std::vector<int64_t> soff(njobs, -1);
+    double batch_us = 0;  // about what the launch takes, at 2.5 TB/s
+    for (int32_t j = 0; j < njobs; ++j) {
+        const edpp_job& q = b->jobs[j];
+        const int64_t per = 2 * q.elem_bytes + (q.kind == EDPP_JOB_SPLIT ? 8 : q.kind == EDPP_JOB_GATHER ? 4 : 0);
+        batch_us += (double)q.n * (double)per * 4e-7;
+    }
     for (int32_t j = 0; j < njobs; ++j) {
         const edpp_job& q = b->jobs[j];
         DJob& d = dj[j];
@@ -654,7 +676,8 @@ static int plan(edpp_batch* b) {
         } else if (q.kind == EDPP_JOB_SPLIT && d.tiles > 1) {
             // (a job of one tile takes its offsets from its own counts)
             const int64_t hlen = ((int64_t)1 << d.lg) * d.tiles;
-            d.hscan_tiles = d.tiles <= kColumnTiles ? 1 : ceil_div(hlen, hscan_tile_elems(sh));
+            d.column = column_scan(sh, d, batch_us);
+            d.hscan_tiles = d.column ? 1 : ceil_div(hlen, hscan_tile_elems(sh));
             words += 2 * d.hscan_tiles + 2 * hlen;  // u64 status, then u64 histogram words
         }
         words = (words + 3) & ~(int64_t)3;  // 16-byte alignment of every job's state
