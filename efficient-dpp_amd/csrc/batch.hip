@@ -381,49 +381,47 @@ __device__ void split_scatter_tile(const DJob& J, int64_t t, uint32_t* lds, uint
 }
 
 // ---------------------------------------------------------------- gather tiles
-// A tile of BLOCK*4*U elements, in steps of one 16-byte vector of output per
-// lane (4 or 2 elements), so that a wave's stores are whole lines for both
-// widths
+// A tile of BLOCK*4*U elements: U rounds of one 16-byte index vector per lane
 template <class T, int BLOCK, int U>
 __device__ void gather_tile(const DJob& J, int64_t t) {
-    typedef typename vec16<T>::type V;
-    constexpr int E = vec16<T>::n, S = 4 * U / E;
-    typedef uint32_t vidx __attribute__((ext_vector_type(E)));
     const T* in = static_cast<const T*>(J.in);
     T* out = static_cast<T*>(J.out);
     const uint32_t n = (uint32_t)J.n;
     const int64_t base = t * (int64_t)BLOCK * 4 * U;
     if (base + (int64_t)BLOCK * 4 * U <= J.n) {
         // a whole tile: every index vector, then every random read, then the
-        // stores, so that each group of loads is in flight at once; a step's
-        // valid indices leave as one 16-byte store (batch buffers are 16-byte
-        // aligned)
-        vidx x[S];
+        // stores, so that each group of loads is in flight at once; four
+        // valid indices leave as one 16-byte store per 16 bytes of output
+        // (batch buffers are 16-byte aligned)
+        v4u32 x[U];
         #pragma unroll
-        for (int u = 0; u < S; ++u)
-            x[u] = ld_stream(reinterpret_cast<const vidx*>(J.idx + base + (int64_t)u * BLOCK * E + threadIdx.x * E));
+        for (int u = 0; u < U; ++u)
+            x[u] = ld_stream(reinterpret_cast<const v4u32*>(J.idx + base + (int64_t)u * BLOCK * 4 + threadIdx.x * 4));
         __builtin_amdgcn_sched_barrier(0);
-        T v[S][E];
+        T v[U][4];
         #pragma unroll
-        for (int u = 0; u < S; ++u)
+        for (int u = 0; u < U; ++u)
             #pragma unroll
-            for (int k = 0; k < E; ++k) v[u][k] = (uint32_t)x[u][k] < n ? in[(uint32_t)x[u][k]] : T(0);
+            for (int k = 0; k < 4; ++k) v[u][k] = (uint32_t)x[u][k] < n ? in[(uint32_t)x[u][k]] : T(0);
         __builtin_amdgcn_sched_barrier(0);
         #pragma unroll
-        for (int u = 0; u < S; ++u) {
-            const int64_t e0 = base + (int64_t)u * BLOCK * E + threadIdx.x * E;
-            bool all = true;
-            V o;
-            #pragma unroll
-            for (int k = 0; k < E; ++k) {
-                all = all && (uint32_t)x[u][k] < n;
-                o[k] = v[u][k];
-            }
+        for (int u = 0; u < U; ++u) {
+            const int64_t e0 = base + (int64_t)u * BLOCK * 4 + threadIdx.x * 4;
+            const bool all = (uint32_t)x[u][0] < n && (uint32_t)x[u][1] < n && (uint32_t)x[u][2] < n &&
+                             (uint32_t)x[u][3] < n;
             if (all) {
-                st_stream(o, reinterpret_cast<V*>(out + e0));
+                typedef typename vec16<T>::type V;
+                constexpr int EPV = vec16<T>::n;
+                #pragma unroll
+                for (int h = 0; h < 4 / EPV; ++h) {
+                    V o;
+                    #pragma unroll
+                    for (int k = 0; k < EPV; ++k) o[k] = v[u][h * EPV + k];
+                    st_stream(o, reinterpret_cast<V*>(out + e0 + h * EPV));
+                }
             } else {
                 #pragma unroll
-                for (int k = 0; k < E; ++k)
+                for (int k = 0; k < 4; ++k)
                     if ((uint32_t)x[u][k] < n) out[e0 + k] = v[u][k];
             }
         }
