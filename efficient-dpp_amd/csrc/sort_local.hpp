@@ -19,7 +19,11 @@
 // in 32 bits (three workgroups per CU instead of four, 1160), several segments
 // per workgroup (1300), the compiler's own form of the match (keys alone 980
 // instead of 830).  Keys far from even pay for the look and the launches
-// that leave: 4790 instead of 4690 (2^28 pairs of 20 bits), 2 to 3 % at 2^26.
+// that leave: 38 us at 2^26, 54 at 2^28, which is 4790 instead of 4740 (2^28
+// pairs of 20 bits) and 3 to 4 % at 2^26.  The look lets a segment pass that
+// holds up to 0.1 % of the keys: one such segment, which a single workgroup
+// then orders, takes the gain (2^26 pairs 1310 instead of 1280, 2^28 5000
+// instead of 4960), three of half the size leave most of it (1210, 4320).
 #pragma once
 #include <algorithm>
 #include "ctx.hpp"
@@ -126,13 +130,15 @@ __global__ __launch_bounds__(256) void k_sort_starts(const uint32_t* __restrict_
 }
 
 // Stable ranks of the wave's rows among its own elements, old[j] + below[j] of
-// a lane's item j < rows, and its counts per digit in row[].
+// a lane's item j < rows, and its counts per digit in row[], which are cleared
+// by pairs (each row starts on a word) before they are counted.
+typedef uint32_t __attribute__((may_alias)) SlPair;
 template <int BITS, int SHIFT, int ROWS>
 __device__ __forceinline__ void sl_rank(const uint32_t (&x)[ROWS], int rows, uint16_t* row, uint32_t (&old)[ROWS],
                                         uint32_t (&below)[ROWS]) {
     constexpr int B = 1 << BITS;
     #pragma unroll
-    for (int i = 0; i < B / kWave / 2; ++i) reinterpret_cast<uint32_t*>(row)[i * kWave + lane_id()] = 0;
+    for (int i = 0; i < B / kWave / 2; ++i) reinterpret_cast<SlPair*>(row)[i * kWave + lane_id()] = 0;
     #pragma unroll
     for (int j = 0; j < ROWS; ++j) {
         if (j >= rows) continue;
@@ -200,7 +206,7 @@ template <int CAP, bool KV, int BITS>
 struct SlLds {
     uint32_t comp[CAP];
     int32_t val[KV ? CAP : 1];
-    uint16_t hist[(kSlBlock / kWave) << BITS];
+    alignas(16) uint16_t hist[(kSlBlock / kWave) << BITS];
     uint32_t wtmp[kSlBlock / kWave];
 };
 
@@ -337,7 +343,7 @@ __device__ __forceinline__ void sl_long_pass(const uint32_t* ks, const int32_t* 
 template <bool KV, int BITS1, int BITS2>
 __global__ __launch_bounds__(kSlBlock) void k_sort_longer(uint32_t* keys, int32_t* vals, uint32_t* tkeys, int32_t* tvals,
                                                           SlGeom g) {
-    __shared__ uint16_t hist[(kSlBlock / kWave) << BITS1];
+    __shared__ alignas(16) uint16_t hist[(kSlBlock / kWave) << BITS1];
     __shared__ uint32_t run[1 << BITS1], wtmp[kSlBlock / kWave];
     if (g.gate[0]) return;
     const uint32_t entries = g.gate[1];
@@ -366,7 +372,7 @@ __global__ __launch_bounds__(kOneBlock) void k_sort_one(const uint32_t* kin, uin
     constexpr int W = kOneBlock / kWave;
     __shared__ uint32_t keys[ROWS * kOneBlock];
     __shared__ int32_t vals[KV ? ROWS * kOneBlock : 1];
-    __shared__ uint16_t hist[W << 8];
+    __shared__ alignas(16) uint16_t hist[W << 8];
     __shared__ uint32_t wtmp[W];
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
     const int all = (g.n + kWave - 1) / kWave, per = all / W, rem = all % W;
