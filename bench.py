@@ -441,7 +441,7 @@ def main():
                      "traffic": round(traffic["FETCH_SIZE"]["bytes"] + traffic["WRITE_SIZE"]["bytes"]) if traffic
                      else None,
                      "kernel": "k_gather, one launch per pass" if passes else
-                     "gather call (k_st_first, k_st_prefix, k_st_split, k_st_gather, k_st_return)",
+                     "gather call (k_st_probe, k_st_first, k_st_groups, k_st_totals, k_st_split, k_st_gather, k_st_return)",
                      "algorithmic_bytes_per_call": 12 * n,
                      "avg_call_ms": round(g_ms, 4),
                      "vs_stream_copy": round(achieved / copy_gbs, 4), "stream_copy_gbs": round(copy_gbs, 2),
