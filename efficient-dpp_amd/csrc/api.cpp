@@ -49,26 +49,32 @@ static int grow(edpp_ctx* c, void** ws, size_t* ws_bytes, size_t bytes, void** o
     return EDPP_OK;
 }
 int ws_reserve(edpp_ctx* c, size_t bytes, void** out) { return grow(c, &c->ws, &c->ws_bytes, bytes, out); }
-// The new block is taken before the old one is given back, so that a refusal
-// changes nothing; a size that was refused is not asked for again.
+// Asks for the room first, so that a refusal changes nothing; a size that was
+// refused is not asked for again.  The old block goes before the new one comes,
+// so that a context never needs room for both.
 int ws_try_reserve(edpp_ctx* c, size_t bytes, void** out) {
     *out = nullptr;
     bytes = (bytes + 255) & ~(size_t)255;
     if (bytes > c->ws_bytes) {
         if (c->ws_refused && bytes >= c->ws_refused) return EDPP_OK;
-        void* p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) {
+        size_t room = 0, all = 0;
+        if (hipMemGetInfo(&room, &all) != hipSuccess || room + c->ws_bytes < bytes) {
             (void)hipGetLastError();
             c->ws_refused = bytes;
             return EDPP_OK;
         }
-        hipError_t e = c->ws ? hipStreamSynchronize(c->stream) : hipSuccess;  // earlier kernels may still use it
-        if (e == hipSuccess && c->ws) e = hipFree(c->ws);
-        if (e != hipSuccess) {
-            hipFree(p);
-            return hip_fail(c, e, "workspace");
+        if (c->ws) {
+            EDPP_HIP(c, hipStreamSynchronize(c->stream));  // earlier kernels may still use it
+            EDPP_HIP(c, hipFree(c->ws));
+            c->ws = nullptr;
+            c->ws_bytes = 0;
         }
-        c->ws = p;
+        if (hipMalloc(&c->ws, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            c->ws = nullptr;
+            c->ws_refused = bytes;
+            return EDPP_OK;
+        }
         c->ws_bytes = bytes;
     }
     *out = c->ws;
