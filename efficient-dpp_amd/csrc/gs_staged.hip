@@ -677,14 +677,15 @@ __global__ __launch_bounds__(kStBinBlock, kStBinBlock / 128) void k_st_bins(StGe
 }
 
 // sval[j] = in[sidx[j]]: workgroups of one XCD walk one range of the window
-// order, so the windows being read at one time are few and stay in its L2
+// order, so the windows being read at one time are few and stay in its L2.
+// 4-byte values take their indices' place: a lane has read all of its indices
+// before it stores.
 template <class T>
 constexpr int kStGe = 128 / (int)sizeof(T);  // staged elements per lane
 template <class T>
 constexpr int kStPart = 256 * kStGe<T>;      // and per workgroup
 template <class T>
-__global__ __launch_bounds__(256) void k_st_gather(const T* __restrict__ in, StGeom g,
-                                                   const uint32_t* __restrict__ sidx, T* __restrict__ sval) {
+__global__ __launch_bounds__(256) void k_st_gather(const T* __restrict__ in, StGeom g, const uint32_t* sidx, T* sval) {
     constexpr int E = kStE<T>;
     if (*g.open == 0) return;
     const int64_t m = std::min<int64_t>(g.base[g.W], g.n);
@@ -900,7 +901,7 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
                  o_rows = take((size_t)g.tiles * g.WP * 4), o_gsum = take((size_t)g.groups * g.WP * 4), o_total = take((size_t)g.WP * 4), o_open = take(4), o_base = take(((size_t)g.WP + 1) * 4),
                  o_tile2 = take(((size_t)g.WP + 1) * 4), o_win2 = take((size_t)tiles2 * 2), o_rows2 = take(((size_t)tiles2 << g.lg_subs) * 4),
                  o_bins = take(((size_t)g.W << g.lg_subs) * 4), o_sidx = take((size_t)n * 4),
-                 o_sval = take((size_t)n * sizeof(T)), o_didx = take(scatter ? (size_t)n * 4 : 0),
+                 o_sval = !scatter && sizeof(T) == 4 ? o_sidx : take((size_t)n * sizeof(T)), o_didx = take(scatter ? (size_t)n * 4 : 0),
                  o_dval = take(scatter ? (size_t)n * sizeof(T) : 0), o_slot = take(scatter ? 0 : (size_t)g.tiles * S * 2),
                  o_probe = take(scatter ? 0 : (size_t)kStProbes * 8);
     void* w;

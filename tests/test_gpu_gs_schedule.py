@@ -34,8 +34,11 @@ def test_calls_without_room_for_the_workspace(torch_gpu, edpp):
     with edpp.Context(0, stream=torch.cuda.current_stream().cuda_stream) as c:
         c.scatter(src, scattered, idx, passes=2)  # a small workspace: one flag per chunk
         hold = []
-        while (free := torch.cuda.mem_get_info()[0]) > (3 << 29):
-            hold.append(torch.empty(min(16 << 30, free - (1 << 30)), dtype=torch.uint8, device="cuda"))
+        for _ in range(64):
+            free = torch.cuda.mem_get_info()[0]
+            if free <= 1 << 29:  # the gather alone needs 6 bytes per element
+                break
+            hold.append(torch.empty(min(16 << 30, free - (1 << 28)), dtype=torch.uint8, device="cuda"))
         for _ in range(2):
             gathered.fill_(-1)
             scattered.fill_(-1)
