@@ -221,7 +221,7 @@ __device__ void hist_scan_tile(const DJob& J, int64_t t, char* smem, uint32_t sp
 }
 
 // The same for a job of at most kColumnTiles tiles by one workgroup, where
-// column_scan says so: a lane takes a bucket (BLOCK >> lg lanes a range of the
+// the planner says so: a lane takes a bucket (BLOCK >> lg lanes a range of the
 // tiles each), so that every access of a wave is whole lines, and nothing is
 // looked back for.  (With
 // bucket-major lanes, the scans of the 10,000-job mix, 11 M words, took 174 us
@@ -621,18 +621,18 @@ static int validate_jobs(edpp_ctx* c, const edpp_job* jobs, int32_t njobs) {
     return EDPP_OK;
 }
 
-// Whether one workgroup scans a split job's counts (hist_column_scan): where
-// the words of a lane are in flight at once, and else where the launch is long
-// enough to hide the workgroup's chain of readings, about 6 us for each
-// kColumnRows words of a lane; 3 times that, as the job's own tiles wait for it.
-// 256 buckets, us, by column / by look-back: 1 job of 40,000 keys 33 / 31, of
-// 100,000 44 / 34, of 524,288 165 / 49; 16 jobs of 524,288 172 / 115, 64 of
-// them 382 / 357, 128 of them 665 / 700; 128 jobs of 100,000 126 / 146.
-static int column_scan(const BatchShape& sh, const DJob& d, double batch_us) {
-    if (d.tiles > kColumnTiles) return 0;
+// Rounds of readings of kColumnRows words a lane that one workgroup takes for a
+// split job's counts (hist_column_scan), about 6 us each.  It scans them where
+// that is one round, where the launch is three times as long, or where the work
+// of the jobs that need fewer rounds is twice as long: the job's own tiles wait
+// for it, and the others' can run meanwhile.  256 buckets, us, by column / by
+// look-back: 1 job of 40,000 keys 33 / 31, of 100,000 44 / 34, of 524,288 165 /
+// 49; 16 jobs of 524,288 172 / 115, 64 of them 382 / 357, 128 of them 665 /
+// 700; 128 jobs of 100,000 126 / 146; mixes of 100 jobs 145 / 107, of 1000
+// short ones 52 / 57.
+static int64_t column_rounds(const BatchShape& sh, const DJob& d) {
     const int64_t ranges = std::min<int64_t>(sh.block >> d.lg, d.tiles);
-    const int64_t rounds = ceil_div(ceil_div(d.tiles, ranges), (int64_t)kColumnRows);
-    return rounds == 1 || 18.0 * (double)rounds <= batch_us ? 1 : 0;
+    return ceil_div(ceil_div(d.tiles, ranges), (int64_t)kColumnRows);
 }
 
 // Builds the work queue and state of b->jobs for b->shape and uploads them.
@@ -646,12 +646,10 @@ static int plan(edpp_batch* b) {
     // its look-back status words and, for a split, its tagged histogram words
     int64_t words = (int64_t)kMaxQueues * kTicketStride;
     std::vector<int64_t> soff(njobs, -1);
-    double batch_us = 0;  // about what the launch takes, at 2.5 TB/s
-    for (int32_t j = 0; j < njobs; ++j) {
-        const edpp_job& q = b->jobs[j];
-        const int64_t per = 2 * q.elem_bytes + (q.kind == EDPP_JOB_SPLIT ? 8 : q.kind == EDPP_JOB_GATHER ? 4 : 0);
-        batch_us += (double)q.n * (double)per * 4e-7;
-    }
+    // about what the launch takes, at 2.5 TB/s: all of it, and the jobs of at
+    // most r column rounds
+    constexpr int kMaxRounds = (int)(kColumnTiles / kColumnRows);
+    double batch_us = 0, free_us[kMaxRounds + 2] = {};
     for (int32_t j = 0; j < njobs; ++j) {
         const edpp_job& q = b->jobs[j];
         DJob& d = dj[j];
@@ -668,13 +666,27 @@ static int plan(edpp_batch* b) {
         if (q.kind == EDPP_JOB_SPLIT)
             while ((1 << d.lg) < q.buckets) ++d.lg;
         d.tiles = ceil_div(q.n, tile_elems(sh, q.kind, d.wide));
+        const int64_t per = 2 * q.elem_bytes + (q.kind == EDPP_JOB_SPLIT ? 8 : q.kind == EDPP_JOB_GATHER ? 4 : 0);
+        const double us = (double)q.n * (double)per * 4e-7;
+        batch_us += us;
+        int64_t r = 0;
+        if (q.kind == EDPP_JOB_SPLIT && d.tiles > 1)
+            r = d.tiles > kColumnTiles ? kMaxRounds + 1 : column_rounds(sh, d);
+        free_us[r] += us;
+    }
+    for (int r = 1; r <= kMaxRounds + 1; ++r) free_us[r] += free_us[r - 1];
+    for (int32_t j = 0; j < njobs; ++j) {
+        const edpp_job& q = b->jobs[j];
+        DJob& d = dj[j];
         soff[j] = words;
         if (q.kind == EDPP_JOB_SCAN) {
             words += (d.wide ? 4 : 2) * d.tiles;  // one or two u64 status words per tile
         } else if (q.kind == EDPP_JOB_SPLIT && d.tiles > 1) {
             // (a job of one tile takes its offsets from its own counts)
             const int64_t hlen = ((int64_t)1 << d.lg) * d.tiles;
-            d.column = column_scan(sh, d, batch_us);
+            const int64_t r = column_rounds(sh, d);
+            d.column = d.tiles <= kColumnTiles &&
+                       (r == 1 || 18.0 * (double)r <= batch_us || 12.0 * (double)r <= free_us[r - 1]);
             d.hscan_tiles = d.column ? 1 : ceil_div(hlen, hscan_tile_elems(sh));
             words += 2 * d.hscan_tiles + 2 * hlen;  // u64 status, then u64 histogram words
         }
