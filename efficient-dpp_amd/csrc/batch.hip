@@ -407,18 +407,18 @@ __device__ void gather_tile(const DJob& J, int64_t t) {
         #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int64_t e0 = base + (int64_t)u * BLOCK * 4 + threadIdx.x * 4;
-            const bool all = (uint32_t)x[u][0] < n && (uint32_t)x[u][1] < n && (uint32_t)x[u][2] < n &&
-                             (uint32_t)x[u][3] < n;
+            typedef typename vec16<T>::type V;
+            constexpr int EPV = vec16<T>::n;
+            bool all = true;
+            V o[4 / EPV];
+            #pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                all = all && (uint32_t)x[u][k] < n;
+                o[k / EPV][k % EPV] = v[u][k];
+            }
             if (all) {
-                typedef typename vec16<T>::type V;
-                constexpr int EPV = vec16<T>::n;
                 #pragma unroll
-                for (int h = 0; h < 4 / EPV; ++h) {
-                    V o;
-                    #pragma unroll
-                    for (int k = 0; k < EPV; ++k) o[k] = v[u][h * EPV + k];
-                    st_stream(o, reinterpret_cast<V*>(out + e0 + h * EPV));
-                }
+                for (int h = 0; h < 4 / EPV; ++h) st_stream(o[h], reinterpret_cast<V*>(out + e0 + h * EPV));
             } else {
                 #pragma unroll
                 for (int k = 0; k < 4; ++k)
