@@ -49,9 +49,10 @@ static int grow(edpp_ctx* c, void** ws, size_t* ws_bytes, size_t bytes, void** o
     return EDPP_OK;
 }
 int ws_reserve(edpp_ctx* c, size_t bytes, void** out) { return grow(c, &c->ws, &c->ws_bytes, bytes, out); }
-// Asks for the room first, so that a refusal changes nothing; a size that was
-// refused is not asked for again.  The old block goes before the new one comes,
-// so that a context never needs room for both.
+// Asks for the room first, so that a refusal changes nothing and the next call
+// finds out anew; only a size that did not come although there was room for it
+// is not tried again.  The old block goes before the new one comes, so that a
+// context never needs room for both.
 int ws_try_reserve(edpp_ctx* c, size_t bytes, void** out) {
     *out = nullptr;
     bytes = (bytes + 255) & ~(size_t)255;
@@ -60,7 +61,6 @@ int ws_try_reserve(edpp_ctx* c, size_t bytes, void** out) {
         size_t room = 0, all = 0;
         if (hipMemGetInfo(&room, &all) != hipSuccess || room + c->ws_bytes < bytes) {
             (void)hipGetLastError();
-            c->ws_refused = bytes;
             return EDPP_OK;
         }
         if (c->ws) {

@@ -18,7 +18,7 @@ struct edpp_ctx {
     // grow-only scratch for per-call temporaries (histograms, partials)
     void* ws = nullptr;
     size_t ws_bytes = 0;
-    size_t ws_refused = 0;  // size of the last ws_try_reserve that was refused, 0: none
+    size_t ws_refused = 0;  // size that ws_try_reserve was refused although there was room, 0: none
     // scratch of composite calls (hash join) that hold buffers across the
     // primitives they call, which use ws
     void* ws_outer = nullptr;

@@ -52,3 +52,9 @@ def test_calls_without_room_for_the_workspace(torch_gpu, edpp):
         assert torch.equal(gathered, want)
         want[idx.long()] = src
         assert torch.equal(scattered, want)
+        free = torch.cuda.mem_get_info()[0]
+        scattered.fill_(-1)
+        c.scatter(src, scattered, idx)  # there is room again
+        c.sync()
+        assert torch.cuda.mem_get_info()[0] < free - 16 * n
+        assert torch.equal(scattered, want)
