@@ -83,7 +83,7 @@ constexpr BatchShape kShapes[] = {
     {256, 16, 8, 8, 8},  // 5: scan 16384 / 4096, split 2048, gather 8192 (the default)
 };
 constexpr int kNumShapes = (int)(sizeof(kShapes) / sizeof(kShapes[0]));
-constexpr int kDefaultShape = 5;  // fastest on the 10 000-job mix (1.67 against 1.76 ms for shape 0)
+constexpr int kDefaultShape = 5;  // fastest on the 10 000-job mix (1.68 against 1.76 ms for shape 0)
 constexpr int kOccupancies[] = {2, 4, 8};
 constexpr int kNumOcc = 3;
 constexpr int kNumOrders = EDPP_BATCH_ORDER_XCD + 1;

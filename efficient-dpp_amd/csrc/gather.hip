@@ -21,7 +21,9 @@ namespace edpp {
 // or 512 of 2 8-byte ones, so that the CU has 32 waves beside LDS windows of 32
 // KiB, not 16, and a wave's 16-byte vectors are contiguous: local, 2^21 and
 // 2^22 positions, 6.2 and 11.2 us, with 256 lanes of 4 9.1 and 18.2; random
-// ones the same.  (Scatters gained a tenth where they are local, but random
+// ones the same; 8 to 64 interleaved streams a power of two apart 5 to 20 %
+// longer (8 streams, 2^22: 15.4 and 12.5), as a wave's loads then touch twice
+// as many.  (512 lanes of 4: local 7.6 and 16.1.  Scatters gained a tenth where they are local, but random
 // ones of 2^24 took 340 us instead of 303.)
 template <class T, bool SC>
 constexpr int kGsE = SC ? 4 : 16 / (int)sizeof(T);
