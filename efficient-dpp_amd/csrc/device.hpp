@@ -6,6 +6,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <algorithm>
 
 namespace edpp {
 
@@ -115,6 +116,18 @@ __device__ __forceinline__ uint64_t read_lane(uint64_t x, int l) {
 template <class T>
 __device__ __forceinline__ T wave_sum(T x) {
     return read_lane(wave_inclusive_add(x), kWave - 1);
+}
+
+// largest of the wave's values, by the network of wave_inclusive_add (0 for no
+// source is the identity here too)
+__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
+    x = std::max(x, dpp_or_zero<0x111, 0xf>(x));
+    x = std::max(x, dpp_or_zero<0x112, 0xf>(x));
+    x = std::max(x, dpp_or_zero<0x114, 0xf>(x));
+    x = std::max(x, dpp_or_zero<0x118, 0xf>(x));
+    x = std::max(x, dpp_or_zero<0x142, 0xa>(x));
+    x = std::max(x, dpp_or_zero<0x143, 0xc>(x));
+    return read_lane(x, kWave - 1);
 }
 
 // ---------------------------------------------------------------- atomics

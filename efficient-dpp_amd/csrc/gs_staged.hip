@@ -162,21 +162,23 @@ __device__ __forceinline__ bool st_scattered(const StGeom& g) {
 // A gather addresses a chunk directly if its indices fall inside g.near
 // elements, as L2 holds that many, and every chunk if the indices are not
 // scattered.  A scatter does so with a chunk that writes at least kStCover
-// sixteenths of the lines it touches, or whole 32-byte sectors by neighbouring
-// lanes, as most of that leaves L2 as whole lines or sectors.  The others are
-// counted.
+// sixteenths of the lines it touches, and soon (its first quarter, of 8-byte
+// values half, touches at most 3 lines per 16 elements), or whole 32-byte
+// sectors by neighbouring lanes, as most of that leaves L2 as whole lines or
+// sectors.  The others are counted.
 //
 // Scatters of 2^28 4-byte elements, us in one direct pass / in four / in
 // window order: two interleaved streams 590 / 1610 / 2690, 64 of them 1150 /
 // 1880 / 2680, rows of 32 elements 670 / 1910 / 2610, every second element
 // 1310 / 2160 / 2700, rows of 8 1950 / 2610 / 2740; but every eighth element
-// 6710 / 5480 / 2690, rows of 2 5620 / 3560 / 2770, 256 streams of random
-// lengths 3210 / 2530 / 2730.  The lines of a chunk are counted by hash in
-// bytes of LDS (k_st_first of a random scatter 166 us without, 202 so, 213 by
-// atomics on a bitmap).  Its lanes take 4 elements per step also of 8-byte
-// values, so that the lanes of one store touch fewer streams (128 streams 1240
-// us, by steps of 2 2040); a gather's stores have to be consecutive (470, by
-// steps of 4 820).
+// 6710 / 5480 / 2690, rows of 2 5620 / 3560 / 2770, 256 interleaved streams
+// 3940 / 3800 / 3090, of random lengths 3210 / 2530 / 2730.  Lines are counted
+// by hash in bytes of LDS; where the indices are scattered, the first part's
+// are too many already (k_st_first of a random scatter 166 us, 183 with all
+// lines counted, 162 without).  A scatter's lanes
+// take 4 elements per step also of 8-byte values, so that the lanes of one
+// store touch fewer streams (128 streams 1240 us, by steps of 2 2040); a
+// gather's stores have to be consecutive (470, by steps of 4 820).
 constexpr uint32_t kStCover = 7;
 constexpr int kStLineLg = 12;
 template <class T>
@@ -216,11 +218,8 @@ __global__ __launch_bounds__(kStFirstBlock<T>) void k_st_first(const T* __restri
             lo = std::min(lo, pos[e]);
             hi = std::max(hi, pos[e]);
         }
-    #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        lo = std::min(lo, (uint32_t)__shfl_xor((int)lo, o));
-        hi = std::max(hi, (uint32_t)__shfl_xor((int)hi, o));
-    }
+    lo = ~wave_max(~lo);
+    hi = wave_max(hi);
     constexpr int kLgLine = sizeof(T) == 4 ? 5 : 4;
     uint32_t broken = 0;  // the wave's lane steps (4-byte elements: pairs of lanes) that touch more than one sector
     if constexpr (SC) {
@@ -253,20 +252,25 @@ __global__ __launch_bounds__(kStFirstBlock<T>) void k_st_first(const T* __restri
         #pragma unroll
         for (int x = 0; x < NW; ++x) broken += wsw[x];
         near = near || 8 * broken <= kStChunk / P;
-        if (!near) {
-            // distinct lines, by hash (a few hundred where it matters)
+        // distinct lines, by hash (a few hundred where it matters), first of the
+        // chunk's leading elements
+        auto lines = [&](int e0, int e1) {
             #pragma unroll
             for (int e = 0; e < N; ++e)
-                if (pos[e] < nall) seen[st_line_hash(pos[e] >> kLgLine, kStLineLg)] = 1;
+                if (e >= e0 && e < e1 && pos[e] < nall) seen[st_line_hash(pos[e] >> kLgLine, kStLineLg)] = 1;
             __syncthreads();
-            uint32_t lines = 0;
+            uint32_t d = 0;
             #pragma unroll
             for (int i = 0; i < (1 << kStLineLg) / 16 / kWave; ++i) {
                 const v4u32 y = reinterpret_cast<const v4u32*>(seen)[i * kWave + lane_id()];
-                lines += __popc(y[0]) + __popc(y[1]) + __popc(y[2]) + __popc(y[3]);
+                d += __popc(y[0]) + __popc(y[1]) + __popc(y[2]) + __popc(y[3]);
             }
-            const uint32_t m = (uint32_t)std::min<int64_t>(g.n - (int64_t)blockIdx.x * kStChunk, kStChunk);
-            near = (wave_sum(lines) << kLgLine) * kStCover <= 16u * m;  // every wave sums all of them
+            return wave_sum(d);  // every wave sums all of them
+        };
+        const uint32_t m = (uint32_t)std::min<int64_t>(g.n - (int64_t)blockIdx.x * kStChunk, kStChunk);
+        if (!near && lines(0, P) * 16u <= 3u * (BL * P)) {
+            __syncthreads();
+            near = (lines(P, N) << kLgLine) * kStCover <= 16u * m;
         }
     } else {
         near = near || hi - lo < g.near || !scattered;
