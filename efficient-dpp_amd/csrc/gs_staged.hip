@@ -35,7 +35,7 @@
 // 2^28 4-byte elements, random permutation, us per kernel: gather 186 (first)
 // + 31 (prefixes) + 522 (split) + 1430 (gather: 290 M L2 requests, 204 G/s) +
 // 587 (return); the others move 10 to 12 B per element at 4.6 to 5 TB/s;
-// scatter 163 + 31 + 874 (split) + 254 (hist2) + 14 (rows2) + 880 (split2) +
+// scatter 168 + 31 + 874 (split) + 254 (hist2) + 14 (rows2) + 880 (split2) +
 // 580 (bins).
 #include <algorithm>
 #include "ctx.hpp"
@@ -174,7 +174,7 @@ __device__ __forceinline__ bool st_scattered(const StGeom& g) {
 // 6710 / 5480 / 2690, rows of 2 5620 / 3560 / 2770, 256 interleaved streams
 // 3940 / 3800 / 3090, of random lengths 3210 / 2530 / 2730.  Lines are counted
 // by hash in bytes of LDS; where the indices are scattered, the first part's
-// are too many already (k_st_first of a random scatter 166 us, 183 with all
+// are too many already (k_st_first of a random scatter 168 us, 183 with all
 // lines counted, 162 without).  A scatter's lanes
 // take 4 elements per step also of 8-byte values, so that the lanes of one
 // store touch fewer streams (128 streams 1240 us, by steps of 2 2040); a
@@ -943,15 +943,15 @@ int launch_gs_staged(edpp_ctx* c, const T* in, T* out, const int32_t* idx, int64
 //   gather  4 B  2^27     2564 / 1337          289 / 317          257 / 285
 //   gather  4 B  2^28     5455 / 2766          562 / 606          518 / 551
 //   scatter 4 B  2^26     1241 /  682          127 / 137          218 / 143
-//   scatter 4 B  2^27     2276 / 1385          345 / 332          811 / 317
-//   scatter 4 B  2^28     4475 / 2826          684 / 650         1601 / 625
+//   scatter 4 B  2^27     2287 / 1367          344 / 332          817 / 317
+//   scatter 4 B  2^28     4481 / 2800          686 / 649         1610 / 626
 //   gather  8 B  2^24      329 /  221           44 /  61           43 /  62
 //   gather  8 B  2^25      663 /  455           84 / 106           80 / 103
 //   gather  8 B  2^26     1317 /  890          226 / 258          222 / 247
 //   gather  8 B  2^27     2931 / 1832          451 / 495          462 / 495
 //   scatter 8 B  2^25      586 /  517          109 / 123          179 / 127
-//   scatter 8 B  2^26     1396 / 1022          286 / 289          620 / 290
-//   scatter 8 B  2^27     2795 / 2109          570 / 569         1216 / 558
+//   scatter 8 B  2^26     1400 / 1014          287 / 289          623 / 294
+//   scatter 8 B  2^27     2800 / 2087          571 / 566         1218 / 560
 // So calls start at 512 MiB, from where a local gather and scatter together
 // take no longer than by the direct schedule or little more (4 B, 2^26: 272
 // against 239 us, 2^27: 649 and 634); a direct gather of smaller tables loses
